@@ -287,7 +287,8 @@ def test_isect_tiles_packed_and_empty(gpu):
 
 
 @pytest.mark.parametrize("n,begin,end", [(1, 0, 64), (100, 0, 46), (4097, 3, 40),
-                                         (1_000_003, 0, 46), (70_000, 0, 64)])
+                                         (1_000_003, 0, 46), (70_000, 0, 64),
+                                         ((1 << 20) - 1, 0, 46), (1 << 20, 0, 46)])
 def test_radix_sort_pairs_stable(gpu, n, begin, end):
     announce(f"radix n={n} bits=[{begin},{end})")
     rng = np.random.default_rng(n)
@@ -302,6 +303,61 @@ def test_radix_sort_pairs_stable(gpu, n, begin, end):
     order = np.argsort(masked, kind="stable")
     np.testing.assert_array_equal(to_np(v), vals[order])
     np.testing.assert_array_equal(to_np(k), keys[order])
+
+
+@pytest.mark.parametrize("segs", [
+    [0, 1025],                                    # a one-key last quarter tile
+    [0, 32 * 1024], [0, 32 * 1024 + 1],           # one group of quarter tiles, and two
+    [0, 0, 40 * 1024, 40 * 1024 + 7, 200_000],    # groups in some segments only
+    [0] + [700 * k for k in range(1, 65)],        # 64 one-tile segments
+    [0] + [2 * k for k in range(1, 64)] + [70_000],  # more group rows than the workspace holds
+    [0, (3 << 19) - 1], [0, 3 << 19],             # either side of the quarter-tile sizes
+    [0, 1 << 22], [0, (1 << 22) + 1],             # either side of the sorts without a scan
+])
+@pytest.mark.parametrize("vbytes", [4, 8])
+def test_segmented_sort_size_rules(gpu, segs, vbytes):
+    """The sort's size rules (quarter tiles, group rows, column sums without a
+    scan) at their edges: each segment equal to numpy's stable argsort."""
+    import ctypes
+    from tidegs_amd import _native as N
+    announce(f"segmented sort size rules n={segs[-1]} segments={len(segs) - 1} vbytes={vbytes}")
+    n = segs[-1]
+    rng = np.random.default_rng(n + vbytes)
+    keys = rng.integers(0, 2 ** 19, size=n, dtype=np.uint64).astype(np.uint32)
+    vdt = np.int32 if vbytes == 4 else np.int64
+    vals = np.arange(n, dtype=vdt)
+    k = torch.from_numpy(keys.view(np.int32)).to(gpu)
+    v = torch.from_numpy(vals).to(gpu)
+    k2, v2 = torch.empty_like(k), torch.empty_like(v)
+    lib = N.load()
+    size = lib.tgs_segmented_sort_workspace_size(n, len(segs) - 1)
+    ws = torch.full((size,), 0xAB, dtype=torch.uint8, device=gpu)  # contents must not matter
+    sel = ctypes.c_int(0)
+    arr = (ctypes.c_uint32 * len(segs))(*segs)
+    N.call("tgs_segmented_sort_pairs_u32", N.ptr(k), N.ptr(v), N.ptr(k2), N.ptr(v2), vbytes, n,
+           len(segs) - 1, arr, 0, 19, N.ptr(ws), ws.numel(), ctypes.byref(sel),
+           N.stream_handle(gpu))
+    rk, rv = (k2, v2) if sel.value else (k, v)
+    order = np.concatenate([np.argsort(keys[a:b], kind="stable") + a
+                            for a, b in zip(segs[:-1], segs[1:])])
+    np.testing.assert_array_equal(to_np(rv), vals[order])
+    np.testing.assert_array_equal(to_np(rk).view(np.uint32), keys[order])
+
+
+@pytest.mark.parametrize("n", [1, 9, 8192, 8193, 16384, 16385])
+def test_scan_size_rules(gpu, n):
+    """One-workgroup and three-kernel scans at the line between them."""
+    from tidegs_amd import _native as N
+    announce(f"scan n={n}")
+    x = torch.from_numpy(np.random.default_rng(n).integers(0, 100, size=n, dtype=np.int32)).to(gpu)
+    ws = torch.empty(N.load().tgs_scan_workspace_size(n), dtype=torch.uint8, device=gpu)
+    s = N.stream_handle(gpu)
+    out, ex = torch.empty(n, dtype=torch.int64, device=gpu), torch.empty_like(x)
+    N.call("tgs_inclusive_scan_i32_i64", N.ptr(x), N.ptr(out), n, N.ptr(ws), ws.numel(), s)
+    N.call("tgs_exclusive_scan_u32", N.ptr(x), N.ptr(ex), n, N.ptr(ws), ws.numel(), s)
+    ref = np.cumsum(to_np(x).astype(np.int64))
+    np.testing.assert_array_equal(to_np(out), ref)
+    np.testing.assert_array_equal(to_np(ex), ref - to_np(x))
 
 
 @pytest.mark.parametrize("segs,bits,vbytes", [

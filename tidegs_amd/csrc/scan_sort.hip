@@ -8,11 +8,13 @@
 // equals "ascending in (key bits, input position)", a total order, so any
 // correct stable sort reproduces the reference output bit for bit.
 //
-// Scan: reduce-then-scan in three kernels (block sums, one-block scan of the
-// sums, per-block rescan), no inter-block spin-waits.
-// Radix pass (<= 8-bit digit, 4096-key tiles of 256 threads x 16 keys):
-//   hist      per-tile digit histogram -> hist[segment][digit][tile]
-//   scan      exclusive scan of hist (digit-major => global digit offsets)
+// Scan: up to SCAN_ONE_BLOCK_MAX values in one workgroup; above, reduce-then-
+// scan in three kernels (block sums, one-block scan of the sums, per-block
+// rescan), no inter-block spin-waits.
+// Radix pass (<= 8-bit digit, tiles of 256 threads x ITEMS keys):
+//   hist      per-tile digit histogram
+//   scan      exclusive scan of the histogram (large sorts only: a small
+//             sort's scatter adds up the counts before its tile by itself)
 //   scatter   per-tile stable ranking (ballot matching + per-wave counters),
 //             LDS reorder, coalesced write of each digit run.
 #include <mutex>
@@ -24,7 +26,7 @@
 #define SCAN_CHUNK (SCAN_THREADS * SCAN_ITEMS)
 
 #define SORT_THREADS 256
-#define SORT_ITEMS 16
+#define SORT_ITEMS 16  // keys per thread of a large sort
 #define SORT_TILE (SORT_THREADS * SORT_ITEMS)
 #define SORT_BINS 256
 #define RADIX_MAX_SEGS 64
@@ -142,11 +144,61 @@ __global__ void __launch_bounds__(SCAN_THREADS) scan_apply_kernel(const InT* __r
   }
 }
 
+// The whole scan in one 1024-thread workgroup, SCAN_ONE_ITEMS consecutive
+// values per thread and round.  The three-kernel form spends its time in
+// launches when the array is short (a pass's histogram, the per-block counts of
+// a few hundred thousand rows): a radix pass over 7.7k counts takes 13 us
+// less with this scan.  At 25k values, three rounds of the one workgroup, the
+// three launches are as fast.
+#define SCAN_ONE_THREADS 1024
+#define SCAN_ONE_ITEMS 8
+#define SCAN_ONE_BLOCK_MAX 16384
+
+template <typename InT, typename OutT, bool INCLUSIVE>
+__global__ void __launch_bounds__(SCAN_ONE_THREADS) scan_one_block_kernel(
+    const InT* __restrict__ in, uint32_t n, OutT* __restrict__ out) {
+  __shared__ OutT s_wave[SCAN_ONE_THREADS / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  OutT carry = 0;
+  for (uint32_t base = 0; base < n; base += SCAN_ONE_THREADS * SCAN_ONE_ITEMS) {
+    const uint32_t i0 = base + threadIdx.x * SCAN_ONE_ITEMS;
+    OutT vals[SCAN_ONE_ITEMS];
+    OutT sum = 0;
+#pragma unroll
+    for (int k = 0; k < SCAN_ONE_ITEMS; ++k) {
+      vals[k] = i0 + k < n ? (OutT)in[i0 + k] : (OutT)0;
+      sum += vals[k];
+    }
+    const OutT inc = wave_inclusive_scan<OutT>(sum);
+    if (lane == 63) s_wave[wave] = inc;
+    __syncthreads();
+    OutT run = carry + inc - sum;
+#pragma unroll
+    for (int w = 0; w < SCAN_ONE_THREADS / 64; ++w) {
+      const OutT t = s_wave[w];
+      if (w < wave) run += t;
+      carry += t;
+    }
+#pragma unroll
+    for (int k = 0; k < SCAN_ONE_ITEMS; ++k) {
+      if (INCLUSIVE) run += vals[k];
+      if (i0 + k < n) out[i0 + k] = run;
+      if (!INCLUSIVE) run += vals[k];
+    }
+    __syncthreads();
+  }
+}
+
 static uint64_t scan_blocks(uint64_t n) { return (n + SCAN_CHUNK - 1) / SCAN_CHUNK; }
 
 template <typename InT, typename OutT, bool INCLUSIVE>
 static int launch_scan(const InT* in, OutT* out, uint64_t n, OutT* sums, hipStream_t stream) {
   if (n == 0) return TGS_OK;
+  if (n <= SCAN_ONE_BLOCK_MAX) {
+    hipLaunchKernelGGL((scan_one_block_kernel<InT, OutT, INCLUSIVE>), dim3(1),
+                       dim3(SCAN_ONE_THREADS), 0, stream, in, (uint32_t)n, out);
+    TGS_RETURN_LAUNCH("scan");
+  }
   const uint64_t nb = scan_blocks(n);
   hipLaunchKernelGGL((scan_reduce_kernel<InT, OutT>), dim3((unsigned)nb), dim3(SCAN_THREADS), 0,
                      stream, in, n, sums);
@@ -199,15 +251,35 @@ extern "C" int tgs_exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint64_
 // Segmented LSD passes: the key range [0, n) is split into segments (one for
 // a plain sort; one per camera for the fused step, where entries and
 // intersections are already grouped by camera) and tiles never straddle a
-// segment, so one pass sorts every segment independently.  The histogram is
-// laid out [segment][digit][tile of segment]; its exclusive scan is then the
-// absolute output offset of (segment, digit, tile).
+// segment, so one pass sorts every segment independently.
+//
+// A pass needs, per (tile, digit), the output slot of the digit's first key:
+// the segment's start, plus the segment's keys of smaller digits, plus the
+// keys of this digit in the segment's earlier tiles.
+//   Large sorts: the histogram is laid out [segment][digit][tile of segment]
+//   and its exclusive scan (three more launches) is that slot.
+//   Small sorts (LOCAL, at most RADIX_LOCAL_KEYS keys): the histogram is laid
+//   out [tile][digit] and the scatter adds its tile's column up by itself,
+//   from one row per RADIX_GROUP earlier tiles (summed by the histogram
+//   kernel's atomics) and the rows since.  A pass is two launches, not five:
+//   the scan's three kernels take 11-16 us of a pass whose histogram and
+//   scatter take 15 us at 10k keys and 25 us at 2.7M.  Above the line the
+//   scatters' row sums cost more than the scan.  Whole sorts, with the scan
+//   and without, in us:
+//     46 bits of 64-bit keys, 4-byte values  10k 134 -> 60, 300k 168 -> 108,
+//                                            2.7M 234 -> 202, 5M 334 -> 376
+//     25 bits of 32-bit keys, 8-byte values  10k 89 -> 39, 300k 112 -> 56,
+//                                            2.7M 147 -> 113, 5M 192 -> 187
 // ---------------------------------------------------------------------------
+#define RADIX_GROUP 32
+#define RADIX_LOCAL_KEYS (1u << 22)
 
 struct RadixSegs {
   uint32_t n;                             // number of segments (>= 1)
   uint32_t key_off[RADIX_MAX_SEGS + 1];   // key_off[0] = 0, key_off[n] = n_keys
   uint32_t tile_base[RADIX_MAX_SEGS + 1]; // first tile of each segment
+  // first group of RADIX_GROUP tiles of each segment (LOCAL passes)
+  uint32_t group_base[RADIX_MAX_SEGS + 1];
   // 32-bit keys are ranked as min(key - key_base, key_cap) (keys below the
   // base as 0): an order-preserving map of a key range onto its low bits, with
   // every key past the range tied at key_cap.  (0, ~0) ranks the keys as they are.
@@ -216,26 +288,24 @@ struct RadixSegs {
 
 struct TileRange {
   uint32_t start, count;  // keys [start, start + count)
-  uint32_t hbase, stride; // hist index of digit d: hbase + d * stride
+  uint32_t seg, t, nts;   // segment, tile within it, tiles of it
 };
 
-// nbins: the pass's digit count (1 << bits); the histogram holds nbins counts
-// per tile, [segment][digit][tile of segment]
-__device__ __forceinline__ TileRange radix_tile(const RadixSegs& sg, uint32_t b, uint32_t nbins) {
+template <uint32_t TILE>
+__device__ __forceinline__ TileRange radix_tile(const RadixSegs& sg, uint32_t b) {
   uint32_t lo = 0, hi = sg.n;  // largest s with tile_base[s] <= b
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
     if (sg.tile_base[mid] <= b) lo = mid;
     else hi = mid;
   }
-  const uint32_t t = b - sg.tile_base[lo];
-  const uint32_t nts = sg.tile_base[lo + 1] - sg.tile_base[lo];
   TileRange r;
-  r.start = sg.key_off[lo] + t * SORT_TILE;
+  r.seg = lo;
+  r.t = b - sg.tile_base[lo];
+  r.nts = sg.tile_base[lo + 1] - sg.tile_base[lo];
+  r.start = sg.key_off[lo] + r.t * TILE;
   const uint32_t end = sg.key_off[lo + 1];
-  r.count = end > r.start ? min((uint32_t)SORT_TILE, end - r.start) : 0u;
-  r.hbase = sg.tile_base[lo] * nbins + t;
-  r.stride = nts;
+  r.count = end > r.start ? min(TILE, end - r.start) : 0u;
   return r;
 }
 
@@ -253,29 +323,34 @@ __device__ __forceinline__ uint32_t digit_of(K key, const RadixSegs& sg, int shi
   }
 }
 
-template <typename K>
+// nbins: the pass's digit count (1 << bits); the histogram holds nbins counts
+// per tile.  LOCAL: hist[tile][digit], and each count is added to its group's
+// row of group_hist [group][digit] (zeroed by the caller; null where no segment
+// has more than one group).
+template <typename K, int ITEMS, bool LOCAL>
 __global__ void __launch_bounds__(SORT_THREADS) radix_hist_kernel(const K* __restrict__ keys,
                                                                   RadixSegs sg, int shift,
                                                                   uint32_t mask, uint32_t nbins,
-                                                                  uint32_t* __restrict__ hist) {
+                                                                  uint32_t* __restrict__ hist,
+                                                                  uint32_t* __restrict__ group_hist) {
   __shared__ uint32_t s_h[SORT_THREADS / 64][SORT_BINS];
   const int wave = threadIdx.x >> 6;
 #pragma unroll
   for (int w = 0; w < SORT_THREADS / 64; ++w) s_h[w][threadIdx.x] = 0;
   __syncthreads();
-  const TileRange tr = radix_tile(sg, blockIdx.x, nbins);
+  const TileRange tr = radix_tile<SORT_THREADS * ITEMS>(sg, blockIdx.x);
   // A wavefront whose keys share one digit (common for the high digits of
   // sorted-ish keys) adds its count once instead of 64 conflicting atomics.
   // all of the thread's keys are loaded before any is counted, so the tile's
   // loads are in flight together
-  K kr[SORT_ITEMS];
+  K kr[ITEMS];
 #pragma unroll
-  for (int r = 0; r < SORT_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t i = (uint32_t)r * SORT_THREADS + threadIdx.x;
     kr[r] = i < tr.count ? keys[tr.start + i] : (K)0;
   }
 #pragma unroll
-  for (int r = 0; r < SORT_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t i = (uint32_t)r * SORT_THREADS + threadIdx.x;
     const bool valid = i < tr.count;
     const uint32_t d = valid ? digit_of(kr[r], sg, shift, mask) : 0u;
@@ -293,44 +368,53 @@ __global__ void __launch_bounds__(SORT_THREADS) radix_hist_kernel(const K* __res
 #pragma unroll
   for (int w = 0; w < SORT_THREADS / 64; ++w) c += s_h[w][threadIdx.x];
   // only the pass's digits: a narrower pass stores (and scans) fewer counts,
-  // each a line of its own in this layout
-  if (threadIdx.x < nbins) hist[tr.hbase + threadIdx.x * tr.stride] = c;
+  // each a line of its own in the [digit][tile] layout
+  if (threadIdx.x < nbins) {
+    if (LOCAL) {
+      hist[blockIdx.x * nbins + threadIdx.x] = c;
+      if (group_hist && c)
+        atomicAdd(&group_hist[(sg.group_base[tr.seg] + tr.t / RADIX_GROUP) * nbins + threadIdx.x],
+                  c);
+    } else {
+      hist[sg.tile_base[tr.seg] * nbins + tr.t + threadIdx.x * tr.nts] = c;
+    }
+  }
 }
 
-// One tile of 4096 keys per block.  Wave w owns keys [w*1024, (w+1)*1024) of
-// the tile in rounds of 64; for each round 8 ballots give a lane the lanes of
+// One tile of 256 x ITEMS keys per block.  Wave w owns 64 x ITEMS consecutive
+// keys of the tile in rounds of 64; for each round 8 ballots give a lane the lanes of
 // its wave with the same digit, and a per-wave digit counter in LDS carries
 // the count of earlier rounds.  The tile is then scattered into LDS in
 // (digit, position) order and written out by consecutive threads, so each
 // digit's run of the tile is one contiguous store.
-template <typename K, typename V>
+template <typename K, typename V, int ITEMS, bool LOCAL>
 __global__ void __launch_bounds__(SORT_THREADS) __attribute__((amdgpu_waves_per_eu(4))) radix_scatter_kernel(
     const K* __restrict__ keys_in, const V* __restrict__ vals_in, RadixSegs sg, int shift,
-    uint32_t mask, uint32_t nbins, const uint32_t* __restrict__ hist_scan,
-    K* __restrict__ keys_out, V* __restrict__ vals_out) {
+    uint32_t mask, uint32_t nbins, const uint32_t* __restrict__ hist,
+    const uint32_t* __restrict__ group_hist, K* __restrict__ keys_out, V* __restrict__ vals_out) {
   constexpr int WAVES = SORT_THREADS / 64;
-  __shared__ K s_k[SORT_TILE];
-  __shared__ V s_v[SORT_TILE];
+  constexpr uint32_t TILE = SORT_THREADS * ITEMS;
+  __shared__ K s_k[TILE];
+  __shared__ V s_v[TILE];
   // per-wave digit counters, then each (wave, digit)'s first position in the
-  // tile (counts and positions stay below SORT_TILE: 16 bits, so the 8-byte
+  // tile (counts and positions stay below the tile size: 16 bits, so the 8-byte
   // value form's LDS lets 3 workgroups share a CU)
   __shared__ uint16_t s_wh[WAVES][SORT_BINS];
   __shared__ uint32_t s_gofs[SORT_BINS];
-  __shared__ uint32_t s_scan[WAVES];
+  __shared__ uint64_t s_scan[WAVES];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const uint64_t lt_mask = (1ull << lane) - 1ull;
-  const TileRange tr = radix_tile(sg, blockIdx.x, nbins);
+  const TileRange tr = radix_tile<TILE>(sg, blockIdx.x);
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) s_wh[w][threadIdx.x] = 0;
-  __syncthreads();
 
-  K k[SORT_ITEMS];
-  V v[SORT_ITEMS];
-  uint32_t rk[SORT_ITEMS];
-  const uint32_t wbase = (uint32_t)wave * 64u * SORT_ITEMS;
+  K k[ITEMS];
+  V v[ITEMS];
+  uint32_t rk[ITEMS];
+  const uint32_t wbase = (uint32_t)wave * 64u * ITEMS;
 #pragma unroll
-  for (int r = 0; r < SORT_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t li = wbase + (uint32_t)r * 64u + lane;
     if (li < tr.count) {
       k[r] = keys_in[tr.start + li];
@@ -340,8 +424,49 @@ __global__ void __launch_bounds__(SORT_THREADS) __attribute__((amdgpu_waves_per_
       v[r] = 0;
     }
   }
+  // LOCAL: this thread's share of digit (thread mod nbins)'s column: the
+  // segment's keys of the digit, and those in the tiles before this one
+  uint32_t seg_total = 0, before_tile = 0;
+  if (LOCAL) {
+    const uint32_t d = threadIdx.x & mask, parts = SORT_THREADS / nbins;
+    const uint32_t p = threadIdx.x / nbins;
+    const uint32_t* rows = hist + (uint64_t)sg.tile_base[tr.seg] * nbins + d;
+    uint32_t r0 = 0;
+    if (group_hist) {
+      const uint32_t* groups = group_hist + (uint64_t)sg.group_base[tr.seg] * nbins + d;
+      const uint32_t ng = sg.group_base[tr.seg + 1] - sg.group_base[tr.seg];
+      const uint32_t tg = tr.t / RADIX_GROUP;
+#pragma unroll 8
+      for (uint32_t g = p; g < ng; g += parts) {
+        const uint32_t c = groups[g * nbins];
+        seg_total += c;
+        before_tile += g < tg ? c : 0u;
+      }
+      r0 = tg * RADIX_GROUP;
+    }
+    const uint32_t r1 = group_hist ? tr.t : tr.nts;
+#pragma unroll 8
+    for (uint32_t r = r0 + p; r < r1; r += parts) {
+      const uint32_t c = rows[r * nbins];
+      seg_total += group_hist ? 0u : c;
+      before_tile += r < tr.t ? c : 0u;
+    }
+    uint32_t* s_part = reinterpret_cast<uint32_t*>(s_k);  // 2 x 256 words, before the reorder
+    static_assert(sizeof(s_k) >= 2 * SORT_THREADS * 4, "the tile holds the partial sums");
+    s_part[threadIdx.x] = seg_total;
+    s_part[SORT_THREADS + threadIdx.x] = before_tile;
+    __syncthreads();
+    seg_total = before_tile = 0;
+    if (threadIdx.x < nbins) {
+      for (uint32_t q = threadIdx.x; q < SORT_THREADS; q += nbins) {
+        seg_total += s_part[q];
+        before_tile += s_part[SORT_THREADS + q];
+      }
+    }
+  }
+  __syncthreads();
 #pragma unroll
-  for (int r = 0; r < SORT_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t li = wbase + (uint32_t)r * 64u + lane;
     const bool valid = li < tr.count;
     const uint32_t d = digit_of(k[r], sg, shift, mask);
@@ -372,8 +497,21 @@ __global__ void __launch_bounds__(SORT_THREADS) __attribute__((amdgpu_waves_per_
     cw[w] = s_wh[w][threadIdx.x];
     tot += cw[w];
   }
-  uint32_t all;
-  const uint32_t st = block_exclusive_scan<uint32_t>(tot, s_scan, all);
+  uint32_t st, first;  // digit's first position in the tile; its first output slot
+  if (LOCAL) {
+    // one scan for both: the tile's counts in the low word (their sum stays
+    // below the tile size), the segment's in the high word
+    uint64_t all;
+    const uint64_t ex =
+        block_exclusive_scan<uint64_t>(((uint64_t)seg_total << 32) | tot, s_scan, all);
+    st = (uint32_t)ex;
+    first = sg.key_off[tr.seg] + (uint32_t)(ex >> 32) + before_tile;
+  } else {
+    uint32_t all;
+    st = block_exclusive_scan<uint32_t>(tot, reinterpret_cast<uint32_t*>(s_scan), all);
+    first = threadIdx.x < nbins
+                ? hist[sg.tile_base[tr.seg] * nbins + tr.t + threadIdx.x * tr.nts] : st;
+  }
   uint32_t run = st;
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) {
@@ -381,11 +519,10 @@ __global__ void __launch_bounds__(SORT_THREADS) __attribute__((amdgpu_waves_per_
     run += cw[w];
   }
   // digits past nbins never occur in this pass
-  s_gofs[threadIdx.x] =
-      threadIdx.x < nbins ? hist_scan[tr.hbase + threadIdx.x * tr.stride] - st : 0u;
+  s_gofs[threadIdx.x] = first - st;
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < SORT_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t li = wbase + (uint32_t)r * 64u + lane;
     if (li < tr.count) {
       const uint32_t d = digit_of(k[r], sg, shift, mask);
@@ -403,7 +540,23 @@ __global__ void __launch_bounds__(SORT_THREADS) __attribute__((amdgpu_waves_per_
   }
 }
 
-static uint64_t sort_tiles(uint64_t n) { return (n + SORT_TILE - 1) / SORT_TILE; }
+// Keys per thread: a small sort takes quarter tiles (1024 keys), so that it
+// spreads over four times the CUs and each workgroup's chain of ranking rounds
+// is a quarter as long (300k keys: 129 -> 108 us with 64-bit keys, 74 -> 56
+// with 32-bit ones).  From a workgroup per CU and more on, the longer digit runs
+// of whole tiles win: with 64-bit keys at 1.2M (172 against 164 us), with
+// 32-bit ones later (1.2M 82 against 97, 2.7M 157 against 113).
+#define SORT_ITEMS_SMALL 4
+static uint32_t sort_items(uint64_t n, uint32_t key_bytes) {
+  return n < (key_bytes == 8 ? 1u << 20 : 3u << 19) ? SORT_ITEMS_SMALL : SORT_ITEMS;
+}
+
+// Most tiles a sort of n keys in n_segments segments can have (a caller's
+// precounted first pass takes SORT_TILE tiles: no more than these).
+static uint64_t sort_tiles_max(uint64_t n, uint32_t key_bytes, uint64_t n_segments) {
+  const uint64_t tile = (uint64_t)SORT_THREADS * sort_items(n, key_bytes);
+  return (n + tile - 1) / tile + n_segments;
+}
 
 static size_t radix_workspace(uint64_t tiles) {
   const uint64_t hist = tiles * SORT_BINS;
@@ -412,48 +565,115 @@ static size_t radix_workspace(uint64_t tiles) {
   return (size_t)(al(hist * 4) * 2 + al(tgs_scan_workspace_size(hist)));
 }
 
-extern "C" size_t tgs_radix_sort_workspace_size(uint64_t n) { return radix_workspace(sort_tiles(n)); }
+extern "C" size_t tgs_radix_sort_workspace_size(uint64_t n) {
+  return radix_workspace(sort_tiles_max(n, 8, 0));
+}
 
 extern "C" size_t tgs_segmented_sort_workspace_size(uint64_t n, uint32_t n_segments) {
-  return radix_workspace(sort_tiles(n) + n_segments);
+  return radix_workspace(sort_tiles_max(n, 4, n_segments));
+}
+
+// Tile and group bases of the segments (key_off set) for tiles of `items` keys
+// per thread.
+static void radix_bases(RadixSegs& sg, uint32_t items) {
+  const uint32_t tile = SORT_THREADS * items;
+  uint32_t tiles = 0, groups = 0;
+  for (uint32_t s = 0; s < sg.n; ++s) {
+    const uint32_t nt = (uint32_t)(((uint64_t)sg.key_off[s + 1] - sg.key_off[s] + tile - 1) / tile);
+    sg.tile_base[s] = tiles;
+    sg.group_base[s] = groups;
+    tiles += nt;
+    groups += (nt + RADIX_GROUP - 1) / RADIX_GROUP;
+  }
+  sg.tile_base[sg.n] = tiles;
+  sg.group_base[sg.n] = groups;
+}
+
+template <typename K, typename V, int ITEMS, bool LOCAL>
+static int radix_pass(const K* kin, const V* vin, K* kout, V* vout, const RadixSegs& sg, int shift,
+                      int bits, uint32_t* hist, uint32_t* scan_or_groups, void* scan_ws,
+                      bool hist_ready, hipStream_t stream) {
+  const uint32_t tiles = sg.tile_base[sg.n];
+  const uint32_t mask = (1u << bits) - 1u;
+  // a histogram the caller counted keeps the 256-digit layout
+  const uint32_t nbins = hist_ready ? (uint32_t)SORT_BINS : mask + 1u;
+  if (!hist_ready) {
+    hipLaunchKernelGGL((radix_hist_kernel<K, ITEMS, LOCAL>), dim3(tiles), dim3(SORT_THREADS), 0,
+                       stream, kin, sg, shift, mask, nbins, hist, LOCAL ? scan_or_groups : nullptr);
+    TGS_LAUNCH_CHECK("radix_hist");
+  }
+  const uint32_t* counts = hist;
+  if (!LOCAL) {
+    const int rc = exclusive_scan_u32(hist, scan_or_groups, (uint64_t)tiles * nbins, scan_ws, stream);
+    if (rc) return rc;
+    counts = scan_or_groups;
+  }
+  hipLaunchKernelGGL((radix_scatter_kernel<K, V, ITEMS, LOCAL>), dim3(tiles), dim3(SORT_THREADS), 0,
+                     stream, kin, vin, sg, shift, mask, nbins, counts,
+                     LOCAL ? scan_or_groups : nullptr, kout, vout);
+  TGS_LAUNCH_CHECK("radix_scatter");
+  return TGS_OK;
 }
 
 // Runs the passes over key bits [begin_bit, end_bit), splitting the range
 // into the fewest passes of at most 8 bits with widths as even as possible.
+// sg holds the segments' key offsets; first_hist_ready: the first pass's
+// histogram (SORT_TILE tiles, 256 digits) is already in the workspace.
 template <typename K, typename V>
-static int radix_passes(K* keys, V* vals, K* keys_alt, V* vals_alt, const RadixSegs& sg,
+static int radix_passes(K* keys, V* vals, K* keys_alt, V* vals_alt, RadixSegs& sg,
                         int begin_bit, int end_bit, void* workspace, int* selector,
                         hipStream_t stream, bool first_hist_ready = false) {
+  const uint32_t items = first_hist_ready ? SORT_ITEMS : sort_items(sg.key_off[sg.n], sizeof(K));
+  radix_bases(sg, items);
   const uint64_t tiles = sg.tile_base[sg.n];
+  if (tiles == 0) return TGS_OK;
   const uint64_t hist_max = tiles * SORT_BINS;  // the workspace's layout
   auto al = [](uint64_t b) { return (b + 255) & ~255ull; };
   uint8_t* ws = (uint8_t*)workspace;
   uint32_t* hist = (uint32_t*)ws;
   uint32_t* hist_scan = (uint32_t*)(ws + al(hist_max * 4));
   void* scan_ws = ws + 2 * al(hist_max * 4);
+  int passes = (end_bit - begin_bit + 7) / 8;
+  // per-pass group rows of a LOCAL sort, in the space of the scanned histogram
+  // (64 short segments can need more rows than that holds: then the scan runs)
+  const uint64_t group_words = (uint64_t)sg.group_base[sg.n] * SORT_BINS;
+  uint32_t most = 0;
+  for (uint32_t s = 0; s < sg.n; ++s) {
+    const uint32_t nt = sg.tile_base[s + 1] - sg.tile_base[s];
+    most = nt > most ? nt : most;
+  }
+  const bool grouped = most > RADIX_GROUP;
+  const bool local = !first_hist_ready && sg.key_off[sg.n] <= RADIX_LOCAL_KEYS &&
+                     (!grouped || group_words * passes <= hist_max);
+  if (local && grouped) {
+    const int rc = tgs_fill_u32(hist_scan, group_words * passes, 0u, stream);
+    if (rc) return rc;
+  }
   K* kin = keys;
   V* vin = vals;
   K* kout = keys_alt;
   V* vout = vals_alt;
   int sel = 0;
   int shift = begin_bit;
-  int passes = (end_bit - begin_bit + 7) / 8;
+  uint32_t* groups = local && grouped ? hist_scan : nullptr;
   while (shift < end_bit) {
     const int bits = (end_bit - shift + passes - 1) / passes;
-    const uint32_t mask = (1u << bits) - 1u;
-    const bool given = first_hist_ready && shift == begin_bit;
-    // a histogram the caller counted keeps the 256-digit layout
-    const uint32_t nbins = given ? (uint32_t)SORT_BINS : mask + 1u;
-    if (!given) {
-      hipLaunchKernelGGL((radix_hist_kernel<K>), dim3((unsigned)tiles), dim3(SORT_THREADS), 0,
-                         stream, kin, sg, shift, mask, nbins, hist);
-      TGS_LAUNCH_CHECK("radix_hist");
-    }
-    int rc = exclusive_scan_u32(hist, hist_scan, tiles * nbins, scan_ws, stream);
+    int rc;
+    if (local && items == SORT_ITEMS_SMALL)
+      rc = radix_pass<K, V, SORT_ITEMS_SMALL, true>(kin, vin, kout, vout, sg, shift, bits, hist,
+                                                    groups, scan_ws, false, stream);
+    else if (local)
+      rc = radix_pass<K, V, SORT_ITEMS, true>(kin, vin, kout, vout, sg, shift, bits, hist, groups,
+                                              scan_ws, false, stream);
+    else if (items == SORT_ITEMS_SMALL)
+      rc = radix_pass<K, V, SORT_ITEMS_SMALL, false>(kin, vin, kout, vout, sg, shift, bits, hist,
+                                                     hist_scan, scan_ws, false, stream);
+    else
+      rc = radix_pass<K, V, SORT_ITEMS, false>(kin, vin, kout, vout, sg, shift, bits, hist,
+                                               hist_scan, scan_ws,
+                                               first_hist_ready && shift == begin_bit, stream);
     if (rc) return rc;
-    hipLaunchKernelGGL((radix_scatter_kernel<K, V>), dim3((unsigned)tiles), dim3(SORT_THREADS), 0,
-                       stream, kin, vin, sg, shift, mask, nbins, hist_scan, kout, vout);
-    TGS_LAUNCH_CHECK("radix_scatter");
+    if (groups) groups += group_words;
     K* tk = kin;
     kin = kout;
     kout = tk;
@@ -491,8 +711,6 @@ extern "C" int tgs_radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* ke
   sg.n = 1;
   sg.key_off[0] = 0;
   sg.key_off[1] = (uint32_t)n;
-  sg.tile_base[0] = 0;
-  sg.tile_base[1] = (uint32_t)sort_tiles(n);
   return radix_passes<uint64_t, uint32_t>(keys, vals, keys_alt, vals_alt, sg, begin_bit, end_bit,
                                           workspace, selector, stream);
 }
@@ -568,9 +786,9 @@ extern "C" int tgs_radix_sort_pairs_noalloc(uint64_t* keys, uint32_t* vals, uint
                         TGS_ALIGN256((TGS_NOALLOC_SORT_HIST + SCAN_CHUNK - 1) / SCAN_CHUNK * 8ull +
                                      8ull),
                 "scratch smaller than the sort workspace");
-  if (radix_workspace(sort_tiles(n)) > TGS_NOALLOC_SORT_BYTES) {
+  if (tgs_radix_sort_workspace_size(n) > TGS_NOALLOC_SORT_BYTES) {
     tgs_set_error("radix_sort_noalloc: workspace %zu exceeds the scratch array",
-                  radix_workspace(sort_tiles(n)));
+                  tgs_radix_sort_workspace_size(n));
     return TGS_ERR_WORKSPACE;
   }
   void* ws = nullptr;
@@ -580,8 +798,6 @@ extern "C" int tgs_radix_sort_pairs_noalloc(uint64_t* keys, uint32_t* vals, uint
   sg.n = 1;
   sg.key_off[0] = 0;
   sg.key_off[1] = (uint32_t)n;
-  sg.tile_base[0] = 0;
-  sg.tile_base[1] = (uint32_t)sort_tiles(n);
   return radix_passes<uint64_t, uint32_t>(keys, vals, keys_alt, vals_alt, sg, begin_bit, end_bit,
                                           ws, selector, stream);
 }
@@ -666,21 +882,16 @@ static int segmented_sort_u32(uint32_t* keys, void* vals, uint32_t* keys_alt, vo
   sg.n = n_segments;
   sg.key_base = key_base;
   sg.key_cap = key_cap;
-  uint32_t tiles = 0;
   for (uint32_t s = 0; s < n_segments; ++s) {
     TGS_CHECK_ARG(seg_offsets[s + 1] >= seg_offsets[s], "segmented_sort: offsets decrease");
     sg.key_off[s] = seg_offsets[s];
-    sg.tile_base[s] = tiles;
-    tiles += (uint32_t)sort_tiles(seg_offsets[s + 1] - seg_offsets[s]);
   }
   sg.key_off[n_segments] = (uint32_t)n;
-  sg.tile_base[n_segments] = tiles;
   if (workspace_bytes < tgs_segmented_sort_workspace_size(n, n_segments)) {
     tgs_set_error("segmented_sort: workspace %zu < %zu", workspace_bytes,
                   tgs_segmented_sort_workspace_size(n, n_segments));
     return TGS_ERR_WORKSPACE;
   }
-  if (tiles == 0) return TGS_OK;
   if (value_bytes == 4)
     return radix_passes<uint32_t, uint32_t>(keys, (uint32_t*)vals, keys_alt, (uint32_t*)vals_alt,
                                             sg, begin_bit, end_bit, workspace, selector, stream,
