@@ -248,6 +248,24 @@ int tgs_fused_ssim_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1, fl
                        const float* img1, const float* img2, const float* dL_dmap,
                        const float* dm_dmu1, const float* dm_dsigma1_sq, const float* dm_dsigma12,
                        float* dL_dimg1, tgs_stream_t stream);
+/* Mean SSIM without the map (clm_kernels/__init__.py:23-61's fused_ssim):
+ * mean = mean of the map over [crop, H - crop) x [crop, W - crop).  img1 is
+ * NCHW, or NHWC with channels_last; img2 NCHW.  partials: scratch of
+ * tgs_fused_ssim_mean_partials doubles.  img1_copy (optional): img1 in NCHW, for
+ * the backward.  The partial maps (NCHW) are all set or all null. */
+uint64_t tgs_fused_ssim_mean_partials(int32_t B, int32_t CH, int32_t H, int32_t W);
+int tgs_fused_ssim_mean_fwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1, float C2,
+                            const float* img1, int32_t channels_last, const float* img2,
+                            int32_t crop, double* partials, float* mean, float* img1_copy,
+                            float* dm_dmu1, float* dm_dsigma1_sq, float* dm_dsigma12,
+                            hipStream_t stream);
+/* Its backward: dL_dmean is one float on the device, img1 and img2 are NCHW;
+ * dL_dimg1 is written NCHW, or NHWC with channels_last. */
+int tgs_fused_ssim_mean_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, const float* img1,
+                            const float* img2, const float* dL_dmean, int32_t crop,
+                            const float* dm_dmu1, const float* dm_dsigma1_sq,
+                            const float* dm_dsigma12, float* dL_dimg1, int32_t channels_last,
+                            hipStream_t stream);
 /* Fused L1 + SSIM training loss of strategies/base_engine.py:464-488 for B
  * rendered images [B,H,W,3] (HWC) against gt [B,3,H,W]: forward and
  * backward in one pass.  sums[2b] += sum|I_b - gt'_b|, sums[2b+1] += sum SSIM
@@ -257,6 +275,12 @@ int tgs_fused_ssim_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1, fl
 int tgs_tide_loss(int32_t B, int32_t H, int32_t W, const float* images_hwc, const float* gt_chw,
                   float gt_div, float lambda_dssim, double* sums, float* v_images_hwc,
                   tgs_stream_t stream);
+/* The same, with sums written instead of added to (no clear needed): partials is
+ * scratch of tgs_tide_loss_partials doubles, added up in a fixed order. */
+uint64_t tgs_tide_loss_partials(int32_t B, int32_t H, int32_t W);
+int tgs_tide_loss_summed(int32_t B, int32_t H, int32_t W, const float* images_hwc,
+                         const float* gt_chw, float gt_div, float lambda_dssim, double* partials,
+                         double* sums, float* v_images_hwc, hipStream_t stream);
 
 /* ---- resident optimizer ------------------------------------------------ */
 /* Replaces the six _fused_resident_adam_kernel launches of GPUResidentAdam.step

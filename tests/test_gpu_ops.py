@@ -585,6 +585,48 @@ def test_fused_ssim(gpu):
     assert abs(float(val) - float(rm[:, :, 5:-5, 5:-5].mean())) < 1e-5
 
 
+@pytest.mark.parametrize("shape,last", [
+    ((1, 1, 1, 1), False), ((1, 3, 11, 54), True), ((2, 3, 12, 55), False), ((1, 4, 35, 53), True),
+    ((3, 2, 46, 109), False), ((1, 3, 300, 217), True), ((2, 6, 64, 64), False),
+])
+@pytest.mark.parametrize("padding", ["same", "valid"])
+def test_fused_ssim_strips_and_bands(gpu, shape, last, padding):
+    """Edges of the strips (54 columns) and bands, one and three planes per
+    workgroup, both image layouts and paddings: the mean and its gradient in
+    the image's layout, and the map form, against the oracle in float64.  The
+    map's conditioning is that of E[x^2] - mu^2 in float32 (about 5e-6)."""
+    announce(f"fused_ssim shape={shape} channels_last={last} padding={padding}")
+    crop = 5 if padding == "valid" else 0
+    B, CH, H, W = shape
+    if min(H, W) <= 2 * crop:
+        pytest.skip("empty map")
+    g = torch.Generator().manual_seed(H + W)
+    a, b = torch.rand(shape, generator=g), torch.rand(shape, generator=g)
+    rm, d1, d2, d3 = S.ssim_fwd(a.numpy(), b.numpy(), dtype=np.float64)
+    inner = (slice(None), slice(None), slice(crop, H - crop), slice(crop, W - crop))
+    gm = np.zeros(shape)
+    gm[inner] = 0.7 / rm[inner].size
+    ref = S.ssim_bwd(a.numpy(), b.numpy(), gm, d1, d2, d3, dtype=np.float64)
+    da = a.to(gpu)
+    da = (da.permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2) if last else da).requires_grad_()
+    val = fused_ssim(da, b.to(gpu), padding=padding)
+    assert abs(float(val.detach()) - rm[inner].mean()) < 2e-5 * max(1.0, abs(rm[inner].mean()))
+    grad, = torch.autograd.grad(0.7 * val, da)
+    assert grad.stride() == da.stride() or 1 in shape[2:]
+    assert rel_l2(to_np(grad), ref) < 2e-5
+    with torch.no_grad():
+        assert float(fused_ssim(da, b.to(gpu), padding=padding)) == float(val.detach())
+    # the map form under an arbitrary gradient
+    w = torch.randn((B, CH, H - 2 * crop, W - 2 * crop), generator=g)
+    m = FusedSSIMMap.apply(0.01 ** 2, 0.03 ** 2, da, b.to(gpu), padding, True)
+    assert rel_l2(to_np(m), rm[inner]) < 2e-5
+    full = np.zeros(shape)
+    full[inner] = w.numpy()
+    grad, = torch.autograd.grad((m * w.to(gpu)).sum(), da)
+    assert rel_l2(to_np(grad), S.ssim_bwd(a.numpy(), b.numpy(), full, d1, d2, d3,
+                                          dtype=np.float64)) < 2e-5
+
+
 @pytest.mark.parametrize("D,tile,bg", [(3, 16, True), (4, 16, False), (40, 8, True)])
 def test_rasterize_masks(gpu, D, tile, bg):
     """Tile masks: a skipped tile's pixels hold the background (zero without
@@ -690,3 +732,11 @@ def test_valu_probe_sums(gpu, form):
             a = 2.0 ** -a
     ref = np.tile(a.sum(1), blocks)
     np.testing.assert_allclose(to_np(out), ref, rtol=1e-4 if form == 5 else 1e-5)
+
+
+@pytest.mark.parametrize("B,H,W", [(1, 13, 44), (1, 14, 45), (1, 300, 200), (64, 60, 90),
+                                   (400, 58, 45)])
+def test_tide_loss_bands(gpu, B, H, W):
+    """The loss at each kind of band: one output row past a band, several short
+    bands, and batches large enough for long ones."""
+    test_tide_loss_kernel(gpu, B, H, W)

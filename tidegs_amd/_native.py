@@ -94,7 +94,14 @@ SIGNATURES = {
     "tgs_fused_ssim_bwd": (
         ctypes.c_int, [I32, I32, I32, I32, F32, F32, P, P, P, P, P, P, P, P]
     ),
+    "tgs_fused_ssim_mean_partials": (U64, [I32, I32, I32, I32]),
+    "tgs_fused_ssim_mean_fwd": (
+        ctypes.c_int, [I32, I32, I32, I32, F32, F32, P, I32, P, I32, P, P, P, P, P, P, P]),
+    "tgs_fused_ssim_mean_bwd": (
+        ctypes.c_int, [I32, I32, I32, I32, P, P, P, I32, P, P, P, P, I32, P]),
     "tgs_tide_loss": (ctypes.c_int, [I32, I32, I32, P, P, F32, F32, P, P, P]),
+    "tgs_tide_loss_partials": (U64, [I32, I32, I32]),
+    "tgs_tide_loss_summed": (ctypes.c_int, [I32, I32, I32, P, P, F32, F32, P, P, P, P]),
     "tgs_tide_camera_centers": (ctypes.c_int, [U32, P, P, P]),
     "tgs_tide_row_blocks": (U32, [U64]),
     "tgs_tide_visibility": (

@@ -10,17 +10,13 @@
 //   dm/dmu1, dm/dsigma1^2 (= -C D / (A B^2)), dm/dsigma12 (= 2 C / (A B))
 // Backward: dL/dx = G*(g dm/dmu1) + 2 x G*(g dm/dsigma1^2) + y G*(g dm/dsigma12).
 //
-// Layout is given by strides (channel, row, column) so one kernel serves NCHW
-// tensors (drop-in fused_ssim) and the HWC rendered image of the fused step.
-// A 16x16 output tile per 256-thread workgroup with a 26x26 halo in LDS;
-// separable passes in the same order as the reference (x first, then y).
-// The fused-step mode also folds in the L1 term and the clamp(gt/255, 0, 1)
-// target normalisation of strategies/base_engine.py:472-488.
+// Separable passes in the same order as the reference (x first, then y), as
+// wavefronts that stream down a strip of columns.  The fused step's loss also
+// folds in the L1 term and the clamp(gt/255, 0, 1) target normalisation of
+// strategies/base_engine.py:472-488.
 #include "tgs_common.cuh"
 
-#define SS_T 16
-#define SS_R 5
-#define SS_H (SS_T + 2 * SS_R)  // 26
+#define SS_R 5  // window radius
 
 // Normalised Gaussian window, w_i = exp(-(i-5)^2 / 4.5) / sum_j exp(-(j-5)^2 / 4.5).
 __constant__ float c_gauss[11] = {
@@ -29,183 +25,328 @@ __constant__ float c_gauss[11] = {
     0.21300552785396576f,  0.10936068743467331f,   0.036000773310661316f,
     0.0075987582094967365f, 0.001028380123898387f};
 
-struct Img {
-  const float* p;
+__device__ __forceinline__ void lr_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The window's distinct weights (the taps mirror about the centre) in VGPRs, so
+// that every window product takes two VGPR sources (forms that issue in pairs
+// on gfx950).
+struct Taps {
+  float w[6];
+  __device__ __forceinline__ Taps() {
+#pragma unroll
+    for (int t = 0; t < 6; ++t) asm volatile("v_mov_b32 %0, %1" : "=v"(w[t]) : "s"(c_gauss[t]));
+  }
+  __device__ __forceinline__ float operator()(int t) const { return w[t < 6 ? t : 10 - t]; }
+};
+
+#define LR_RING 11  // rows a streaming wavefront keeps in registers: the window's height
+
+// ---------------------------------------------------------------------------
+// Drop-in fused SSIM: forward and backward each in one row-streaming pass.
+//
+// One wavefront per (image, channel, strip of SR_OUT output columns, band of
+// rows); lane L holds column x0 - 5 + L.  The wavefront walks the band's input
+// rows top to bottom (10 more than its output rows), passes each row through a
+// wavefront's LDS row for the horizontal window sums and keeps their last 11
+// rows in registers for the vertical ones: no row is filtered twice and no
+// workgroup barrier is taken.  The step loop is unrolled by the ring length,
+// so every ring index is a constant, and each row is loaded two steps ahead.
+// 16x16 tiles with a 26x26 halo in LDS, the form before, filtered 2.6 rows and
+// columns per output and idled threads at its barriers: one 1080p image of 3
+// channels took 90 us forward and 115 us backward, here 58 and 48 (the backward
+// at 3.1 TB/s; the forward is bound by its window products).
+// The mean form writes neither the map nor its gradient (a constant): forward
+// 20 bytes, backward 24 bytes per value, against 24 + 4 and 28 + 12 with the
+// mean's reduction and the gradient's expansion as passes of their own.
+//
+// The three channel wavefronts of an RGB strip share a workgroup (their reads
+// of a channels-last image are the same lines).
+// ---------------------------------------------------------------------------
+#define SR_OUT (64 - 2 * SS_R)  // output columns per strip
+
+// Band rows for a launch of `planes` planes of H x W: input rows of a band
+// (a multiple of the ring) chosen for the least time of the slowest CU, rows
+// times the larger of a lone wavefront's time per row and the CU's share.
+// `halo`: input rows beyond the output rows; `lone`: the time per row of a
+// workgroup that has its CU to itself, in units of a busy CU's time per row and
+// workgroup.
+static int band_input_rows(int H, int64_t strips_planes, int halo, float lone, int max_periods) {
+  int best = LR_RING * 2;
+  float best_cost = 0.f;
+  for (int k = (halo + LR_RING) / LR_RING; k <= max_periods; ++k) {
+    const int rows = k * LR_RING, band = rows - halo;
+    if (band <= 0) continue;
+    const int64_t wgs = strips_planes * ((H + band - 1) / band);
+    const float per_cu = (float)((wgs + 255) / 256);
+    const float cost = (float)rows * (per_cu > lone ? per_cu : lone);
+    if (best_cost == 0.f || cost < best_cost) {
+      best_cost = cost;
+      best = rows;
+    }
+  }
+  return best;
+}
+
+struct Plane {
   int64_t bs, cs, ys, xs;  // batch, channel, row, column strides (elements)
-  float div;               // value = clamp?(p / div)
-  int clamp01;
-  __device__ __forceinline__ float at(int b, int c, int y, int x, int H, int W) const {
-    if (x < 0 || y < 0 || x >= W || y >= H) return 0.f;
-    float v = p[b * bs + c * cs + (int64_t)y * ys + (int64_t)x * xs] / div;
-    if (clamp01) v = fminf(fmaxf(v, 0.f), 1.f);
-    return v;
-  }
 };
 
-struct OutImg {
-  float* p;
-  int64_t bs, cs, ys, xs;
-  __device__ __forceinline__ float& at(int b, int c, int y, int x) const {
-    return p[b * bs + c * cs + (int64_t)y * ys + (int64_t)x * xs];
-  }
-};
+__global__ void __launch_bounds__(192) ssim_fwd_rows_kernel(
+    int CH, int H, int W, float C1, float C2, const float* __restrict__ img1, Plane lay,
+    const float* __restrict__ img2, float* __restrict__ img1_copy, float* __restrict__ map,
+    float* __restrict__ d_mu1, float* __restrict__ d_s11, float* __restrict__ d_s12,
+    double* __restrict__ partial, int crop, int rows) {
+  __shared__ float2 s_xy[3][64 + 2 * SS_R];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int groups = CH / nw, strips = (W + SR_OUT - 1) / SR_OUT;
+  const int pg = blockIdx.x / strips;  // group of nw planes
+  const int b = pg / groups, c = (pg % groups) * nw + wave;
+  const int band = rows - 2 * SS_R;
+  const int x0 = (blockIdx.x % strips) * SR_OUT, y0 = blockIdx.y * band;
+  const int xi = x0 - SS_R + lane;
+  const bool col_in = xi >= 0 && xi < W;
+  const bool col_out = col_in && lane >= SS_R && lane < SS_R + SR_OUT;
+  const bool col_sum = col_out && xi >= crop && xi < W - crop;
+  const int xc = min(max(xi, 0), W - 1);
+  const int64_t plane = ((int64_t)b * CH + c) * H * W;
+  const float* p1 = img1 + b * lay.bs + c * lay.cs + xc * lay.xs;
+  const float* p2 = img2 + plane + xc;
+  float2* xy = s_xy[wave];
+  const Taps wgt;
+  // values of input row r, loaded from clamped (always valid) addresses
+  // without a branch, so that the two-row prefetch really overlaps
+  auto load_row = [&](int r, float& u, float& w) {
+    const int rc = min(max(r, 0), H - 1);
+    u = p1[rc * lay.ys];
+    w = p2[(int64_t)rc * W];
+  };
+  float Hr[5][LR_RING];
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+#pragma unroll
+    for (int t = 0; t < LR_RING; ++t) Hr[k][t] = 0.f;
+  const int ys = y0 - SS_R;  // first input row
+  float u1, w1, u2, w2;
+  load_row(ys, u1, w1);
+  load_row(ys + 1, u2, w2);
+  float m_acc = 0.f;
 
-// Horizontal pass over the 26 halo rows for the 16 output columns, then the
-// vertical pass for this thread's output pixel.  `q` computes the quantity to
-// filter from the two halo tiles.
-template <int NQ, class Q>
-__device__ __forceinline__ void sep_conv(float (*h)[SS_H][SS_T], Q q, float out[NQ]) {
-  const int tid = threadIdx.x;
-  for (int e = tid; e < SS_H * SS_T; e += 256) {
-    const int r = e / SS_T, c = e % SS_T;
-    float acc[NQ];
+#pragma unroll 1
+  for (int n0 = 0; n0 < rows; n0 += LR_RING) {
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) acc[k] = 0.f;
+    for (int p = 0; p < LR_RING; ++p) {
+      const int n = n0 + p;
+      const int ri = ys + n;
+      const bool ok = col_in && ri >= 0 && ri < H;
+      const float u = ok ? u1 : 0.f, w = ok ? w1 : 0.f;
+      u1 = u2;
+      w1 = w2;
+      load_row(ri + 2, u2, w2);
+      xy[lane + SS_R] = make_float2(u, w);
+      if (img1_copy && col_out && ok && ri >= y0 && ri < y0 + band)
+        img1_copy[plane + (int64_t)ri * W + xi] = u;
+      lr_wave_sync();
+      float h0 = 0.f, h1 = 0.f, h2 = 0.f, h3 = 0.f, h4 = 0.f;
 #pragma unroll
-    for (int t = 0; t < 11; ++t) {
-      float v[NQ];
-      q(r, c + t, v);
+      for (int t = 0; t < 11; ++t) {
+        const float2 v = xy[lane + t];
+        const float wx = wgt(t) * v.x, wy = wgt(t) * v.y;
+        h0 += wx;
+        h1 += wy;
+        h2 = fmaf(wx, v.x, h2);
+        h3 = fmaf(wy, v.y, h3);
+        h4 = fmaf(wx, v.y, h4);
+      }
+      Hr[0][p] = h0;
+      Hr[1][p] = h1;
+      Hr[2][p] = h2;
+      Hr[3][p] = h3;
+      Hr[4][p] = h4;
+      lr_wave_sync();  // every lane has read the row before the next one is written
+      if (n >= 2 * SS_R) {
+        // output row from input rows ri - 10 .. ri (slots p+1 .. p+11)
+        const int ro = ri - SS_R;
+        float f[5];
 #pragma unroll
-      for (int k = 0; k < NQ; ++k) acc[k] += c_gauss[t] * v[k];
+        for (int k = 0; k < 5; ++k) {
+          float acc = wgt(0) * Hr[k][(p + 1) % LR_RING];
+#pragma unroll
+          for (int t = 1; t < 11; ++t) acc = fmaf(wgt(t), Hr[k][(p + 1 + t) % LR_RING], acc);
+          f[k] = acc;
+        }
+        if (col_out && ro < H) {
+          const float mu1 = f[0], mu2 = f[1];
+          const float sigma1_sq = f[2] - mu1 * mu1;
+          const float sigma2_sq = f[3] - mu2 * mu2;
+          const float sigma12 = f[4] - mu1 * mu2;
+          const float Cc = 2.f * mu1 * mu2 + C1;
+          const float D = 2.f * sigma12 + C2;
+          const float A = mu1 * mu1 + mu2 * mu2 + C1;
+          const float Bb = sigma1_sq + sigma2_sq + C2;
+          const float r = 1.f / (A * Bb);
+          const float CD = Cc * D;
+          const float m = CD * r;
+          const int64_t o = plane + (int64_t)ro * W + xi;
+          if (map) map[o] = m;
+          if (d_mu1) {
+            const float rA = Bb * r, rB = A * r;  // 1/A, 1/Bb
+            d_mu1[o] = 2.f * r * (mu2 * D - mu2 * Cc + mu1 * CD * (rB - rA));
+            d_s11[o] = -CD * r * rB;
+            d_s12[o] = 2.f * Cc * r;
+          }
+          if (col_sum && ro >= crop && ro < H - crop) m_acc += m;
+        }
+      }
     }
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) h[k][r][c] = acc[k];
   }
+  if (partial) {
+    const float s = tgs_wave_sum(m_acc);
+    if (lane == 0)
+      partial[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * nw + wave] = (double)s;
+  }
+}
+
+// Mean of the map from the wavefronts' sums, in a fixed order.
+__global__ void __launch_bounds__(256) ssim_mean_kernel(const double* __restrict__ partial,
+                                                        int64_t n, double count,
+                                                        float* __restrict__ mean) {
+  __shared__ double s[256];
+  double acc = 0.0;
+  for (int64_t i = threadIdx.x; i < n; i += 256) acc += partial[i];
+  s[threadIdx.x] = acc;
   __syncthreads();
-  const int ty = tid / SS_T, tx = tid % SS_T;
+  for (int h = 128; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) s[threadIdx.x] += s[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *mean = (float)(s[0] / count);
+}
+
+// dL/dimg1 = G*(g dm/dmu1) + 2 x G*(g dm/dsigma1^2) + y G*(g dm/dsigma12), with
+// g = dL/dmap read from `dmap`, or *g_mean / count inside the crop and 0 outside.
+__global__ void __launch_bounds__(192) ssim_bwd_rows_kernel(
+    int CH, int H, int W, const float* __restrict__ img1, const float* __restrict__ img2,
+    const float* __restrict__ dmap, const float* __restrict__ g_mean, float count, int crop,
+    const float* __restrict__ d_mu1, const float* __restrict__ d_s11,
+    const float* __restrict__ d_s12, float* __restrict__ grad, Plane lay, int rows) {
+  __shared__ float2 s_ab[3][64 + 2 * SS_R];
+  __shared__ float s_c[3][64 + 2 * SS_R];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int groups = CH / nw, strips = (W + SR_OUT - 1) / SR_OUT;
+  const int pg = blockIdx.x / strips;  // group of nw planes
+  const int b = pg / groups, c = (pg % groups) * nw + wave;
+  const int band = rows - 2 * SS_R;
+  const int x0 = (blockIdx.x % strips) * SR_OUT, y0 = blockIdx.y * band;
+  const int xi = x0 - SS_R + lane;
+  const bool col_in = xi >= 0 && xi < W;
+  const bool col_out = col_in && lane >= SS_R && lane < SS_R + SR_OUT;
+  const bool col_g = xi >= crop && xi < W - crop;
+  const int xc = min(max(xi, 0), W - 1);
+  const int64_t plane = ((int64_t)b * CH + c) * H * W;
+  const float g_const = dmap ? 0.f : *g_mean / count;
+  const float *pa = d_mu1 + plane + xc, *pb = d_s11 + plane + xc, *pc = d_s12 + plane + xc;
+  const float *px = img1 + plane + xc, *py = img2 + plane + xc;
+  const float* pd = dmap ? dmap + plane + xc : nullptr;
+  float* out = grad + b * lay.bs + c * lay.cs + xc * lay.xs;
+  float2* ab = s_ab[wave];
+  float* cc = s_c[wave];
+  const Taps wgt;
+  struct Row {
+    float a, b, c, g, x, y;
+  };
+  // the partial maps (and dL/dmap) of row r, x and y of the output row r - 5
+  auto load_row = [&](int r) {
+    const int64_t in = (int64_t)min(max(r, 0), H - 1) * W;
+    const int64_t o = (int64_t)min(max(r - SS_R, 0), H - 1) * W;
+    Row v;
+    v.a = pa[in];
+    v.b = pb[in];
+    v.c = pc[in];
+    v.g = pd ? pd[in] : g_const;
+    v.x = px[o];
+    v.y = py[o];
+    return v;
+  };
+  float Qr[3][LR_RING];
 #pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    float acc = 0.f;
+  for (int k = 0; k < 3; ++k)
 #pragma unroll
-    for (int t = 0; t < 11; ++t) acc += c_gauss[t] * h[k][ty + t][tx];
-    out[k] = acc;
-  }
-}
+    for (int t = 0; t < LR_RING; ++t) Qr[k][t] = 0.f;
+  const int ys = y0 - SS_R;
+  Row r1 = load_row(ys), r2 = load_row(ys + 1);
 
-__global__ void __launch_bounds__(256) ssim_fwd_kernel(int B, int CH, int H, int W, float C1,
-                                                       float C2, Img a, Img b, OutImg map,
-                                                       OutImg d_mu1, OutImg d_s11, OutImg d_s12,
-                                                       double* __restrict__ sums) {
-  __shared__ float s1[SS_H][SS_H];
-  __shared__ float s2[SS_H][SS_H];
-  __shared__ float h[5][SS_H][SS_T];
-  __shared__ float red[2][4];
-  const int bidx = blockIdx.z;
-  const int x0 = blockIdx.x * SS_T, y0 = blockIdx.y * SS_T;
-  const int tid = threadIdx.x;
-  const int ty = tid / SS_T, tx = tid % SS_T;
-  const int px = x0 + tx, py = y0 + ty;
-  const bool inside = px < W && py < H;
-  float l1_acc = 0.f, m_acc = 0.f;
-
-  for (int c = 0; c < CH; ++c) {
-    __syncthreads();
-    for (int e = tid; e < SS_H * SS_H; e += 256) {
-      const int r = e / SS_H, col = e % SS_H;
-      s1[r][col] = a.at(bidx, c, y0 + r - SS_R, x0 + col - SS_R, H, W);
-      s2[r][col] = b.at(bidx, c, y0 + r - SS_R, x0 + col - SS_R, H, W);
-    }
-    __syncthreads();
-    float f[5];
-    sep_conv<5>(h, [&](int r, int col, float v[5]) {
-      const float u = s1[r][col], w = s2[r][col];
-      v[0] = u;
-      v[1] = w;
-      v[2] = u * u;
-      v[3] = w * w;
-      v[4] = u * w;
-    }, f);
-    const float mu1 = f[0], mu2 = f[1];
-    const float sigma1_sq = f[2] - mu1 * mu1;
-    const float sigma2_sq = f[3] - mu2 * mu2;
-    const float sigma12 = f[4] - mu1 * mu2;
-    const float Cc = 2.f * mu1 * mu2 + C1;
-    const float D = 2.f * sigma12 + C2;
-    const float A = mu1 * mu1 + mu2 * mu2 + C1;
-    const float Bb = sigma1_sq + sigma2_sq + C2;
-    const float m = (Cc * D) / (A * Bb);
-    if (inside) {
-      if (map.p) map.at(bidx, c, py, px) = m;
-      if (d_mu1.p) {
-        d_mu1.at(bidx, c, py, px) = (mu2 * 2.f * D) / (A * Bb) - (mu2 * 2.f * Cc) / (A * Bb) -
-                                    (mu1 * 2.f * Cc * D) / (A * A * Bb) +
-                                    (mu1 * 2.f * Cc * D) / (A * Bb * Bb);
-        d_s11.at(bidx, c, py, px) = (-Cc * D) / (A * Bb * Bb);
-        d_s12.at(bidx, c, py, px) = (2.f * Cc) / (A * Bb);
+#pragma unroll 1
+  for (int n0 = 0; n0 < rows; n0 += LR_RING) {
+#pragma unroll
+    for (int p = 0; p < LR_RING; ++p) {
+      const int n = n0 + p;
+      const int ri = ys + n;
+      const Row cur = r1;
+      r1 = r2;
+      r2 = load_row(ri + 2);
+      const bool ok = col_in && ri >= 0 && ri < H &&
+                      (dmap || (col_g && ri >= crop && ri < H - crop));
+      ab[lane + SS_R] = ok ? make_float2(cur.g * cur.a, cur.g * cur.b) : make_float2(0.f, 0.f);
+      cc[lane + SS_R] = ok ? cur.g * cur.c : 0.f;
+      lr_wave_sync();
+      float q0 = 0.f, q1 = 0.f, q2 = 0.f;
+#pragma unroll
+      for (int t = 0; t < 11; ++t) {
+        const float2 v = ab[lane + t];
+        q0 = fmaf(wgt(t), v.x, q0);
+        q1 = fmaf(wgt(t), v.y, q1);
+        q2 = fmaf(wgt(t), cc[lane + t], q2);
       }
-      if (sums) {
-        l1_acc += fabsf(s1[ty + SS_R][tx + SS_R] - s2[ty + SS_R][tx + SS_R]);
-        m_acc += m;
+      Qr[0][p] = q0;
+      Qr[1][p] = q1;
+      Qr[2][p] = q2;
+      lr_wave_sync();
+      if (n >= 2 * SS_R) {
+        const int ro = ri - SS_R;
+        float f[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          float acc = wgt(0) * Qr[k][(p + 1) % LR_RING];
+#pragma unroll
+          for (int t = 1; t < 11; ++t) acc = fmaf(wgt(t), Qr[k][(p + 1 + t) % LR_RING], acc);
+          f[k] = acc;
+        }
+        if (col_out && ro < H) out[ro * lay.ys] = f[0] + 2.f * cur.x * f[1] + cur.y * f[2];
       }
     }
   }
-  if (sums) {
-    const float l1 = tgs_wave_sum(l1_acc);
-    const float ms = tgs_wave_sum(m_acc);
-    const int lane = tid & 63, wave = tid >> 6;
-    if (lane == 0) {
-      red[0][wave] = l1;
-      red[1][wave] = ms;
-    }
-    __syncthreads();
-    if (tid == 0) {
-      atomicAdd(&sums[2 * bidx + 0], (double)(red[0][0] + red[0][1] + red[0][2] + red[0][3]));
-      atomicAdd(&sums[2 * bidx + 1], (double)(red[1][0] + red[1][1] + red[1][2] + red[1][3]));
-    }
-  }
 }
 
-// dL/dimg1.  dmap == null means dL/dmap is the constant `dmap_const` (the
-// fused step's mean-SSIM loss).  When l1_weight != 0 the L1 term
-// l1_weight * sign(x - y) is added (sign(0) = 0, as torch's abs backward).
-__global__ void __launch_bounds__(256) ssim_bwd_kernel(int B, int CH, int H, int W, Img a, Img b,
-                                                       Img dmap, float dmap_const, Img d_mu1,
-                                                       Img d_s11, Img d_s12, float l1_weight,
-                                                       OutImg out) {
-  __shared__ float s[3][SS_H][SS_H];
-  __shared__ float h[3][SS_H][SS_T];
-  const int bidx = blockIdx.z;
-  const int x0 = blockIdx.x * SS_T, y0 = blockIdx.y * SS_T;
-  const int tid = threadIdx.x;
-  const int ty = tid / SS_T, tx = tid % SS_T;
-  const int px = x0 + tx, py = y0 + ty;
-  const bool inside = px < W && py < H;
-  for (int c = 0; c < CH; ++c) {
-    __syncthreads();
-    for (int e = tid; e < SS_H * SS_H; e += 256) {
-      const int r = e / SS_H, col = e % SS_H;
-      const int yy = y0 + r - SS_R, xx = x0 + col - SS_R;
-      const bool in_img = xx >= 0 && yy >= 0 && xx < W && yy < H;
-      const float g = dmap.p ? dmap.at(bidx, c, yy, xx, H, W) : (in_img ? dmap_const : 0.f);
-      s[0][r][col] = g * d_mu1.at(bidx, c, yy, xx, H, W);
-      s[1][r][col] = g * d_s11.at(bidx, c, yy, xx, H, W);
-      s[2][r][col] = g * d_s12.at(bidx, c, yy, xx, H, W);
-    }
-    __syncthreads();
-    float f[3];
-    sep_conv<3>(h, [&](int r, int col, float v[3]) {
-      v[0] = s[0][r][col];
-      v[1] = s[1][r][col];
-      v[2] = s[2][r][col];
-    }, f);
-    if (inside) {
-      const float x = a.at(bidx, c, py, px, H, W);
-      const float y = b.at(bidx, c, py, px, H, W);
-      float gr = f[0] + 2.f * x * f[1] + y * f[2];
-      if (l1_weight != 0.f) {
-        const float d = x - y;
-        gr += d > 0.f ? l1_weight : (d < 0.f ? -l1_weight : 0.f);
-      }
-      out.at(bidx, c, py, px) = gr;
-    }
-  }
+struct SsimGrid {
+  dim3 grid, block;
+  int rows;
+};
+
+// Bands: a lone workgroup's row takes 0.5 us forward and 0.6 us backward, about
+// three times a busy CU's.  Bands of more than 78 rows gain nothing (sixteen
+// 1080p images, 45-, 78- and 133-row bands: forward 780, 758, 766 us, backward
+// 664, 633, 734); one 256x256 image in 12-, 23- and 78-row bands: 15, 20, 49 us.
+static SsimGrid ssim_grid(int64_t B, int64_t CH, int H, int W) {
+  const int nw = CH % 3 == 0 ? 3 : 1;
+  const int64_t planes = B * (CH / nw);
+  const int strips = (W + SR_OUT - 1) / SR_OUT;
+  SsimGrid g;
+  g.rows = band_input_rows(H, planes * strips, 2 * SS_R, 3.f, 8);
+  const int band = g.rows - 2 * SS_R;
+  g.grid = dim3((unsigned)(planes * strips), (H + band - 1) / band);
+  g.block = dim3(64 * nw);
+  return g;
 }
 
-static Img nchw(const float* p, int CH, int H, int W) {
-  return Img{p, (int64_t)CH * H * W, (int64_t)H * W, W, 1, 1.f, 0};
+static Plane nchw(int CH, int H, int W) {
+  return Plane{(int64_t)CH * H * W, (int64_t)H * W, W, 1};
 }
-static OutImg nchw_out(float* p, int CH, int H, int W) {
-  return OutImg{p, (int64_t)CH * H * W, (int64_t)H * W, W, 1};
+static Plane nhwc(int CH, int H, int W) {
+  return Plane{(int64_t)CH * H * W, 1, (int64_t)W * CH, CH};
 }
 
 extern "C" int tgs_fused_ssim_fwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1, float C2,
@@ -217,11 +358,10 @@ extern "C" int tgs_fused_ssim_fwd(int32_t B, int32_t CH, int32_t H, int32_t W, f
   TGS_CHECK_ARG((dm_dmu1 && dm_dsigma1_sq && dm_dsigma12) ||
                     (!dm_dmu1 && !dm_dsigma1_sq && !dm_dsigma12),
                 "fused_ssim_fwd: partial maps must be all set or all null");
-  dim3 grid((W + SS_T - 1) / SS_T, (H + SS_T - 1) / SS_T, B);
-  hipLaunchKernelGGL(ssim_fwd_kernel, grid, dim3(256), 0, stream, B, CH, H, W, C1, C2,
-                     nchw(img1, CH, H, W), nchw(img2, CH, H, W), nchw_out(ssim_map, CH, H, W),
-                     nchw_out(dm_dmu1, CH, H, W), nchw_out(dm_dsigma1_sq, CH, H, W),
-                     nchw_out(dm_dsigma12, CH, H, W), (double*)nullptr);
+  const SsimGrid g = ssim_grid(B, CH, H, W);
+  hipLaunchKernelGGL(ssim_fwd_rows_kernel, g.grid, g.block, 0, stream, CH, H, W, C1, C2, img1,
+                     nchw(CH, H, W), img2, (float*)nullptr, ssim_map, dm_dmu1, dm_dsigma1_sq,
+                     dm_dsigma12, (double*)nullptr, 0, g.rows);
   TGS_RETURN_LAUNCH("tgs_fused_ssim_fwd");
 }
 
@@ -234,12 +374,59 @@ extern "C" int tgs_fused_ssim_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, f
   if ((int64_t)B * CH * H * W == 0) return TGS_OK;
   TGS_CHECK_ARG(img1 && img2 && dL_dmap && dm_dmu1 && dm_dsigma1_sq && dm_dsigma12 && dL_dimg1,
                 "fused_ssim_bwd: null pointer");
-  dim3 grid((W + SS_T - 1) / SS_T, (H + SS_T - 1) / SS_T, B);
-  hipLaunchKernelGGL(ssim_bwd_kernel, grid, dim3(256), 0, stream, B, CH, H, W,
-                     nchw(img1, CH, H, W), nchw(img2, CH, H, W), nchw(dL_dmap, CH, H, W), 0.f,
-                     nchw(dm_dmu1, CH, H, W), nchw(dm_dsigma1_sq, CH, H, W),
-                     nchw(dm_dsigma12, CH, H, W), 0.f, nchw_out(dL_dimg1, CH, H, W));
+  const SsimGrid g = ssim_grid(B, CH, H, W);
+  hipLaunchKernelGGL(ssim_bwd_rows_kernel, g.grid, g.block, 0, stream, CH, H, W, img1, img2,
+                     dL_dmap, (const float*)nullptr, 1.f, 0, dm_dmu1, dm_dsigma1_sq, dm_dsigma12,
+                     dL_dimg1, nchw(CH, H, W), g.rows);
   TGS_RETURN_LAUNCH("tgs_fused_ssim_bwd");
+}
+
+extern "C" uint64_t tgs_fused_ssim_mean_partials(int32_t B, int32_t CH, int32_t H, int32_t W) {
+  if ((int64_t)B * CH * H * W == 0) return 0;
+  const SsimGrid g = ssim_grid(B, CH, H, W);
+  return (uint64_t)g.grid.x * g.grid.y * (g.block.x / 64);
+}
+
+extern "C" int tgs_fused_ssim_mean_fwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1,
+                                       float C2, const float* img1, int32_t channels_last,
+                                       const float* img2, int32_t crop, double* partials,
+                                       float* mean, float* img1_copy, float* dm_dmu1,
+                                       float* dm_dsigma1_sq, float* dm_dsigma12,
+                                       hipStream_t stream) {
+  TGS_CHECK_ARG((int64_t)B * CH * H * W > 0 && crop >= 0 && H > 2 * crop && W > 2 * crop,
+                "fused_ssim_mean_fwd: empty map");
+  TGS_CHECK_ARG(img1 && img2 && partials && mean, "fused_ssim_mean_fwd: null pointer");
+  TGS_CHECK_ARG((dm_dmu1 && dm_dsigma1_sq && dm_dsigma12) ||
+                    (!dm_dmu1 && !dm_dsigma1_sq && !dm_dsigma12),
+                "fused_ssim_mean_fwd: partial maps must be all set or all null");
+  const SsimGrid g = ssim_grid(B, CH, H, W);
+  hipLaunchKernelGGL(ssim_fwd_rows_kernel, g.grid, g.block, 0, stream, CH, H, W, C1, C2, img1,
+                     channels_last ? nhwc(CH, H, W) : nchw(CH, H, W), img2, img1_copy,
+                     (float*)nullptr, dm_dmu1, dm_dsigma1_sq, dm_dsigma12, partials, crop, g.rows);
+  TGS_LAUNCH_CHECK("tgs_fused_ssim_mean_fwd");
+  const double count = (double)B * CH * (H - 2 * crop) * (W - 2 * crop);
+  hipLaunchKernelGGL(ssim_mean_kernel, dim3(1), dim3(256), 0, stream, partials,
+                     (int64_t)tgs_fused_ssim_mean_partials(B, CH, H, W), count, mean);
+  TGS_RETURN_LAUNCH("tgs_fused_ssim_mean_fwd");
+}
+
+extern "C" int tgs_fused_ssim_mean_bwd(int32_t B, int32_t CH, int32_t H, int32_t W,
+                                       const float* img1, const float* img2, const float* dL_dmean,
+                                       int32_t crop, const float* dm_dmu1,
+                                       const float* dm_dsigma1_sq, const float* dm_dsigma12,
+                                       float* dL_dimg1, int32_t channels_last,
+                                       hipStream_t stream) {
+  TGS_CHECK_ARG((int64_t)B * CH * H * W > 0 && crop >= 0 && H > 2 * crop && W > 2 * crop,
+                "fused_ssim_mean_bwd: empty map");
+  TGS_CHECK_ARG(img1 && img2 && dL_dmean && dm_dmu1 && dm_dsigma1_sq && dm_dsigma12 && dL_dimg1,
+                "fused_ssim_mean_bwd: null pointer");
+  const SsimGrid g = ssim_grid(B, CH, H, W);
+  const float count = (float)((double)B * CH * (H - 2 * crop) * (W - 2 * crop));
+  hipLaunchKernelGGL(ssim_bwd_rows_kernel, g.grid, g.block, 0, stream, CH, H, W, img1, img2,
+                     (const float*)nullptr, dL_dmean, count, crop, dm_dmu1, dm_dsigma1_sq,
+                     dm_dsigma12, dL_dimg1, channels_last ? nhwc(CH, H, W) : nchw(CH, H, W),
+                     g.rows);
+  TGS_RETURN_LAUNCH("tgs_fused_ssim_mean_bwd");
 }
 
 // Fused-step loss of strategies/base_engine.py:464-488 for a batch of B
@@ -254,10 +441,10 @@ extern "C" int tgs_fused_ssim_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, f
 // sums[2b] += sum|I-gt'|, sums[2b+1] += sum SSIM (double, caller-zeroed).
 //
 // One wavefront per (image, channel, strip of 44 output columns, band of
-// LR_BAND output rows); lane L holds column x0 - 10 + L, so the strip's
+// output rows); lane L holds column x0 - 10 + L, so the strip's
 // 64 columns cover the outputs and the 10-column halo on each side.  The
-// wavefront walks the band's input rows top to bottom (LR_BAND + 20 of them:
-// 10 rows of halo above and below) and keeps each stage's last 11 rows in
+// wavefront walks the band's `rows` input rows top to bottom (20 more than it
+// outputs: 10 rows of halo above and below) and keeps each stage's last 11 rows in
 // registers, so no row is filtered twice:
 //   input row r:   x, y into an 11-row LDS ring; horizontal window sums of
 //                  x, y, x^2, y^2, xy at the lane's column -> register ring H;
@@ -268,17 +455,7 @@ extern "C" int tgs_fused_ssim_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, f
 // The three channel wavefronts of a strip and band share one workgroup (the
 // HWC image rows they read and write are the same lines).  The step loop is
 // unrolled by the ring length, so every ring index is a constant.
-#define LR_OUT 44                 // output columns per strip
-#define LR_BAND 123               // output rows per band (LR_BAND + 20 = 13 x 11)
-#define LR_ROWS (LR_BAND + 4 * SS_R)
-#define LR_RING 11
-static_assert(LR_ROWS % LR_RING == 0, "band rows must fill whole ring periods");
-
-__device__ __forceinline__ void lr_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+#define LR_OUT 44  // output columns per strip
 
 __global__ void __launch_bounds__(192) tide_loss_rows_kernel(int H, int W,
                                                              const float* __restrict__ images_hwc,
@@ -286,14 +463,16 @@ __global__ void __launch_bounds__(192) tide_loss_rows_kernel(int H, int W,
                                                              float gt_div, float C1, float C2,
                                                              float g_ssim, float g_l1,
                                                              float* __restrict__ v_images_hwc,
-                                                             double* __restrict__ sums) {
+                                                             double* __restrict__ sums,
+                                                             double* __restrict__ partials,
+                                                             int rows) {
   // per channel wavefront: ring of (x, y) rows and one row of scaled partial
   // maps, each padded by the window radius on both sides
   __shared__ float2 s_xy[3][LR_RING][64 + 2 * SS_R];
   __shared__ float4 s_dm[3][64 + 2 * SS_R];
   const int c = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = blockIdx.z;
-  const int x0 = blockIdx.x * LR_OUT, y0 = blockIdx.y * LR_BAND;
+  const int x0 = blockIdx.x * LR_OUT, y0 = blockIdx.y * (rows - 4 * SS_R);
   const int xi = x0 - 2 * SS_R + lane;
   const bool col_in = xi >= 0 && xi < W;
   const bool col_out = col_in && lane >= 2 * SS_R && lane < 2 * SS_R + LR_OUT;
@@ -319,13 +498,7 @@ __global__ void __launch_bounds__(192) tide_loss_rows_kernel(int H, int W,
     u = img[pix * 3];
     g = gtc[pix];
   };
-  // the window's distinct weights (the taps mirror about the centre) in
-  // VGPRs, so that every window product takes two VGPR sources (forms that
-  // issue in pairs on gfx950)
-  float wt[6];
-#pragma unroll
-  for (int t = 0; t < 6; ++t) asm volatile("v_mov_b32 %0, %1" : "=v"(wt[t]) : "s"(c_gauss[t]));
-  auto wgt = [&](int t) { return wt[t < 6 ? t : 10 - t]; };
+  const Taps wgt;
 
   float Hr[5][LR_RING];  // horizontal sums of the last 11 input rows
   float Qr[3][LR_RING];  // horizontal sums of the partial maps, last 11 stats rows
@@ -344,7 +517,7 @@ __global__ void __launch_bounds__(192) tide_loss_rows_kernel(int H, int W,
   float l1_acc = 0.f, m_acc = 0.f;
 
 #pragma unroll 1
-  for (int n0 = 0; n0 < LR_ROWS; n0 += LR_RING) {
+  for (int n0 = 0; n0 < rows; n0 += LR_RING) {
 #pragma unroll
     for (int p = 0; p < LR_RING; ++p) {
       const int n = n0 + p;
@@ -417,7 +590,7 @@ __global__ void __launch_bounds__(192) tide_loss_rows_kernel(int H, int W,
           d0 = 2.f * rAB * (mu2 * D - mu2 * Cc + mu1 * CD * (rB - rA));
           d1 = -CD * rAB * rB;
           d2 = 2.f * Cc * rAB;
-          if (col_out && rs >= y0 && rs < y0 + LR_BAND) m_acc += CD * rAB;
+          if (col_out && rs >= y0 && rs < y0 + rows - 4 * SS_R) m_acc += CD * rAB;
         }
         dm[lane + SS_R] = make_float4(g_ssim * d0, g_ssim * d1, g_ssim * d2, 0.f);
         lr_wave_sync();
@@ -458,24 +631,105 @@ __global__ void __launch_bounds__(192) tide_loss_rows_kernel(int H, int W,
   }
   const float l1 = tgs_wave_sum(l1_acc);
   const float ms = tgs_wave_sum(m_acc);
+  __shared__ float s_red[3][2];
   if (lane == 0) {
-    atomicAdd(&sums[2 * b + 0], (double)l1);
-    atomicAdd(&sums[2 * b + 1], (double)ms);
+    s_red[c][0] = l1;
+    s_red[c][1] = ms;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const double l1_sum = (double)s_red[0][0] + s_red[1][0] + s_red[2][0];
+    const double m_sum = (double)s_red[0][1] + s_red[1][1] + s_red[2][1];
+    if (partials) {
+      double* o = partials + 2 * (((int64_t)b * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x);
+      o[0] = l1_sum;
+      o[1] = m_sum;
+    } else {
+      atomicAdd(&sums[2 * b + 0], l1_sum);
+      atomicAdd(&sums[2 * b + 1], m_sum);
+    }
+  }
+}
+
+// sums[2b], sums[2b + 1] from image b's workgroup sums, in a fixed order.
+__global__ void __launch_bounds__(128) tide_loss_sums_kernel(const double* __restrict__ partials,
+                                                             int per_image,
+                                                             double* __restrict__ sums) {
+  __shared__ double s[128];
+  const double* p = partials + 2 * (int64_t)blockIdx.x * per_image;
+  double acc = 0.0;  // even threads L1, odd threads SSIM
+  for (int i = threadIdx.x; i < 2 * per_image; i += 128) acc += p[i];
+  s[threadIdx.x] = acc;
+  __syncthreads();
+  for (int h = 64; h >= 2; h >>= 1) {
+    if ((int)threadIdx.x < h) s[threadIdx.x] += s[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x < 2) sums[2 * blockIdx.x + threadIdx.x] = s[threadIdx.x];
+}
+
+struct LossGrid {
+  dim3 grid;
+  int rows;
+};
+
+// A lone workgroup takes 0.71 us per row, four on a CU 1.2 us: 2.4 times a busy
+// CU's 0.3 us per row and workgroup.  Bands of 123 rows at every size, the rule
+// before, left small batches to a few long-running wavefronts: one 256x256 image
+// 102 -> 25 us, four 979x546 132 -> 91, one 1080p 126 -> 94; sixteen 1080p images
+// keep the 123 rows (1.10 ms; in 13-row bands 1.86).
+static LossGrid loss_grid(int B, int H, int W) {
+  LossGrid g;
+  const int strips = (W + LR_OUT - 1) / LR_OUT;
+  g.rows = band_input_rows(H, (int64_t)strips * B, 4 * SS_R, 2.4f, 13);
+  const int band = g.rows - 4 * SS_R;
+  g.grid = dim3(strips, (H + band - 1) / band, B);
+  return g;
+}
+
+static int launch_tide_loss(int32_t B, int32_t H, int32_t W, const float* images_hwc,
+                            const float* gt_chw, float gt_div, float lambda_dssim, double* sums,
+                            double* partials, float* v_images_hwc, hipStream_t stream) {
+  TGS_CHECK_ARG(images_hwc && gt_chw && sums && v_images_hwc, "tide_loss: null pointer");
+  TGS_CHECK_ARG((int64_t)H * W * 3 < (1ll << 31), "tide_loss: image too large");
+  const float inv_n = 1.f / (float)((int64_t)3 * H * W);
+  TGS_CHECK_ARG(B <= 65535, "tide_loss: more than 65535 images");
+  const LossGrid g = loss_grid(B, H, W);
+  hipLaunchKernelGGL(tide_loss_rows_kernel, g.grid, dim3(192), 0, stream, H, W, images_hwc, gt_chw,
+                     gt_div, 1e-4f, 9e-4f, -lambda_dssim * inv_n, (1.f - lambda_dssim) * inv_n,
+                     v_images_hwc, sums, partials, g.rows);
+  if (partials) {
+    TGS_LAUNCH_CHECK("tgs_tide_loss");
+    hipLaunchKernelGGL(tide_loss_sums_kernel, dim3(B), dim3(128), 0, stream, partials,
+                       (int)(g.grid.x * g.grid.y), sums);
+  }
+  TGS_RETURN_LAUNCH("tgs_tide_loss");
 }
 
 extern "C" int tgs_tide_loss(int32_t B, int32_t H, int32_t W, const float* images_hwc,
                              const float* gt_chw, float gt_div, float lambda_dssim, double* sums,
                              float* v_images_hwc, hipStream_t stream) {
   if ((int64_t)B * H * W == 0) return TGS_OK;
-  TGS_CHECK_ARG(images_hwc && gt_chw && sums && v_images_hwc, "tide_loss: null pointer");
-  TGS_CHECK_ARG((int64_t)H * W * 3 < (1ll << 31), "tide_loss: image too large");
-  const float inv_n = 1.f / (float)((int64_t)3 * H * W);
-  TGS_CHECK_ARG(B <= 65535, "tide_loss: more than 65535 images");
-  dim3 grid((W + LR_OUT - 1) / LR_OUT, (H + LR_BAND - 1) / LR_BAND, B);
-  hipLaunchKernelGGL(tide_loss_rows_kernel, grid, dim3(192), 0, stream, H, W, images_hwc, gt_chw,
-                     gt_div,
-                     1e-4f, 9e-4f, -lambda_dssim * inv_n, (1.f - lambda_dssim) * inv_n,
-                     v_images_hwc, sums);
-  TGS_RETURN_LAUNCH("tgs_tide_loss");
+  return launch_tide_loss(B, H, W, images_hwc, gt_chw, gt_div, lambda_dssim, sums, nullptr,
+                          v_images_hwc, stream);
+}
+
+// The same with the sums written (not added to): every workgroup leaves its own
+// in `partials` and a small launch adds them in a fixed order.  The atomics of
+// the other form queue on one image's two addresses (one 979x546 image in 33-row
+// bands: 966 workgroups, 95 us with one atomic per wavefront).
+extern "C" uint64_t tgs_tide_loss_partials(int32_t B, int32_t H, int32_t W) {
+  if ((int64_t)B * H * W == 0) return 0;
+  const LossGrid g = loss_grid(B, H, W);
+  return 2ull * g.grid.x * g.grid.y * g.grid.z;
+}
+
+extern "C" int tgs_tide_loss_summed(int32_t B, int32_t H, int32_t W, const float* images_hwc,
+                                    const float* gt_chw, float gt_div, float lambda_dssim,
+                                    double* partials, double* sums, float* v_images_hwc,
+                                    hipStream_t stream) {
+  if ((int64_t)B * H * W == 0) return TGS_OK;
+  TGS_CHECK_ARG(partials, "tide_loss_summed: null pointer");
+  return launch_tide_loss(B, H, W, images_hwc, gt_chw, gt_div, lambda_dssim, sums, partials,
+                          v_images_hwc, stream);
 }

@@ -478,10 +478,10 @@ class TideStep:
         self._end()
         sums = self._buf("loss_sums", 2 * C, torch.float64)
         v_images = self._buf("v_images", C * H * W * 3, torch.float32)
+        partials = self._buf("loss_partials", lib.tgs_tide_loss_partials(C, H, W), torch.float64)
         self._begin("loss")
-        N.call("tgs_fill_u32", N.ptr(sums), 4 * C, 0, s)
-        N.call("tgs_tide_loss", C, H, W, N.ptr(images), N.ptr(gt), self.gt_div,
-               self.lambda_dssim, N.ptr(sums), N.ptr(v_images), s)
+        N.call("tgs_tide_loss_summed", C, H, W, N.ptr(images), N.ptr(gt), self.gt_div,
+               self.lambda_dssim, N.ptr(partials), N.ptr(sums), N.ptr(v_images), s)
         self._end()
         self._begin("raster_bwd")
         N.call("tgs_tide_rasterize_bwd", C, N.ptr(splats), N.ptr(bg), W, H, tw, th,
