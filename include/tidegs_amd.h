@@ -258,14 +258,14 @@ int tgs_fused_ssim_mean_fwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C
                             const float* img1, int32_t channels_last, const float* img2,
                             int32_t crop, double* partials, float* mean, float* img1_copy,
                             float* dm_dmu1, float* dm_dsigma1_sq, float* dm_dsigma12,
-                            hipStream_t stream);
+                            tgs_stream_t stream);
 /* Its backward: dL_dmean is one float on the device, img1 and img2 are NCHW;
  * dL_dimg1 is written NCHW, or NHWC with channels_last. */
 int tgs_fused_ssim_mean_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, const float* img1,
                             const float* img2, const float* dL_dmean, int32_t crop,
                             const float* dm_dmu1, const float* dm_dsigma1_sq,
                             const float* dm_dsigma12, float* dL_dimg1, int32_t channels_last,
-                            hipStream_t stream);
+                            tgs_stream_t stream);
 /* Fused L1 + SSIM training loss of strategies/base_engine.py:464-488 for B
  * rendered images [B,H,W,3] (HWC) against gt [B,3,H,W]: forward and
  * backward in one pass.  sums[2b] += sum|I_b - gt'_b|, sums[2b+1] += sum SSIM
@@ -280,7 +280,7 @@ int tgs_tide_loss(int32_t B, int32_t H, int32_t W, const float* images_hwc, cons
 uint64_t tgs_tide_loss_partials(int32_t B, int32_t H, int32_t W);
 int tgs_tide_loss_summed(int32_t B, int32_t H, int32_t W, const float* images_hwc,
                          const float* gt_chw, float gt_div, float lambda_dssim, double* partials,
-                         double* sums, float* v_images_hwc, hipStream_t stream);
+                         double* sums, float* v_images_hwc, tgs_stream_t stream);
 
 /* ---- resident optimizer ------------------------------------------------ */
 /* Replaces the six _fused_resident_adam_kernel launches of GPUResidentAdam.step
@@ -493,6 +493,29 @@ int tgs_tide_rasterize_bwd(uint32_t C, const float* splats, const float* backgro
                            uint32_t n_isects, const float* alphas, const int32_t* last_ids,
                            const float* v_images, const float* v_alphas, float* splat_grads,
                            tgs_stream_t stream);
+/* The same two calls with the backward split along the tiles' lists, for images
+ * of few tiles: the forward leaves each pixel's state at the end of every
+ * segment of a list, and the backward runs one workgroup per (tile, segment).
+ * tgs_tide_raster_split_items: the items of this size (0: not split, use the
+ * calls above).  states: 1024 floats per item, 16-byte aligned; item_tile: one
+ * int32 per item; neither needs clearing.  Both calls take the same sizes. */
+uint64_t tgs_tide_raster_split_items(uint32_t C, uint32_t tile_width, uint32_t tile_height,
+                                     uint32_t n_isects);
+int tgs_tide_rasterize_fwd_split(uint32_t C, const float* splats, const float* backgrounds,
+                                 uint32_t W, uint32_t H, uint32_t tile_width,
+                                 uint32_t tile_height, const int32_t* tile_offsets,
+                                 const int32_t* flatten_ids, uint32_t n_isects, float* images,
+                                 float* alphas, int32_t* last_ids, float* clear,
+                                 uint64_t clear_words, float* states, int32_t* item_tile,
+                                 tgs_stream_t stream);
+int tgs_tide_rasterize_bwd_split(uint32_t C, const float* splats, const float* backgrounds,
+                                 uint32_t W, uint32_t H, uint32_t tile_width,
+                                 uint32_t tile_height, const int32_t* tile_offsets,
+                                 const int32_t* flatten_ids, uint32_t n_isects,
+                                 const float* alphas, const int32_t* last_ids,
+                                 const float* v_images, const float* v_alphas,
+                                 float* splat_grads, const float* states,
+                                 const int32_t* item_tile, tgs_stream_t stream);
 /* The drop-in rasterizer's 3-channel path (rasterize_to_pixels_fwd.cu:162-284,
  * rasterize_to_pixels_bwd.cu:251-402 with 3 channels): gsplat's SoA tensors
  * means2d [n,2], conics [n,3], colors [n,3], opacities [n] packed into the

@@ -740,3 +740,66 @@ def test_tide_loss_bands(gpu, B, H, W):
     """The loss at each kind of band: one output row past a band, several short
     bands, and batches large enough for long ones."""
     test_tide_loss_kernel(gpu, B, H, W)
+
+
+def _dense_tiles(gpu, n, tw, th, seed, opacity=(0.02, 0.9)):
+    """n Gaussians in every tile of a tw x th image, in list order: (means2d,
+    conics, colors, opacities, offsets, flatten ids), [1, N] splats."""
+    rng = np.random.default_rng(seed)
+    tiles = tw * th
+    N_ = n * tiles
+    org = np.stack([np.tile(np.arange(tw), th), np.repeat(np.arange(th), tw)], 1) * 16.0
+    m = np.repeat(org, n, 0) + rng.uniform(0, 16, (N_, 2))
+    s = rng.uniform(0.6, 2.0, (N_, 2))
+    conics = np.stack([1 / s[:, 0] ** 2, rng.uniform(-0.1, 0.1, N_), 1 / s[:, 1] ** 2], 1)
+    op = rng.uniform(*opacity, N_)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32))[None].to(gpu)  # noqa: E731
+    offs = (torch.arange(tiles, dtype=torch.int32) * n).view(1, th, tw).to(gpu)
+    flat = torch.arange(N_, dtype=torch.int32, device=gpu)
+    return t(m), t(conics), t(rng.uniform(0, 1, (N_, 3))), t(op), offs, flat
+
+
+@pytest.mark.parametrize("n,tw,th,crop,what", [
+    (1, 1, 1, 0, ""), (63, 2, 1, 3, ""), (64, 1, 2, 0, ""), (65, 2, 2, 5, ""), (129, 3, 1, 0, ""),
+    (193, 2, 2, 0, "bg"), (700, 3, 3, 7, "bg"), (200, 4, 1, 0, "inf"), (300, 2, 2, 0, "skip"),
+    (3000, 10, 10, 0, "thin"),     # 300k intersections: segments of 128
+    (6000, 14, 14, 0, "thin"),     # 1.2M: 512
+    (8, 78, 78, 0, ""),            # 6084 tiles, the last size split
+])
+def test_rasterize_split_matches_whole_tiles(gpu, n, tw, th, crop, what):
+    """The backward split along the tiles' lists against the whole-tile kernels
+    (the SoA ones, which absgrad selects): bit-identical images, gradients to
+    the order of the sums (float32, relative 2-norm 2e-5), the same NaN and
+    infinities behind and in front of a Gaussian of infinite colour; lists at
+    the segments' edges, ragged images, backgrounds, offsets that skip the
+    first entries, thin Gaussians that composite past many segments."""
+    announce(f"split raster n={n} tiles={tw}x{th} {what}")
+    from tidegs_amd import _native as N
+    m, q, col, op, offs, flat = _dense_tiles(gpu, n, tw, th, n + tw,
+                                             (0.005, 0.02) if what == "thin" else (0.02, 0.9))
+    W, H = tw * 16 - crop, th * 16 - crop
+    if what == "inf":
+        col[0, n // 2::n, 1] = float("inf")
+        col[0, 70::n, 2] = float("nan")
+    if what == "skip":
+        offs = offs.clone()
+        offs[0, 0, 0] = 150
+    bg = torch.tensor([[0.2, 0.7, 0.4]], device=gpu) if what == "bg" else None
+    assert N.load().tgs_tide_raster_split_items(1, tw, th, flat.numel()) > 0
+    g = torch.Generator(device=gpu).manual_seed(1)
+    v = [torch.randn((1, H, W, k), generator=g, device=gpu) for k in (3, 1)]
+    out = []
+    for absgrad in (False, True):
+        leaves = [t.clone().requires_grad_() for t in (m, q, col, op)]
+        rc, ra = ops.rasterize_to_pixels(*leaves, W, H, 16, offs, flat, backgrounds=bg,
+                                         absgrad=absgrad)
+        out.append((rc, ra, torch.autograd.grad((rc, ra), leaves, v)))
+    (rc, ra, grads), (rc2, ra2, grads2) = out
+    assert torch.equal(torch.nan_to_num(rc, 3.0, 5.0, 7.0), torch.nan_to_num(rc2, 3.0, 5.0, 7.0))
+    assert torch.equal(ra, ra2)
+    for a, b in zip(grads, grads2):
+        a, b = to_np(a), to_np(b)
+        fine = np.isfinite(b)
+        np.testing.assert_array_equal(np.isfinite(a), fine)
+        np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
+        assert rel_l2(a[fine], b[fine]) < 2e-5

@@ -479,20 +479,47 @@ __device__ __forceinline__ void xcd_line_order(uint32_t lin, uint32_t n_lines, u
 }
 
 // ---------------------------------------------------------------------------
+// Split tiles.  A tile's list is one serial chain per pixel, so a small image
+// (256 tiles on 256 CUs) runs one workgroup per CU and waits for the deepest
+// tile.  Split, the forward leaves each pixel's state at the end of every
+// segment of 1 << shift list entries (transmittance, and the colour composited
+// within the segment), and the backward runs one workgroup per (tile, segment):
+// a pixel that composites beyond its segment starts from the stored
+// transmittance, with the later segments' colours as the sum behind.  Sums per
+// segment, not running totals, keep the colour behind free of cancellation,
+// and a non-finite colour where it was: in front of it.
+//   Tile t (camera-major) of range [start, end) has the item numbers t +
+//   (start >> shift) up to the next tile's first: at least one per segment,
+//   and at most n_tiles + (n_isects >> shift) over all tiles.  item_tile[item]
+//   is the item's tile, written by the forward; states[item][pixel] its
+//   segment's {T at its end, r, g, b}.
+// ---------------------------------------------------------------------------
+struct RasterSplit {
+  float4* states;
+  int32_t* item_tile;
+  uint32_t shift;
+  uint32_t items;  // n_tiles + (n_isects >> shift)
+};
+
+// ---------------------------------------------------------------------------
 // Forward
 // ---------------------------------------------------------------------------
 #define RF_BATCH 128  // Gaussians staged per batch
 
-// (up to 4 channels the forward fits 64 VGPRs: 8 wavefronts per SIMD)
+// (up to 4 channels the forward fits 64 VGPRs: 8 wavefronts per SIMD; the split
+// form's 80 for 6: its records read ahead and its segment's colours, in 64
+// registers, spill: 87 -> 105 us at 4056 tiles)
 // COUNT: also count each pixel's composited Gaussians into n_contrib (a
 // measurement aid; the plain variant leaves that counter out of the walk)
-template <int CDIM, int TILE, class Src, bool COUNT = false>
-__global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 8 : 1) raster_fwd_kernel(
+// SPLIT (3 channels): leave the segments' states for a split backward
+template <int CDIM, int TILE, class Src, bool COUNT = false, bool SPLIT = false>
+__global__ void __launch_bounds__(TILE* TILE, SPLIT ? 6 : CDIM <= 4 ? 8 : 1) raster_fwd_kernel(
     RasterGeom G, Src src, const float* __restrict__ backgrounds,
     const int32_t* __restrict__ tile_offsets, const int32_t* __restrict__ flatten_ids,
     float* __restrict__ render_colors, float* __restrict__ render_alphas,
     int32_t* __restrict__ last_ids, float4* __restrict__ clear = nullptr, uint64_t clear_n4 = 0,
-    int32_t* __restrict__ n_contrib = nullptr) {
+    int32_t* __restrict__ n_contrib = nullptr, RasterSplit split = RasterSplit{}) {
+  static_assert(!SPLIT || CDIM == 3, "a segment's state is four floats");
   constexpr int BLOCK = TILE * TILE;
   constexpr int WAVES = BLOCK / 64;
   constexpr int ROWS = 64 / TILE;  // pixel rows per wavefront
@@ -550,14 +577,50 @@ __global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 8 : 1) raster_fwd_kern
   float pix[CDIM];
 #pragma unroll
   for (int k = 0; k < CDIM; ++k) pix[k] = 0.f;
+  // SPLIT: the current segment's share of pix
+  float part[CDIM];
+  uint32_t item0 = 0;
+  bool open = inside;  // the pixel composites in the current segment
+  if (SPLIT) {
+#pragma unroll
+    for (int k = 0; k < CDIM; ++k) part[k] = 0.f;
+    const uint32_t tile_lin = cam * G.tile_h * G.tile_w + tile_id;
+    item0 = tile_lin + ((uint32_t)range_start >> split.shift);
+    // (offsets that decrease name an empty tile)
+    const uint32_t n_items =
+        1u + ((uint32_t)max(range_start, range_end) >> split.shift) -
+        ((uint32_t)range_start >> split.shift);
+    for (uint32_t k = item0 + tr; k < min(item0 + n_items, split.items); k += BLOCK)
+      split.item_tile[k] = (int32_t)tile_lin;
+  }
+  auto close_segment = [&](uint32_t seg) {
+    if (open && item0 + seg < split.items)
+      split.states[(uint64_t)(item0 + seg) * BLOCK + tr] =
+          make_float4(fabsf(T), part[0], part[CDIM > 1 ? 1 : 0], part[CDIM > 2 ? 2 : 0]);
+    open = T > 0.f;
+#pragma unroll
+    for (int k = 0; k < CDIM; ++k) part[k] = 0.f;
+  };
 
-  for (int32_t b = 0; b < n_batches; ++b) {
+  SplatData<CDIM> ahead;  // SPLIT: the next batch's record of this thread
+  int32_t b = 0;
+  for (; b < n_batches; ++b) {
+    if (SPLIT && b > 0 && (((uint32_t)b * BATCH) & ((1u << split.shift) - 1u)) == 0u)
+      close_segment((((uint32_t)b * BATCH) >> split.shift) - 1u);
     if (__syncthreads_count(T < 0.f) >= BLOCK) break;
     const int32_t batch_start = range_start + BATCH * b;
     const int32_t idx = batch_start + (int32_t)tr;
     const bool have = (int)tr < BATCH && idx < range_end;
     SplatData<CDIM> s;
-    if (have) src.load(flatten_ids[idx], s);
+    if (SPLIT) {
+      // few tiles: no other workgroup hides the two dependent loads, so each
+      // batch's records are read during the walk of the batch before
+      if (b == 0 && have) src.load(flatten_ids[idx], ahead);
+      s = ahead;
+      if ((int)tr < BATCH && idx + BATCH < range_end) src.load(flatten_ids[idx + BATCH], ahead);
+    } else if (have) {
+      src.load(flatten_ids[idx], s);
+    }
     bool odd_colour = false;
     if (have) {
       const StagedGeo sg = stage_geo<CDIM>(s);
@@ -603,12 +666,18 @@ __global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 8 : 1) raster_fwd_kern
     // record offset of this batch's last composited Gaussian (0xffff: none);
     // the contributor index is derived from it once per batch, not per step
     uint32_t cur_off = 0xffffu;
-    auto walk = [&](auto safe_tag) {
+    // walks list positions [from, to); the plain variant walks them all
+    auto walk = [&](auto safe_tag, int from, int to) {
       constexpr bool SAFE = decltype(safe_tag)::value;
 #pragma unroll
       for (int W = 0; W < WORDS; ++W) {
-        if (W * 32 >= n_list) break;
+        if (W * 32 >= to) break;
         uint32_t m = T < 0.f ? 0u : mw[W];
+        if (SPLIT) {
+          const int lo = min(max(from - W * 32, 0), 32), hi = min(to - W * 32, 32);
+          m &= (hi >= 32 ? 0xffffffffu : (1u << hi) - 1u) &
+               ~(lo >= 32 ? 0xffffffffu : (1u << lo) - 1u);
+        }
         // every lane runs the body (no exec-mask branches): a lane with no
         // entry left reads staged record 0 and changes nothing; a Gaussian
         // failing the alpha test, or the one that would take T to the
@@ -636,15 +705,37 @@ __global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 8 : 1) raster_fwd_kern
           for (int k = 0; k < CDIM; ++k)
             pix[k] = SAFE ? (comp ? fmaf(rec.col[k], vis, pix[k]) : pix[k])
                           : fmaf(rec.col[k], vis, pix[k]);
+          if (SPLIT) {
+#pragma unroll
+            for (int k = 0; k < CDIM; ++k)
+              part[k] = SAFE ? (comp ? fmaf(rec.col[k], vis, part[k]) : part[k])
+                             : fmaf(rec.col[k], vis, part[k]);
+          }
           cur_off = comp ? off : cur_off;
           if (COUNT) n_comp += comp ? 1 : 0;
           T = comp ? next_T : (stop ? -T : T);
         } while (tgs_ballot(m != 0u));
       }
     };
-    if (safe_walk) walk(std::true_type{});
-    else walk(std::false_type{});
+    int from = 0;
+    if (SPLIT && split.shift == 6 && batch_size > 64) {
+      // 64-entry segments: the list positions of the batch's first half, then
+      // the second half's
+      from = __popcll(hits);
+      if (safe_walk) walk(std::true_type{}, 0, from);
+      else walk(std::false_type{}, 0, from);
+      close_segment(2u * (uint32_t)b);
+    }
+    if (safe_walk) walk(std::true_type{}, from, n_list);
+    else walk(std::false_type{}, from, n_list);
     if (cur_off != 0xffffu) cur_idx = (uint32_t)batch_start + cur_off / (uint32_t)RSZ;
+  }
+  if (SPLIT && n_batches > 0) {
+    // the segment still open: the last batch's (its second half's where that is
+    // a segment of its own); after a break, the one the break was in
+    const uint32_t at = (uint32_t)min(b, n_batches - 1) * BATCH;
+    const uint32_t size = (uint32_t)(range_end - range_start) - at;
+    close_segment((at + (split.shift == 6 && size > 64u ? 64u : 0u)) >> split.shift);
   }
   T = fabsf(T);
   if (inside) {
@@ -706,12 +797,15 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
 #define RB_PAIRS 304
 #define RB_BATCH 64  // Gaussians staged per batch
 
-template <int CDIM, int TILE, class Src, class Sink>
+// SPLIT: workgroup = item (tile, segment) instead of tile
+template <int CDIM, int TILE, class Src, class Sink, bool SPLIT = false>
 __global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 6 : 1) raster_bwd_kernel(
     RasterGeom G, Src src, Sink sink, const float* __restrict__ backgrounds,
     const int32_t* __restrict__ tile_offsets, const int32_t* __restrict__ flatten_ids,
     const float* __restrict__ render_alphas, const int32_t* __restrict__ last_ids,
-    const float* __restrict__ v_render_colors, const float* __restrict__ v_render_alphas) {
+    const float* __restrict__ v_render_colors, const float* __restrict__ v_render_alphas,
+    RasterSplit split = RasterSplit{}) {
+  static_assert(!SPLIT || CDIM == 3, "a segment's state is four floats");
   constexpr int BLOCK = TILE * TILE;
   constexpr int WAVES = BLOCK / 64;
   constexpr int ROWS = 64 / TILE;
@@ -745,9 +839,20 @@ __global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 6 : 1) raster_bwd_kern
   __shared__ float s_stage[WAVES][32 * (Sink::MAY_ABS ? NA : NV)];  // one owner group's values
   __shared__ int32_t s_gid[WAVES][32];            // and their Gaussian ids
 
-  const uint32_t cam = blockIdx.z;
-  uint32_t ty, tx;
-  xcd_line_order(blockIdx.y * G.tile_h + blockIdx.x, G.tile_w, G.tile_h, tx, ty);
+  uint32_t cam, ty, tx;
+  if (SPLIT) {
+    // an item that no tile has (offsets that do not start at 0) holds anything:
+    // the range test below refuses what is not this tile's
+    const uint32_t tile_lin =
+        min((uint32_t)split.item_tile[blockIdx.x], G.C * G.tile_h * G.tile_w - 1u);
+    cam = tile_lin / (G.tile_h * G.tile_w);
+    const uint32_t t = tile_lin - cam * (G.tile_h * G.tile_w);
+    ty = t / G.tile_w;
+    tx = t - ty * G.tile_w;
+  } else {
+    cam = blockIdx.z;
+    xcd_line_order(blockIdx.y * G.tile_h + blockIdx.x, G.tile_w, G.tile_h, tx, ty);
+  }
   const uint32_t tile_id = ty * G.tile_w + tx;
   const uint32_t tr = threadIdx.x;
   static_assert(BATCH == 64, "one list entry per lane");
@@ -765,10 +870,23 @@ __global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 6 : 1) raster_bwd_kern
   const uint64_t pid = img + min((uint64_t)i * G.W + j, (uint64_t)G.W * G.H - 1);
 
   const int32_t* offs = tile_offsets + (uint64_t)cam * G.tile_h * G.tile_w;
-  const int32_t range_start = offs[tile_id];
-  const int32_t range_end = (cam == G.C - 1 && tile_id == G.tile_w * G.tile_h - 1)
-                                ? (int32_t)G.n_isects
-                                : offs[tile_id + 1];
+  const int32_t tile_start = offs[tile_id];
+  const int32_t tile_end = (cam == G.C - 1 && tile_id == G.tile_w * G.tile_h - 1)
+                               ? (int32_t)G.n_isects
+                               : offs[tile_id + 1];
+  // the list entries of this workgroup: the tile's, or its segment's
+  int32_t range_start = tile_start, range_end = tile_end;
+  uint32_t seg = 0;
+  if (SPLIT) {
+    const uint32_t item0 =
+        cam * (G.tile_h * G.tile_w) + tile_id + ((uint32_t)tile_start >> split.shift);
+    if (blockIdx.x < item0) return;
+    seg = blockIdx.x - item0;
+    if (seg >= ((uint32_t)max(tile_end - tile_start, 0) + (1u << split.shift) - 1u) >> split.shift)
+      return;  // an item past the tile's segments
+    range_start = tile_start + (int32_t)(seg << split.shift);
+    range_end = min(tile_end, range_start + (int32_t)(1u << split.shift));
+  }
 
   const float T_final = 1.f - render_alphas[pid];
   float T = T_final;
@@ -790,7 +908,28 @@ __global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 6 : 1) raster_bwd_kern
   // dot product with dL/dcolor, buffer_dot = sum_k buffer_k v_rc_k, and only as
   // tf_term - buffer_dot: the walk carries that difference
   float tf_dot = tf_term;
-  const int32_t bin_final = inside ? last_ids[pid] : -1;
+  int32_t bin_final = inside ? last_ids[pid] : -1;
+  if (SPLIT && bin_final < range_start) bin_final = -1;
+  if (SPLIT && bin_final >= range_end) {
+    // the pixel composites beyond this segment: its transmittance here, and the
+    // colours of its later segments behind.  The walk back from the last
+    // contributor starts at 1 - alpha, the final transmittance as rounded in
+    // the rendered alpha (the reference's rasterize_to_pixels_bwd.cu:92-94), and
+    // carries that rounding to every entry and to the colours behind it: so
+    // does the factor here.
+    const uint32_t seg_final = (uint32_t)(bin_final - tile_start) >> split.shift;
+    const float4* st = split.states + (uint64_t)(blockIdx.x - seg) * BLOCK + tr;
+    const float rounded = T_final / st[(uint64_t)seg_final * BLOCK].x;
+    T = st[(uint64_t)seg * BLOCK].x * rounded;
+    float behind = 0.f;
+    for (uint32_t k = seg_final; k > seg; --k) {
+      const float4 c = st[(uint64_t)k * BLOCK];
+      behind += fmaf(c.w, v_rc[CDIM > 2 ? 2 : 0],
+                     fmaf(c.z, v_rc[CDIM > 1 ? 1 : 0], c.y * v_rc[0]));
+    }
+    tf_dot = fmaf(-rounded, behind, tf_dot);
+    bin_final = range_end - 1;
+  }
   const int32_t wave_bin_final = tgs_wave_max_i32(bin_final);
   // entries behind the tile's last contributor (any pixel's last_id) touch no
   // pixel: the back-to-front walk starts at the last one

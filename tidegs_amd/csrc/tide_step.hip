@@ -1721,6 +1721,95 @@ extern "C" int tgs_tide_rasterize_fwd(uint32_t C, const float* splats, const flo
   TGS_RETURN_LAUNCH("tgs_tide_rasterize_fwd");
 }
 
+// Segment size of a split rasterization (raster.cuh, RasterSplit) as a shift, 0
+// for none.  A workgroup per tile leaves CUs idle until there are some 24 tiles
+// per CU; from there on the forward's extra work and the items' plain order cost
+// more than the even finish gains.  Backward, whole tiles and split, in us:
+//   256 tiles, 41k intersections 128 -> 28 (segments of 64; 128: 44, 256: 66)
+//   475, 87k 124 -> 41; 1000, 311k 162 -> 78; 1000, 4.8M 612 -> 226 (512)
+//   4056, 1.4M 264 -> 219 (512; 64: 251); 4096, 1.9M 398 -> 257
+//   8160, 2.9M 407 -> 420 (512); 32640, 11.6M 1487 -> 1593
+// (the forward takes 0-8% longer).  Shorter segments spread a short list over
+// more workgroups, longer ones spare states and per-workgroup set-up, so the
+// segments are the shortest with at most 4096 of them.
+#define RASTER_SPLIT_TILES 6144
+static uint32_t raster_split_shift(uint64_t n_tiles, uint64_t n_isects) {
+  if (n_tiles > RASTER_SPLIT_TILES || n_isects == 0) return 0;
+  uint32_t shift = 6;
+  while (shift < 9 && (n_isects >> shift) > 4096) ++shift;
+  return shift;
+}
+
+extern "C" uint64_t tgs_tide_raster_split_items(uint32_t C, uint32_t tile_width,
+                                                uint32_t tile_height, uint32_t n_isects) {
+  const uint64_t n_tiles = (uint64_t)C * tile_width * tile_height;
+  const uint32_t shift = raster_split_shift(n_tiles, n_isects);
+  return shift ? n_tiles + (n_isects >> shift) : 0;
+}
+
+static int raster_split_args(uint32_t C, uint32_t tile_width, uint32_t tile_height,
+                             uint32_t n_isects, float* states, int32_t* item_tile,
+                             RasterSplit& sp) {
+  const uint64_t n_tiles = (uint64_t)C * tile_width * tile_height;
+  sp.states = (float4*)states;
+  sp.item_tile = item_tile;
+  sp.shift = raster_split_shift(n_tiles, n_isects);
+  sp.items = (uint32_t)tgs_tide_raster_split_items(C, tile_width, tile_height, n_isects);
+  TGS_CHECK_ARG(sp.shift, "tide_rasterize_split: this size is not split");
+  TGS_CHECK_ARG(states && item_tile && ((uintptr_t)states & 15u) == 0,
+                "tide_rasterize_split: states (16-byte aligned) and item_tile are needed");
+  return TGS_OK;
+}
+
+extern "C" int tgs_tide_rasterize_fwd_split(
+    uint32_t C, const float* splats, const float* backgrounds, uint32_t W, uint32_t H,
+    uint32_t tile_width, uint32_t tile_height, const int32_t* tile_offsets,
+    const int32_t* flatten_ids, uint32_t n_isects, float* images, float* alphas,
+    int32_t* last_ids, float* clear, uint64_t clear_words, float* states, int32_t* item_tile,
+    hipStream_t stream) {
+  TGS_CHECK_ARG(clear_words % 4 == 0 && (clear_words == 0 || clear) &&
+                    ((uintptr_t)clear & 15u) == 0,
+                "tide_rasterize_fwd: clear needs a 16-byte aligned buffer of 4k words");
+  TGS_CHECK_ARG(C && W && H, "tide_rasterize_fwd_split: empty image");
+  TGS_CHECK_ARG(tile_offsets && images && alphas && last_ids && splats && flatten_ids,
+                "tide_rasterize_fwd_split: null");
+  TGS_CHECK_ARG(tile_width * 16 >= W && tile_height * 16 >= H, "tide_rasterize_fwd: tile grid");
+  TGS_CHECK_ARG(C <= 65535 && tile_width <= 65535 && tile_height <= 65535,
+                "tide_rasterize_fwd: at most 65535 cameras and tiles per image side");
+  RasterSplit sp;
+  const int rc = raster_split_args(C, tile_width, tile_height, n_isects, states, item_tile, sp);
+  if (rc) return rc;
+  const RasterGeom G{C, W, H, tile_width, tile_height, n_isects};
+  hipLaunchKernelGGL((raster_fwd_kernel<3, 16, PackedSplats, false, true>), raster_fwd_grid(G),
+                     dim3(256), 0, stream, G, PackedSplats{(const float4*)splats}, backgrounds,
+                     tile_offsets, flatten_ids, images, alphas, last_ids, (float4*)clear,
+                     (uint64_t)clear_words / 4, (int32_t*)nullptr, sp);
+  TGS_RETURN_LAUNCH("tgs_tide_rasterize_fwd_split");
+}
+
+extern "C" int tgs_tide_rasterize_bwd_split(
+    uint32_t C, const float* splats, const float* backgrounds, uint32_t W, uint32_t H,
+    uint32_t tile_width, uint32_t tile_height, const int32_t* tile_offsets,
+    const int32_t* flatten_ids, uint32_t n_isects, const float* alphas, const int32_t* last_ids,
+    const float* v_images, const float* v_alphas, float* splat_grads, const float* states,
+    const int32_t* item_tile, hipStream_t stream) {
+  TGS_CHECK_ARG(C && W && H, "tide_rasterize_bwd_split: empty image");
+  TGS_CHECK_ARG(splats && tile_offsets && flatten_ids && alphas && last_ids && v_images &&
+                    splat_grads,
+                "tide_rasterize_bwd_split: null");
+  TGS_CHECK_ARG(tile_width * 16 >= W && tile_height * 16 >= H, "tide_rasterize_bwd: tile grid");
+  RasterSplit sp;
+  const int rc = raster_split_args(C, tile_width, tile_height, n_isects, (float*)states,
+                                   (int32_t*)item_tile, sp);
+  if (rc) return rc;
+  const RasterGeom G{C, W, H, tile_width, tile_height, n_isects};
+  hipLaunchKernelGGL((raster_bwd_kernel<3, 16, PackedSplats, PackedGrads, true>), dim3(sp.items),
+                     dim3(256), 0, stream, G, PackedSplats{(const float4*)splats},
+                     PackedGrads{splat_grads}, backgrounds, tile_offsets, flatten_ids, alphas,
+                     last_ids, v_images, v_alphas, sp);
+  TGS_RETURN_LAUNCH("tgs_tide_rasterize_bwd_split");
+}
+
 extern "C" int tgs_tide_rasterize_bwd(uint32_t C, const float* splats, const float* backgrounds,
                                       uint32_t W, uint32_t H, uint32_t tile_width,
                                       uint32_t tile_height, const int32_t* tile_offsets,

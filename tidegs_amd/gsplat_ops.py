@@ -447,14 +447,23 @@ class _RasterizeToPixels(torch.autograd.Function):
         dev = means2d.device
         render_alphas = torch.empty((C, height, width, 1), dtype=torch.float32, device=dev)
         last_ids = torch.empty((C, height, width), dtype=torch.int32, device=dev)
-        records = None
+        records = states = item_tile = None
         if ch == 3 and tile_size == 16 and not absgrad:
             render_colors = torch.empty((C, height, width, ch), dtype=torch.float32, device=dev)
             records = _packed_splats(means2d, conics, colors, opacities)
-            N.call("tgs_tide_rasterize_fwd", C, N.ptr(records), N.ptr(backgrounds), width, height,
-                   tw, th, N.ptr(isect_offsets), N.ptr(flatten_ids), flatten_ids.numel(),
-                   N.ptr(render_colors), N.ptr(render_alphas), N.ptr(last_ids), None, None, 0,
-                   _stream())
+            args = (C, N.ptr(records), N.ptr(backgrounds), width, height, tw, th,
+                    N.ptr(isect_offsets), N.ptr(flatten_ids), flatten_ids.numel(),
+                    N.ptr(render_colors), N.ptr(render_alphas), N.ptr(last_ids))
+            # few tiles: split the backward along the tiles' lists
+            items = (N.load().tgs_tide_raster_split_items(C, tw, th, flatten_ids.numel())
+                     if any(ctx.needs_input_grad[:4]) and C * width * height else 0)
+            if items:
+                states = torch.empty((items, 1024), dtype=torch.float32, device=dev)
+                item_tile = torch.empty(items, dtype=torch.int32, device=dev)
+                N.call("tgs_tide_rasterize_fwd_split", *args, None, 0, N.ptr(states),
+                       N.ptr(item_tile), _stream())
+            else:
+                N.call("tgs_tide_rasterize_fwd", *args, None, None, 0, _stream())
         else:
             outs = []
             for s0, w, cw in _channel_chunks(ch):
@@ -478,14 +487,16 @@ class _RasterizeToPixels(torch.autograd.Function):
             render_alphas = torch.where(pmask[..., None], render_alphas,
                                         torch.zeros((), dtype=torch.float32, device=dev))
         ctx.save_for_backward(means2d, conics, colors, opacities, backgrounds, isect_offsets,
-                              flatten_ids, kernel_alphas, render_alphas, last_ids, records, pmask)
+                              flatten_ids, kernel_alphas, render_alphas, last_ids, records, pmask,
+                              states, item_tile)
         ctx.width, ctx.height, ctx.tile_size, ctx.absgrad = width, height, tile_size, absgrad
         return render_colors, render_alphas
 
     @staticmethod
     def backward(ctx, v_render_colors, v_render_alphas):
         (means2d, conics, colors, opacities, backgrounds, isect_offsets, flatten_ids,
-         render_alphas, out_alphas, last_ids, records, pmask) = ctx.saved_tensors
+         render_alphas, out_alphas, last_ids, records, pmask, states,
+         item_tile) = ctx.saved_tensors
         C = isect_offsets.shape[0]
         th, tw = isect_offsets.shape[1], isect_offsets.shape[2]
         ch = colors.shape[-1]
@@ -506,10 +517,15 @@ class _RasterizeToPixels(torch.autograd.Function):
         if records is not None:
             n = opacities.numel()
             grads = torch.zeros((max(n, 1), 9), dtype=torch.float32, device=means2d.device)
-            N.call("tgs_tide_rasterize_bwd", C, N.ptr(records), N.ptr(backgrounds), ctx.width,
-                   ctx.height, tw, th, N.ptr(isect_offsets), N.ptr(flatten_ids),
-                   flatten_ids.numel(), N.ptr(render_alphas), N.ptr(last_ids),
-                   N.ptr(v_render_colors), N.ptr(v_render_alphas), N.ptr(grads), _stream())
+            args = (C, N.ptr(records), N.ptr(backgrounds), ctx.width, ctx.height, tw, th,
+                    N.ptr(isect_offsets), N.ptr(flatten_ids), flatten_ids.numel(),
+                    N.ptr(render_alphas), N.ptr(last_ids), N.ptr(v_render_colors),
+                    N.ptr(v_render_alphas), N.ptr(grads))
+            if states is not None:
+                N.call("tgs_tide_rasterize_bwd_split", *args, N.ptr(states), N.ptr(item_tile),
+                       _stream())
+            else:
+                N.call("tgs_tide_rasterize_bwd", *args, _stream())
             N.call("tgs_unpack_splat_grads", n, N.ptr(grads), N.ptr(v_means2d), N.ptr(v_conics),
                    N.ptr(v_colors), N.ptr(v_opacities), _stream())
         else:

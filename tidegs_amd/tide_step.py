@@ -472,9 +472,18 @@ class TideStep:
         # with timing, also each pixel's composited-Gaussian count (the live
         # (Gaussian, pixel) pairs the backward replays)
         n_contrib = self._buf("n_contrib", C * H * W, torch.int32) if self._count_pairs else None
-        N.call("tgs_tide_rasterize_fwd", C, N.ptr(splats), N.ptr(bg), W, H, tw, th,
-               N.ptr(offsets), N.ptr(fids), n_isects, N.ptr(images), N.ptr(alphas),
-               N.ptr(last_ids), N.ptr(n_contrib), N.ptr(sgrads), sg_words, s)
+        # batches of few tiles split the backward along the tiles' lists
+        items = 0 if self._count_pairs else lib.tgs_tide_raster_split_items(C, tw, th, n_isects)
+        if items:
+            states = self._buf("raster_states", items * 1024, torch.float32)
+            item_tile = self._buf("raster_items", items, torch.int32)
+            N.call("tgs_tide_rasterize_fwd_split", C, N.ptr(splats), N.ptr(bg), W, H, tw, th,
+                   N.ptr(offsets), N.ptr(fids), n_isects, N.ptr(images), N.ptr(alphas),
+                   N.ptr(last_ids), N.ptr(sgrads), sg_words, N.ptr(states), N.ptr(item_tile), s)
+        else:
+            N.call("tgs_tide_rasterize_fwd", C, N.ptr(splats), N.ptr(bg), W, H, tw, th,
+                   N.ptr(offsets), N.ptr(fids), n_isects, N.ptr(images), N.ptr(alphas),
+                   N.ptr(last_ids), N.ptr(n_contrib), N.ptr(sgrads), sg_words, s)
         self._end()
         sums = self._buf("loss_sums", 2 * C, torch.float64)
         v_images = self._buf("v_images", C * H * W * 3, torch.float32)
@@ -484,9 +493,13 @@ class TideStep:
                self.lambda_dssim, N.ptr(partials), N.ptr(sums), N.ptr(v_images), s)
         self._end()
         self._begin("raster_bwd")
-        N.call("tgs_tide_rasterize_bwd", C, N.ptr(splats), N.ptr(bg), W, H, tw, th,
-               N.ptr(offsets), N.ptr(fids), n_isects, N.ptr(alphas), N.ptr(last_ids),
-               N.ptr(v_images), None, N.ptr(sgrads), s)
+        bwd_args = (C, N.ptr(splats), N.ptr(bg), W, H, tw, th, N.ptr(offsets), N.ptr(fids),
+                    n_isects, N.ptr(alphas), N.ptr(last_ids), N.ptr(v_images), None,
+                    N.ptr(sgrads))
+        if items:
+            N.call("tgs_tide_rasterize_bwd_split", *bwd_args, N.ptr(states), N.ptr(item_tile), s)
+        else:
+            N.call("tgs_tide_rasterize_bwd", *bwd_args, s)
         self._end()
 
         # 5. per touched row: projection + SH + activation backward (and, with
