@@ -438,7 +438,8 @@ int tgs_tide_isect_emit_blocked_hist(uint32_t n_entries, const int32_t* cam_offs
 /* Beside the reference's interface: the emission fused with the first pass of
  * the tile-bit sort (the form TideStep uses).  The depth-ordered entries of
  * each camera (cam_offsets: the C + 1 host-side first entries per camera) are
- * taken in blocks of 1024 that never span two cameras.
+ * taken in blocks (256 entries up to 2M of them, else 1024) that never span two
+ * cameras.
  *   tgs_tide_isect_fused_digit_bits  the first pass's width w over tile_n_bits
  *                                    bits (ceil(bits / 8) passes of
  *                                    ceil(bits / passes) bits);

@@ -505,3 +505,11 @@ def test_fused_step_trains(gpu):
     assert bool(torch.isfinite(ts.params).all())
     assert losses[-1] < 0.97 * losses[0]
     assert sum(losses[-5:]) < sum(losses[:5])
+
+
+@pytest.mark.parametrize("V,C,big", [(1, 1, 0.0), (257, 1, 1.0), ((1 << 21) - 1, 3, 0.001),
+                                     (1 << 21, 3, 0.001)])
+def test_fused_emission_block_sizes(gpu, V, C, big):
+    """The fused emission with 256- and with 1024-entry blocks: one entry, one
+    past a block, and either side of the line between the two forms."""
+    test_fused_emission_sort_matches_stable_tile_sort(gpu, V, C, big, 40, 30)

@@ -706,7 +706,7 @@ __global__ void __launch_bounds__(256) tide_isect_emit_blocked_kernel(
 
 // ---------------------------------------------------------------------------
 // Emission fused with the tile-bit sort's first pass.  The depth-ordered
-// entries of each camera are taken in blocks of FE_ENTRIES (a block never
+// entries of each camera are taken in blocks of fe.entries (a block never
 // spans two cameras).  tide_isect_fused_count_kernel counts every block's
 // intersections by first-pass digit (tile & mask) into hist, laid out
 // [camera][digit][block of the camera], so that its exclusive scan is the
@@ -719,13 +719,12 @@ __global__ void __launch_bounds__(256) tide_isect_emit_blocked_kernel(
 // reach memory in emission order.  Stable in the emission order, so the
 // remaining tile-bit passes give the reference's order unchanged.
 // ---------------------------------------------------------------------------
-#define FE_ENTRIES 1024
-#define FE_ITEMS (FE_ENTRIES / 256)
 #define FE_CHUNK 2048
 #define FE_KEYS (FE_CHUNK / 256)
 
 struct FusedEmit {
   uint32_t C;
+  uint32_t entries;                       // entries per block
   uint32_t tw, tile_n_bits;
   uint32_t mask;                          // first-pass digit of a tile: tile & mask
   uint32_t ent_off[TIDE_MAX_CAMS + 1];    // first depth-ordered entry of each camera
@@ -737,8 +736,8 @@ __device__ __forceinline__ void fe_block(const FusedEmit& fe, uint32_t b, uint32
   c = 0;
   while (c + 1 < fe.C && fe.blk_first[c + 1] <= b) ++c;
   bl = b - fe.blk_first[c];
-  e0 = fe.ent_off[c] + bl * FE_ENTRIES;
-  e1 = min(e0 + FE_ENTRIES, fe.ent_off[c + 1]);
+  e0 = fe.ent_off[c] + bl * fe.entries;
+  e1 = min(e0 + fe.entries, fe.ent_off[c + 1]);
 }
 
 // hist word of (camera c, digit d, block bl of c)
@@ -748,6 +747,7 @@ __device__ __forceinline__ uint64_t fe_hist_index(const FusedEmit& fe, uint32_t 
   return (uint64_t)fe.blk_first[c] * (fe.mask + 1u) + (uint64_t)d * nb + bl;
 }
 
+template <int FE_ITEMS>  // entries per thread: fe.entries = 256 * FE_ITEMS
 __global__ void __launch_bounds__(256) tide_isect_fused_count_kernel(
     FusedEmit fe, const uint64_t* __restrict__ rects, uint32_t* __restrict__ hist) {
   __shared__ uint32_t s_cnt[256];
@@ -773,6 +773,7 @@ __global__ void __launch_bounds__(256) tide_isect_fused_count_kernel(
   if (threadIdx.x <= fe.mask) hist[fe_hist_index(fe, c, threadIdx.x, bl)] = s_cnt[threadIdx.x];
 }
 
+template <int FE_ITEMS>
 __global__ void __launch_bounds__(256) tide_isect_fused_scatter_kernel(
     FusedEmit fe, const uint64_t* __restrict__ rects, const uint32_t* __restrict__ hist_scan,
     uint32_t n_isects, uint32_t* __restrict__ keys, int32_t* __restrict__ flatten_ids) {
@@ -1585,6 +1586,22 @@ extern "C" uint32_t tgs_tide_isect_fused_digit_bits(uint32_t tile_n_bits) {
   return (tile_n_bits + passes - 1) / passes;
 }
 
+// Entries per block of the fused emission: few entries make few blocks, each a
+// serial chain of chunks, so up to 2M entries a block takes 256 of them; more
+// entries write longer digit runs from larger blocks.  Count, scan, emission
+// and tile pass with 256 and 1024, in us: 9.6k entries 34 and 52, 37k 41 and
+// 81, 0.46M 58 and 73, 1.1M 188 and 202 (with the depth sort), 3.6M 323 and 303;
+// 58M 1957 and 1418.
+static uint32_t fe_entries(uint32_t n_entries) { return n_entries < (1u << 21) ? 256 : 1024; }
+
+#define FE_LAUNCH(kernel, entries, ...)                                                       \
+  do {                                                                                        \
+    if ((entries) == 256)                                                                     \
+      hipLaunchKernelGGL(kernel<1>, dim3(nb), dim3(256), 0, stream, __VA_ARGS__);             \
+    else                                                                                      \
+      hipLaunchKernelGGL(kernel<4>, dim3(nb), dim3(256), 0, stream, __VA_ARGS__);             \
+  } while (0)
+
 static int fused_emit_setup(uint32_t C, const uint32_t* cam_offsets, uint32_t tile_width,
                             uint32_t tile_n_bits, FusedEmit& fe, uint32_t& n_blocks,
                             const char* who) {
@@ -1595,6 +1612,7 @@ static int fused_emit_setup(uint32_t C, const uint32_t* cam_offsets, uint32_t ti
   TGS_CHECK_ARG(tile_width >= 1 && tile_width <= 255, "%s: tile_width must be in [1, 255]", who);
   fe = FusedEmit{};
   fe.C = C;
+  fe.entries = fe_entries(cam_offsets[C]);
   fe.tw = tile_width;
   fe.tile_n_bits = tile_n_bits;
   fe.mask = (1u << tgs_tide_isect_fused_digit_bits(tile_n_bits)) - 1u;
@@ -1604,7 +1622,7 @@ static int fused_emit_setup(uint32_t C, const uint32_t* cam_offsets, uint32_t ti
                   who);
     fe.ent_off[c] = cam_offsets[c];
     fe.blk_first[c] = (uint32_t)blocks;
-    if (c < C) blocks += (cam_offsets[c + 1] - cam_offsets[c] + FE_ENTRIES - 1) / FE_ENTRIES;
+    if (c < C) blocks += (cam_offsets[c + 1] - cam_offsets[c] + fe.entries - 1) / fe.entries;
   }
   TGS_CHECK_ARG(blocks < (1ull << 31), "%s: too many entry blocks", who);
   n_blocks = (uint32_t)blocks;
@@ -1633,8 +1651,7 @@ extern "C" int tgs_tide_isect_fused_count(uint32_t C, const uint32_t* cam_offset
   TGS_CHECK_ARG(entry_rects && hist, "tide_isect_fused_count: null");
   TGS_CHECK_ARG((uint64_t)nb * (fe.mask + 1u) <= hist_words,
                 "tide_isect_fused_count: histogram buffer too small");
-  hipLaunchKernelGGL(tide_isect_fused_count_kernel, dim3(nb), dim3(256), 0, stream, fe, entry_rects,
-                     hist);
+  FE_LAUNCH(tide_isect_fused_count_kernel, fe.entries, fe, entry_rects, hist);
   TGS_RETURN_LAUNCH("tgs_tide_isect_fused_count");
 }
 
@@ -1655,8 +1672,8 @@ extern "C" int tgs_tide_isect_fused_scatter(uint32_t C, const uint32_t* cam_offs
                 "tide_isect_fused_scatter: histogram buffer too small");
   TGS_CHECK_ARG(C - 1 < (1u << (32 - tile_n_bits)),
                 "tide_isect_fused_scatter: camera | tile keys do not fit 32 bits");
-  hipLaunchKernelGGL(tide_isect_fused_scatter_kernel, dim3(nb), dim3(256), 0, stream, fe,
-                     entry_rects, hist_scan, n_isects, keys, flatten_ids);
+  FE_LAUNCH(tide_isect_fused_scatter_kernel, fe.entries, fe, entry_rects, hist_scan, n_isects, keys,
+            flatten_ids);
   TGS_RETURN_LAUNCH("tgs_tide_isect_fused_scatter");
 }
 
