@@ -320,6 +320,29 @@ int tgs_resident_sophia_step(int64_t n_rows, const void* local_rows, int index_i
 int tgs_block_touch_counts(int64_t n_rows, const void* rows, int index_is_i64,
                            const int64_t* block_starts, const int64_t* block_ends,
                            int64_t n_layout, int64_t* counts, tgs_stream_t stream);
+/* The counts with their check on the device: *go = 1 when they add up to n_rows,
+ * else 0; and the updates that do nothing where *go is 0, so that an update can be
+ * queued before the host has read the counts. */
+int tgs_block_touch_check(int64_t n_rows, const void* rows, int index_is_i64,
+                           const int64_t* block_starts, const int64_t* block_ends,
+                           int64_t n_layout, int64_t* counts, int* go, tgs_stream_t stream);
+int tgs_resident_adam_step_checked(int64_t n_rows, const void* local_rows, int index_is_i64,
+                           const int64_t* block_starts, const int64_t* block_ends,
+                           const int64_t* block_slots, int64_t n_layout, int64_t block_size,
+                           const float* bias_correction1, const float* denom_scale,
+                           int n_components, float* const* params, const float* const* grads,
+                           float* const* exp_avg, float* const* exp_avg_sq,
+                           const int32_t* widths, const int64_t* row_strides, const float* lrs,
+                           float beta1, float beta2, float eps, float batch_size,
+                           int* error_flag, const int* go, tgs_stream_t stream);
+int tgs_resident_sophia_step_checked(int64_t n_rows, const void* local_rows, int index_is_i64,
+                             const int64_t* block_starts, const int64_t* block_ends,
+                             const int64_t* block_slots, int64_t n_layout, int64_t block_size,
+                             int n_components, float* const* params, const float* const* grads,
+                             float* const* exp_avg, float* const* hessian, const int32_t* widths,
+                             const int64_t* row_strides, const float* lrs, float beta1,
+                             float beta2, float eps, float rho, float batch_size,
+                             int update_hessian, int* error_flag, const int* go, tgs_stream_t stream);
 
 /* ---- fused resident step (one launch per stage for a batch of cameras) ---- */
 /* These replace TideGS's per-camera loop (strategies/tide_engine/engine.py:
@@ -371,6 +394,26 @@ int tgs_tide_compact(uint64_t n_rows, uint32_t C, const uint32_t* masks, const u
  * that the depth sort's key range, taken from tgs_tide_visibility's
  * depth_range, holds every key. */
 int tgs_tide_project_fwd(uint32_t n_touched, const uint32_t* n_touched_dev,
+                         const int32_t* touched, const int32_t* visit_base,
+                         const int32_t* visits, const uint32_t* masks, uint32_t C,
+                         const float* params, uint32_t row_stride, const float* viewmats,
+                         const float* Ks,
+                         const float* campos, int32_t W, int32_t H, float eps2d, float near_plane,
+                         float far_plane, float radius_clip, int32_t sh_degree,
+                         uint32_t tile_size, uint32_t tile_width, uint32_t tile_height,
+                         float* splats, uint32_t* depth_keys, uint64_t* entry_rects,
+                         int64_t* isect_totals, uint32_t* depth_range, tgs_stream_t stream);
+/* tgs_tide_camera_centers, the emptied {min, max} pairs of both passes' depth_range
+ * and the cleared isect_totals [C] in one launch; the two passes then run without
+ * set-up launches of their own: the same calls, given the buffers prepared here. */
+int tgs_tide_begin(uint32_t C, const float* viewmats, float* campos, uint32_t* visible_range,
+                   uint32_t* projected_range, int64_t* isect_totals, tgs_stream_t stream);
+int tgs_tide_visibility_begun(uint64_t n_rows, const float* params, uint32_t row_stride, uint32_t C,
+                        const float* viewmats, const float* Ks, const float* campos, int32_t W,
+                        int32_t H, float eps2d,
+                        float near_plane, float far_plane, float radius_clip, uint32_t* masks,
+                        uint32_t* counts, uint32_t* depth_range, tgs_stream_t stream);
+int tgs_tide_project_fwd_begun(uint32_t n_touched, const uint32_t* n_touched_dev,
                          const int32_t* touched, const int32_t* visit_base,
                          const int32_t* visits, const uint32_t* masks, uint32_t C,
                          const float* params, uint32_t row_stride, const float* viewmats,

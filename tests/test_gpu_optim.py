@@ -191,3 +191,37 @@ def test_row_outside_layout_raises(gpu):
     opt.set_resident_blocks([0])
     with pytest.raises(RuntimeError, match="outside every resident block"):
         opt.step(1, gs, torch.tensor([1, 6], device=gpu), _rand(2, 1, gpu))
+
+
+@pytest.mark.parametrize("cls", [GPUResidentAdam, GPUResidentSophia])
+@pytest.mark.parametrize("blocks,block", [(3, 8), (1024, 4), (1025, 4)])
+def test_step_outside_blocks_changes_nothing(gpu, cls, blocks, block):
+    """A touched row outside every block (layouts either side of the counting
+    kernel's two forms): the step raises and the queued update leaves table,
+    moments and step counts as they were; the next valid step advances the
+    touched blocks once, and equals the oracle's first step."""
+    announce(f"{cls.__name__} row outside {blocks} blocks")
+    # every second block-sized slice is resident, so rows in between have no block
+    layout = [(b, slice(2 * b * block, (2 * b + 1) * block)) for b in range(blocks)]
+    mgr = _Manager(layout, gpu)
+    rows = 2 * blocks * block
+    table = _unified(rows, 3, gpu)
+    lrs = [0.01, 0.02, 0.03, 0.04, 0.05, 0.06]
+    gs = _UnifiedGaussians(mgr, table, lrs, (0.9, 0.999), 1e-15)
+    opt = cls(batch_size=1, block_size=block, capacity_blocks=blocks, device="cuda")
+    opt.set_resident_blocks([b for b, _ in layout])
+    grads = lambda n: {name: torch.ones((n, w), device=gpu) for name, _, w, _ in SPECS}  # noqa: E731
+    before, m, v = table.clone(), opt._exp_avg.clone(), opt._exp_avg_sq.clone()
+    bad = torch.tensor([0, block, rows - 2 * block], device=gpu)
+    with pytest.raises(RuntimeError, match="outside every resident block"):
+        opt.step(1, gs, bad, grads(3))
+    torch.cuda.synchronize()
+    assert torch.equal(table, before) and torch.equal(opt._exp_avg, m)
+    assert torch.equal(opt._exp_avg_sq, v) and int(opt.slots.steps.sum()) == 0
+    good = torch.tensor([0, rows - 2 * block], device=gpu)
+    stats = opt.step(2, gs, good, grads(2))
+    assert stats["updated_block_ids"] == [0, blocks - 1] and int(opt.slots.steps.sum()) == 2
+    changed = (table != before).any(1).nonzero().flatten()
+    assert torch.equal(changed, good)
+    if cls is GPUResidentAdam:  # first step of a unit gradient: p -= lr
+        np.testing.assert_allclose(to_np(before - table)[to_np(good), 0], lrs[0], rtol=1e-4)

@@ -16,6 +16,7 @@ import torch
 _LIB_PATH = Path(__file__).resolve().parent / "libtidegs_amd.so"
 _lock = threading.Lock()
 _lib = None
+_entries = {}  # name -> bound entry point of _lib
 
 P = ctypes.c_void_p
 I32 = ctypes.c_int32
@@ -106,11 +107,18 @@ SIGNATURES = {
     "tgs_tide_row_blocks": (U32, [U64]),
     "tgs_tide_visibility": (
         ctypes.c_int, [U64, P, U32, U32, P, P, P, I32, I32, F32, F32, F32, F32, P, P, P, P]),
+    "tgs_tide_visibility_begun": (
+        ctypes.c_int, [U64, P, U32, U32, P, P, P, I32, I32, F32, F32, F32, F32, P, P, P, P]),
     "tgs_tide_compact": (ctypes.c_int, [U64, U32, P, P, P, P, P, P, P, P, P, P]),
     "tgs_tide_project_fwd": (
         ctypes.c_int,
         [U32, P, P, P, P, P, U32, P, U32, P, P, P, I32, I32, F32, F32, F32, F32, I32, U32, U32,
          U32, P, P, P, P, P, P]),
+    "tgs_tide_project_fwd_begun": (
+        ctypes.c_int,
+        [U32, P, P, P, P, P, U32, P, U32, P, P, P, I32, I32, F32, F32, F32, F32, I32, U32, U32,
+         U32, P, P, P, P, P, P]),
+    "tgs_tide_begin": (ctypes.c_int, [U32, P, P, P, P, P, P]),
     "tgs_tide_isect_totals": (ctypes.c_int, [U32, P, P, P, U32, P, P]),
     "tgs_tide_isect_count": (ctypes.c_int, [U32, P, P, P]),
     "tgs_tide_isect_segments": (ctypes.c_int, [U32, P, P, P, P]),
@@ -156,12 +164,23 @@ SIGNATURES = {
         [I64, P, ctypes.c_int, P, P, P, I64, I64, P, P, ctypes.c_int, P, P, P, P, P, P, P,
          F32, F32, F32, F32, P, P],
     ),
+    "tgs_resident_adam_step_checked": (
+        ctypes.c_int,
+        [I64, P, ctypes.c_int, P, P, P, I64, I64, P, P, ctypes.c_int, P, P, P, P, P, P, P,
+         F32, F32, F32, F32, P, P, P],
+    ),
     "tgs_resident_sophia_step": (
         ctypes.c_int,
         [I64, P, ctypes.c_int, P, P, P, I64, I64, ctypes.c_int, P, P, P, P, P, P, P,
          F32, F32, F32, F32, F32, ctypes.c_int, P, P],
     ),
+    "tgs_resident_sophia_step_checked": (
+        ctypes.c_int,
+        [I64, P, ctypes.c_int, P, P, P, I64, I64, ctypes.c_int, P, P, P, P, P, P, P,
+         F32, F32, F32, F32, F32, ctypes.c_int, P, P, P],
+    ),
     "tgs_block_touch_counts": (ctypes.c_int, [I64, P, ctypes.c_int, P, P, I64, P, P]),
+    "tgs_block_touch_check": (ctypes.c_int, [I64, P, ctypes.c_int, P, P, I64, P, P, P]),
     "tgs_ws_copy_rows": (ctypes.c_int, [P, U32, P, P, P, U32, I64, U32, P, U32, P, P]),
     "tgs_ws_fill_global_ids": (ctypes.c_int, [P, U32, P, I64, I64, U32, P]),
     "tgs_ws_unpack_rows": (ctypes.c_int, [P, ctypes.c_int, I64, P, U32, I64, P, U32, U32, P, P]),
@@ -204,6 +223,8 @@ def load() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+        _entries.clear()
+        _entries.update((name, getattr(lib, name)) for name in SIGNATURES)
         _lib = lib
     return _lib
 
@@ -215,8 +236,9 @@ def last_error() -> str:
 
 def call(name: str, *args) -> int:
     """Call an int-returning entry point and raise RuntimeError on failure."""
-    fn = getattr(load(), name)
-    rc = fn(*args)
+    if _lib is None:
+        load()
+    rc = _entries[name](*args)
     if rc != 0:
         raise RuntimeError(f"{name} failed (code {rc}): {last_error()}")
     return rc
@@ -230,7 +252,13 @@ def ptr(t) -> int | None:
 
 
 def stream_handle(device=None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's raw handle (without building a torch stream object:
+    every launch asks for it)."""
+    if device is not None and not isinstance(device, int):
+        device = torch.device(device).index
+    if device is None:
+        device = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 def require_cuda(*tensors, names=None) -> None:

@@ -54,7 +54,8 @@ __global__ void __launch_bounds__(256) resident_optim_unified_kernel(
     int64_t n_rows, const IdxT* __restrict__ local_rows, OptimLayout L,
     const float* __restrict__ bias1, const float* __restrict__ denom_scale, OptimComponents C,
     float beta1, float beta2, float eps, float batch_size, float rho, int update_h,
-    int* __restrict__ error_flag) {
+    int* __restrict__ error_flag, const int* __restrict__ go) {
+  if (go && *go == 0) return;  // a row outside every block: the host raises, nothing changes
   const int lane = threadIdx.x & 63;
   // threadIdx.x >> 6 is the same in every lane of a wavefront; readfirstlane
   // tells the compiler so, which keeps the row range and every address derived
@@ -232,7 +233,8 @@ __global__ void __launch_bounds__(256) resident_optim_kernel(
     int64_t n_rows, const IdxT* __restrict__ local_rows, OptimLayout L,
     const float* __restrict__ bias1, const float* __restrict__ denom_scale, OptimComponents C,
     float beta1, float beta2, float eps, float batch_size, float rho, int update_h,
-    int* __restrict__ error_flag) {
+    int* __restrict__ error_flag, const int* __restrict__ go) {
+  if (go && *go == 0) return;  // a row outside every block: the host raises, nothing changes
   const int lane = threadIdx.x & 63;
   const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) +
                        __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -386,6 +388,62 @@ static int fill_components(OptimComponents& C, int n_comp, float* const* params,
   return TGS_OK;
 }
 
+// The counts of a whole layout and their check in one workgroup: *go = 1 when they
+// add up to n_rows (every row lies in exactly one block), else 0.  The update can
+// then be queued behind the count without the host reading it in between, and
+// does nothing where the host will raise.
+// (Layouts of more than TOUCH_CHECK_THREADS blocks count with a workgroup per 256
+// of them and add up after: one workgroup searches 1024 blocks in 13 us, 8000 in
+// eight such rounds.)
+#define TOUCH_CHECK_THREADS 1024
+__device__ __forceinline__ void touch_check_sum(int64_t sum, int64_t n_rows, int* go) {
+  __shared__ int64_t s_sum[TOUCH_CHECK_THREADS / 64];
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int64_t total = 0;
+#pragma unroll
+    for (int w = 0; w < TOUCH_CHECK_THREADS / 64; ++w) total += s_sum[w];
+    *go = total == n_rows ? 1 : 0;
+  }
+}
+
+__global__ void __launch_bounds__(TOUCH_CHECK_THREADS) touch_counts_sum_kernel(
+    int64_t n_rows, int64_t n, const int64_t* __restrict__ counts, int* __restrict__ go) {
+  int64_t sum = 0;
+  for (int64_t i = threadIdx.x; i < n; i += TOUCH_CHECK_THREADS) sum += counts[i];
+  touch_check_sum(sum, n_rows, go);
+}
+
+template <typename IdxT>
+__global__ void __launch_bounds__(TOUCH_CHECK_THREADS) block_touch_check_kernel(
+    int64_t n_rows, const IdxT* __restrict__ rows, OptimLayout L, int64_t* __restrict__ counts,
+    int* __restrict__ go) {
+  int64_t sum = 0;
+  for (int64_t i = threadIdx.x; i < L.n; i += TOUCH_CHECK_THREADS) {
+    // both bounds in step: two independent probes per round
+    const int64_t k0 = L.starts[i], k1 = L.ends[i];
+    int64_t lo0 = 0, hi0 = n_rows, lo1 = 0, hi1 = n_rows;
+    while (lo0 < hi0 || lo1 < hi1) {
+      const int64_t m0 = (lo0 + hi0) >> 1, m1 = (lo1 + hi1) >> 1;
+      const int64_t r0 = lo0 < hi0 ? (int64_t)rows[m0] : 0, r1 = lo1 < hi1 ? (int64_t)rows[m1] : 0;
+      if (lo0 < hi0) {
+        if (r0 < k0) lo0 = m0 + 1;
+        else hi0 = m0;
+      }
+      if (lo1 < hi1) {
+        if (r1 < k1) lo1 = m1 + 1;
+        else hi1 = m1;
+      }
+    }
+    counts[i] = lo1 - lo0;
+    sum += lo1 - lo0;
+  }
+  touch_check_sum(sum, n_rows, go);
+}
+
 template <bool SOPHIA>
 static int launch_optim(int64_t n_rows, const void* local_rows, int index_is_i64,
                         const int64_t* starts, const int64_t* ends, const int64_t* slots,
@@ -394,7 +452,7 @@ static int launch_optim(int64_t n_rows, const void* local_rows, int index_is_i64
                         const float* const* grads, float* const* m, float* const* v,
                         const int32_t* widths, const int64_t* strides, const float* lrs,
                         float beta1, float beta2, float eps, float batch_size, float rho,
-                        int update_h, int* error_flag, hipStream_t stream) {
+                        int update_h, int* error_flag, const int* go, hipStream_t stream) {
   TGS_CHECK_ARG(n_rows >= 0, "n_rows must be >= 0");
   if (n_rows == 0) return TGS_OK;
   TGS_CHECK_ARG(local_rows && starts && ends && slots && error_flag, "null index pointer");
@@ -424,7 +482,7 @@ static int launch_optim(int64_t n_rows, const void* local_rows, int index_is_i64
 #define TGS_OPTIM_LAUNCH(KERNEL, IDX)                                                     \
   hipLaunchKernelGGL((KERNEL<IDX, SOPHIA>), dim3((unsigned)blocks), dim3(threads), 0, stream,  \
                      n_rows, (const IDX*)local_rows, L, bias1, denom_scale, C, beta1, beta2, eps, \
-                     batch_size, rho, update_h, error_flag)
+                     batch_size, rho, update_h, error_flag, go)
   if (C.unified) {
     if (index_is_i64)
       TGS_OPTIM_LAUNCH(resident_optim_unified_kernel, int64_t);
@@ -450,7 +508,7 @@ extern "C" int tgs_resident_adam_step(
   return launch_optim<false>(n_rows, local_rows, index_is_i64, block_starts, block_ends,
                              block_slots, n_layout, block_size, bias_correction1, denom_scale,
                              n_components, params, grads, exp_avg, exp_avg_sq, widths, row_strides,
-                             lrs, beta1, beta2, eps, batch_size, 0.f, 1, error_flag, stream);
+                             lrs, beta1, beta2, eps, batch_size, 0.f, 1, error_flag, nullptr, stream);
 }
 
 extern "C" int tgs_resident_sophia_step(
@@ -463,7 +521,37 @@ extern "C" int tgs_resident_sophia_step(
   return launch_optim<true>(n_rows, local_rows, index_is_i64, block_starts, block_ends,
                             block_slots, n_layout, block_size, nullptr, nullptr, n_components,
                             params, grads, exp_avg, hessian, widths, row_strides, lrs, beta1,
-                            beta2, eps, batch_size, rho, update_hessian, error_flag, stream);
+                            beta2, eps, batch_size, rho, update_hessian, error_flag, nullptr, stream);
+}
+
+// The same updates behind tgs_block_touch_check: nothing changes where *go is 0.
+extern "C" int tgs_resident_adam_step_checked(
+    int64_t n_rows, const void* local_rows, int index_is_i64, const int64_t* block_starts,
+    const int64_t* block_ends, const int64_t* block_slots, int64_t n_layout, int64_t block_size,
+    const float* bias_correction1, const float* denom_scale, int n_components,
+    float* const* params, const float* const* grads, float* const* exp_avg,
+    float* const* exp_avg_sq, const int32_t* widths, const int64_t* row_strides, const float* lrs,
+    float beta1, float beta2, float eps, float batch_size, int* error_flag, const int* go,
+    hipStream_t stream) {
+  TGS_CHECK_ARG(go, "null go flag");
+  return launch_optim<false>(n_rows, local_rows, index_is_i64, block_starts, block_ends,
+                             block_slots, n_layout, block_size, bias_correction1, denom_scale,
+                             n_components, params, grads, exp_avg, exp_avg_sq, widths, row_strides,
+                             lrs, beta1, beta2, eps, batch_size, 0.f, 1, error_flag, go, stream);
+}
+
+extern "C" int tgs_resident_sophia_step_checked(
+    int64_t n_rows, const void* local_rows, int index_is_i64, const int64_t* block_starts,
+    const int64_t* block_ends, const int64_t* block_slots, int64_t n_layout, int64_t block_size,
+    int n_components, float* const* params, const float* const* grads, float* const* exp_avg,
+    float* const* hessian, const int32_t* widths, const int64_t* row_strides, const float* lrs,
+    float beta1, float beta2, float eps, float rho, float batch_size, int update_hessian,
+    int* error_flag, const int* go, hipStream_t stream) {
+  TGS_CHECK_ARG(go, "null go flag");
+  return launch_optim<true>(n_rows, local_rows, index_is_i64, block_starts, block_ends,
+                            block_slots, n_layout, block_size, nullptr, nullptr, n_components,
+                            params, grads, exp_avg, hessian, widths, row_strides, lrs, beta1,
+                            beta2, eps, batch_size, rho, update_hessian, error_flag, go, stream);
 }
 
 extern "C" int tgs_block_touch_counts(int64_t n_rows, const void* rows, int index_is_i64,
@@ -480,4 +568,30 @@ extern "C" int tgs_block_touch_counts(int64_t n_rows, const void* rows, int inde
     hipLaunchKernelGGL(block_touch_counts_kernel<int32_t>, dim3(tgs_blocks(n_layout, 256)),
                        dim3(256), 0, stream, n_rows, (const int32_t*)rows, L, counts);
   TGS_RETURN_LAUNCH("tgs_block_touch_counts");
+}
+
+extern "C" int tgs_block_touch_check(int64_t n_rows, const void* rows, int index_is_i64,
+                                     const int64_t* block_starts, const int64_t* block_ends,
+                                     int64_t n_layout, int64_t* counts, int* go,
+                                     hipStream_t stream) {
+  TGS_CHECK_ARG(n_layout >= 0 && n_rows >= 0, "negative size");
+  TGS_CHECK_ARG(go && (n_layout == 0 || (block_starts && block_ends && counts)) &&
+                    (rows || n_rows == 0),
+                "null pointer");
+  if (n_layout > TOUCH_CHECK_THREADS) {
+    const int rc = tgs_block_touch_counts(n_rows, rows, index_is_i64, block_starts, block_ends,
+                                          n_layout, counts, stream);
+    if (rc) return rc;
+    hipLaunchKernelGGL(touch_counts_sum_kernel, dim3(1), dim3(TOUCH_CHECK_THREADS), 0, stream,
+                       n_rows, n_layout, counts, go);
+    TGS_RETURN_LAUNCH("tgs_block_touch_check");
+  }
+  OptimLayout L{block_starts, block_ends, nullptr, n_layout, 0, -1};
+  if (index_is_i64)
+    hipLaunchKernelGGL(block_touch_check_kernel<int64_t>, dim3(1), dim3(TOUCH_CHECK_THREADS), 0,
+                       stream, n_rows, (const int64_t*)rows, L, counts, go);
+  else
+    hipLaunchKernelGGL(block_touch_check_kernel<int32_t>, dim3(1), dim3(TOUCH_CHECK_THREADS), 0,
+                       stream, n_rows, (const int32_t*)rows, L, counts, go);
+  TGS_RETURN_LAUNCH("tgs_block_touch_check");
 }

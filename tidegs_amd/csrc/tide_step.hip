@@ -1318,8 +1318,8 @@ __global__ void __launch_bounds__(FUSED_THREADS) tide_project_bwd_optim_kernel(
 // Camera centres: the translation of inverse(viewmat) for an affine world->camera
 // matrix [A | t; 0 0 0 1], i.e. -A^{-1} t (engine.py:459 via the SH
 // directions), evaluated in double from the adjugate.
-__global__ void tide_camera_centers_kernel(uint32_t C, const float* __restrict__ viewmats,
-                                           float* __restrict__ campos) {
+__device__ __forceinline__ void camera_center(uint32_t C, const float* __restrict__ viewmats,
+                                              float* __restrict__ campos) {
   const uint32_t c = threadIdx.x;
   if (c >= C) return;
   const float* M = viewmats + (uint64_t)c * 16;
@@ -1346,6 +1346,11 @@ __global__ void tide_camera_centers_kernel(uint32_t C, const float* __restrict__
     campos[c * 3 + i] = (float)(-(adj[i][0] * t[0] + adj[i][1] * t[1] + adj[i][2] * t[2]) / det);
 }
 
+__global__ void tide_camera_centers_kernel(uint32_t C, const float* __restrict__ viewmats,
+                                           float* __restrict__ campos) {
+  camera_center(C, viewmats, campos);
+}
+
 // ---------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------
@@ -1353,6 +1358,29 @@ static int check_cams(uint32_t C) {
   TGS_CHECK_ARG(C >= 1 && C <= TIDE_MAX_CAMS, "tide step: 1..%d cameras per batch (got %u)",
                 TIDE_MAX_CAMS, C);
   return TGS_OK;
+}
+
+// The step's small set-up in one launch: camera centres, both depth-key ranges
+// emptied, the intersection totals cleared (as launches of their own they cost
+// 3 us each plus their gaps, of a 340 us step at 10k Gaussians).
+__global__ void __launch_bounds__(2 * TIDE_RANGE_SLOTS) tide_begin_kernel(
+    uint32_t C, const float* __restrict__ viewmats, float* __restrict__ campos,
+    uint32_t* __restrict__ range0, uint32_t* __restrict__ range1, int64_t* __restrict__ totals) {
+  camera_center(C, viewmats, campos);
+  if (threadIdx.x < C) totals[threadIdx.x] = 0;
+  range0[threadIdx.x] = range1[threadIdx.x] = (threadIdx.x & 1u) ? 0u : 0xffffffffu;
+}
+
+extern "C" int tgs_tide_begin(uint32_t C, const float* viewmats, float* campos,
+                              uint32_t* visible_range, uint32_t* projected_range,
+                              int64_t* isect_totals, hipStream_t stream) {
+  int rc = check_cams(C);
+  if (rc) return rc;
+  TGS_CHECK_ARG(viewmats && campos && visible_range && projected_range && isect_totals,
+                "tide_begin: null");
+  hipLaunchKernelGGL(tide_begin_kernel, dim3(1), dim3(2 * TIDE_RANGE_SLOTS), 0, stream, C, viewmats,
+                     campos, visible_range, projected_range, isect_totals);
+  TGS_RETURN_LAUNCH("tgs_tide_begin");
 }
 
 extern "C" int tgs_tide_camera_centers(uint32_t C, const float* viewmats, float* campos,
@@ -1368,15 +1396,15 @@ extern "C" uint32_t tgs_tide_row_blocks(uint64_t n_rows) {
   return (uint32_t)((n_rows + VIS_THREADS - 1) / VIS_THREADS);
 }
 
-extern "C" int tgs_tide_visibility(uint64_t n_rows, const float* params, uint32_t row_stride,
+static int tide_visibility(uint64_t n_rows, const float* params, uint32_t row_stride,
                                    uint32_t C,
                                    const float* viewmats, const float* Ks, const float* campos,
                                    int32_t W, int32_t H, float eps2d, float near_plane,
                                    float far_plane, float radius_clip, uint32_t* masks,
-                                   uint32_t* counts, uint32_t* depth_range, hipStream_t stream) {
+                                   uint32_t* counts, uint32_t* depth_range, bool init, hipStream_t stream) {
   int rc = check_cams(C);
   if (rc) return rc;
-  if (depth_range)
+  if (init && depth_range)
     hipLaunchKernelGGL(tide_range_init_kernel, dim3(1), dim3(2 * TIDE_RANGE_SLOTS), 0, stream,
                        depth_range);
   if (n_rows == 0) TGS_RETURN_LAUNCH("tgs_tide_visibility");
@@ -1388,6 +1416,29 @@ extern "C" int tgs_tide_visibility(uint64_t n_rows, const float* params, uint32_
                      0, stream, n_rows, params, row_stride, tc, W, H, eps2d, near_plane, far_plane,
                      radius_clip, masks, counts, depth_range);
   TGS_RETURN_LAUNCH("tgs_tide_visibility");
+}
+
+extern "C" int tgs_tide_visibility(uint64_t n_rows, const float* params, uint32_t row_stride,
+                                   uint32_t C, const float* viewmats, const float* Ks,
+                                   const float* campos, int32_t W, int32_t H, float eps2d,
+                                   float near_plane, float far_plane, float radius_clip,
+                                   uint32_t* masks, uint32_t* counts, uint32_t* depth_range,
+                                   hipStream_t stream) {
+  return tide_visibility(n_rows, params, row_stride, C, viewmats, Ks, campos, W, H, eps2d,
+                         near_plane, far_plane, radius_clip, masks, counts, depth_range, true,
+                         stream);
+}
+
+// After tgs_tide_begin: the range is already empty.
+extern "C" int tgs_tide_visibility_begun(uint64_t n_rows, const float* params, uint32_t row_stride,
+                                   uint32_t C, const float* viewmats, const float* Ks,
+                                   const float* campos, int32_t W, int32_t H, float eps2d,
+                                   float near_plane, float far_plane, float radius_clip,
+                                   uint32_t* masks, uint32_t* counts, uint32_t* depth_range,
+                                   hipStream_t stream) {
+  return tide_visibility(n_rows, params, row_stride, C, viewmats, Ks, campos, W, H, eps2d,
+                         near_plane, far_plane, radius_clip, masks, counts, depth_range, false,
+                         stream);
 }
 
 extern "C" int tgs_tide_compact(uint64_t n_rows, uint32_t C, const uint32_t* masks,
@@ -1410,7 +1461,7 @@ extern "C" int tgs_tide_compact(uint64_t n_rows, uint32_t C, const uint32_t* mas
   TGS_RETURN_LAUNCH("tgs_tide_compact");
 }
 
-extern "C" int tgs_tide_project_fwd(uint32_t n_touched, const uint32_t* n_touched_dev,
+static int tide_project_fwd(uint32_t n_touched, const uint32_t* n_touched_dev,
                                     const int32_t* touched,
                                     const int32_t* visit_base, const int32_t* visits,
                                     const uint32_t* masks, uint32_t C, const float* params,
@@ -1420,13 +1471,13 @@ extern "C" int tgs_tide_project_fwd(uint32_t n_touched, const uint32_t* n_touche
                                     int32_t sh_degree, uint32_t tile_size, uint32_t tile_width,
                                     uint32_t tile_height,
                                     float* splats, uint32_t* depth_keys, uint64_t* entry_rects,
-                                    int64_t* isect_totals, uint32_t* depth_range,
+                                    int64_t* isect_totals, uint32_t* depth_range, bool init,
                                     hipStream_t stream) {
   int rc = check_cams(C);
   if (rc) return rc;
-  if (isect_totals)
+  if (init && isect_totals)
     hipLaunchKernelGGL(tide_zero_i64_kernel, dim3(1), dim3(64), 0, stream, isect_totals, C);
-  if (depth_range)
+  if (init && depth_range)
     hipLaunchKernelGGL(tide_range_init_kernel, dim3(1), dim3(2 * TIDE_RANGE_SLOTS), 0, stream,
                        depth_range);
   if (n_touched == 0) TGS_RETURN_LAUNCH("tgs_tide_project_fwd");
@@ -1448,6 +1499,35 @@ extern "C" int tgs_tide_project_fwd(uint32_t n_touched, const uint32_t* n_touche
                      tile_height, (float4*)splats, depth_keys, entry_rects, isect_totals,
                      depth_range);
   TGS_RETURN_LAUNCH("tgs_tide_project_fwd");
+}
+
+extern "C" int tgs_tide_project_fwd(
+    uint32_t n_touched, const uint32_t* n_touched_dev, const int32_t* touched,
+    const int32_t* visit_base, const int32_t* visits, const uint32_t* masks, uint32_t C,
+    const float* params, uint32_t row_stride, const float* viewmats, const float* Ks,
+    const float* campos, int32_t W, int32_t H, float eps2d, float near_plane, float far_plane,
+    float radius_clip, int32_t sh_degree, uint32_t tile_size, uint32_t tile_width,
+    uint32_t tile_height, float* splats, uint32_t* depth_keys, uint64_t* entry_rects,
+    int64_t* isect_totals, uint32_t* depth_range, hipStream_t stream) {
+  return tide_project_fwd(n_touched, n_touched_dev, touched, visit_base, visits, masks, C, params,
+                          row_stride, viewmats, Ks, campos, W, H, eps2d, near_plane, far_plane,
+                          radius_clip, sh_degree, tile_size, tile_width, tile_height, splats,
+                          depth_keys, entry_rects, isect_totals, depth_range, true, stream);
+}
+
+// After tgs_tide_begin: the totals are cleared and the range is empty.
+extern "C" int tgs_tide_project_fwd_begun(
+    uint32_t n_touched, const uint32_t* n_touched_dev, const int32_t* touched,
+    const int32_t* visit_base, const int32_t* visits, const uint32_t* masks, uint32_t C,
+    const float* params, uint32_t row_stride, const float* viewmats, const float* Ks,
+    const float* campos, int32_t W, int32_t H, float eps2d, float near_plane, float far_plane,
+    float radius_clip, int32_t sh_degree, uint32_t tile_size, uint32_t tile_width,
+    uint32_t tile_height, float* splats, uint32_t* depth_keys, uint64_t* entry_rects,
+    int64_t* isect_totals, uint32_t* depth_range, hipStream_t stream) {
+  return tide_project_fwd(n_touched, n_touched_dev, touched, visit_base, visits, masks, C, params,
+                          row_stride, viewmats, Ks, campos, W, H, eps2d, near_plane, far_plane,
+                          radius_clip, sh_degree, tile_size, tile_width, tile_height, splats,
+                          depth_keys, entry_rects, isect_totals, depth_range, false, stream);
 }
 
 

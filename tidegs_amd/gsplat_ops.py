@@ -89,6 +89,7 @@ class _FullyFusedProjection(torch.autograd.Function):
         ctx.save_for_backward(means, covars, quats, scales, viewmats, Ks, radii, conics, comps)
         ctx.width, ctx.height, ctx.eps2d = int(width), int(height), float(eps2d)
         ctx.mark_non_differentiable(radii)
+        ctx.set_materialize_grads(False)
         return radii, means2d, depths, conics, comps
 
     @staticmethod
@@ -96,12 +97,16 @@ class _FullyFusedProjection(torch.autograd.Function):
         means, covars, quats, scales, viewmats, Ks, radii, conics, comps = ctx.saved_tensors
         C, Nn = viewmats.shape[0], means.shape[0]
 
-        def _c(t, like):
-            return torch.zeros_like(like) if t is None else t.contiguous()
+        if v_means2d is None and v_depths is None and v_conics is None and v_comps is None:
+            return (None,) * 13
 
-        v_means2d = _c(v_means2d, radii.unsqueeze(-1).expand(C, Nn, 2).float())
-        v_depths = _c(v_depths, radii.float())
-        v_conics = _c(v_conics, conics)
+        def _c(t, shape):
+            return torch.zeros(shape, dtype=torch.float32, device=means.device) if t is None \
+                else t.contiguous()
+
+        v_means2d = _c(v_means2d, (C, Nn, 2))
+        v_depths = None if v_depths is None else v_depths.contiguous()
+        v_conics = _c(v_conics, (C, Nn, 3))
         v_comps = v_comps.contiguous() if (v_comps is not None and comps is not None) else None
         v_means = torch.empty_like(means)
         v_covars = torch.empty_like(covars) if covars is not None else None
@@ -490,6 +495,7 @@ class _RasterizeToPixels(torch.autograd.Function):
                               flatten_ids, kernel_alphas, render_alphas, last_ids, records, pmask,
                               states, item_tile)
         ctx.width, ctx.height, ctx.tile_size, ctx.absgrad = width, height, tile_size, absgrad
+        ctx.set_materialize_grads(False)
         return render_colors, render_alphas
 
     @staticmethod
@@ -509,10 +515,10 @@ class _RasterizeToPixels(torch.autograd.Function):
             v_render_colors = (v_render_colors * pmask[..., None]).contiguous()
             if v_render_alphas is not None:
                 v_render_alphas = (v_render_alphas * pmask[..., None]).contiguous()
-        v_means2d = torch.zeros_like(means2d)
-        v_conics = torch.zeros_like(conics)
-        v_colors = torch.zeros_like(colors)
-        v_opacities = torch.zeros_like(opacities)
+        # the record path writes every value; the SoA kernels add into zeros
+        new = torch.zeros_like if records is None else torch.empty_like
+        v_means2d, v_conics, v_colors, v_opacities = (
+            new(t) for t in (means2d, conics, colors, opacities))
         v_abs = torch.zeros_like(means2d) if ctx.absgrad else None
         if records is not None:
             n = opacities.numel()

@@ -215,6 +215,7 @@ class GPUResidentAdam:
     # moment table row pitch: 64 floats = two whole 128-byte lines per row
     STATE_PITCH = 64
     _STATE_COLS = _STATE_COLUMNS
+    _bias_corrected = True  # the update reads the per-slot bias terms
     # kernel component order = state column order
     _LAUNCH_ORDER = tuple(sorted(COMPONENT_SPECS, key=lambda spec: _STATE_COLUMNS[spec[0]]))
     # learning-rate order of tgs_tide_project_bwd_update (CACHE column groups)
@@ -244,7 +245,8 @@ class GPUResidentAdam:
         self._counts_dev: Optional[torch.Tensor] = None
         self._counts_host: Optional[torch.Tensor] = None
         self._fused_lrs = None
-        self._error_flag = torch.zeros(1, dtype=torch.int32, device=self.device)
+        # [a launch met a row outside every block, the step's rows all have one]
+        self._error_flag, self._go = torch.zeros(2, dtype=torch.int32, device=self.device)
         self._counters = {"cold_restarts": 0, "optimizer_rows_touched_total": 0,
                           "cold_restarted_rows_touched_total": 0}
 
@@ -299,14 +301,24 @@ class GPUResidentAdam:
         (``1 - b1^t``, ``sqrt(1 - b2^t)`` in float64, stored as float32) and
         queue the whole table's upload from the staging table whose previous
         copy has finished."""
-        t = self.slots.steps[slots].astype(np.float64)
-        self._bias_host[0, slots] = 1.0 - beta1 ** t
-        self._bias_host[1, slots] = np.sqrt(1.0 - beta2 ** t)
+        self._set_bias_terms(self._bias_host, slots, self.slots.steps[slots], beta1, beta2)
+        self._upload_bias_table(self._bias_host)
+
+    @staticmethod
+    def _set_bias_terms(table: np.ndarray, slots: np.ndarray, steps: np.ndarray, beta1: float,
+                        beta2: float) -> None:
+        t = steps.astype(np.float64)
+        table[0, slots] = 1.0 - beta1 ** t
+        table[1, slots] = np.sqrt(1.0 - beta2 ** t)
+
+    def _upload_bias_table(self, table: np.ndarray) -> None:
+        """Queue the upload of a whole bias table from the staging table whose
+        previous copy has finished."""
         turn = self._staging[self._staging_turn]
         self._staging_turn ^= 1
         if turn[1] is not None:
             turn[1].synchronize()
-        turn[0].numpy()[:] = self._bias_host
+        turn[0].numpy()[:] = table
         self._bias_terms.copy_(turn[0], non_blocking=True)
         if self.device.type == "cuda":
             turn[1] = torch.cuda.Event()
@@ -343,16 +355,19 @@ class GPUResidentAdam:
         beta1, beta2 = group["betas"]
         return float(beta1), float(beta2), float(group["eps"])
 
-    def _count_touches(self, layout: _Layout, rows: torch.Tensor) -> torch.Tensor:
-        """Queue the per-layout-block count of ``rows`` (ascending) on the
-        device stream and its copy into pinned host memory; the host tensor is
-        valid after the stream's next synchronisation."""
-        n = len(layout)
+    def _count_buffers(self, n: int) -> None:
         if self._counts_dev is None or self._counts_dev.numel() < n:
             size = max(n, 64)
             self._counts_dev = torch.empty(size, dtype=torch.int64, device=self.device)
             self._counts_host = torch.empty(size, dtype=torch.int64,
                                             pin_memory=self.device.type == "cuda")
+
+    def _count_touches(self, layout: _Layout, rows: torch.Tensor) -> torch.Tensor:
+        """Queue the per-layout-block count of ``rows`` (ascending) on the
+        device stream and its copy into pinned host memory; the host tensor is
+        valid after the stream's next synchronisation."""
+        n = len(layout)
+        self._count_buffers(n)
         N.call("tgs_block_touch_counts", rows.numel(), N.ptr(rows),
                1 if rows.dtype == torch.int64 else 0, N.ptr(layout.d_starts),
                N.ptr(layout.d_stops), n, N.ptr(self._counts_dev), N.stream_handle(self.device))
@@ -360,11 +375,26 @@ class GPUResidentAdam:
         host.copy_(self._counts_dev[:n], non_blocking=True)
         return host
 
+    def _check_touches(self, layout: _Layout, rows: torch.Tensor) -> torch.cuda.Event:
+        """Queue the per-block counts of ``rows`` and their check on the device
+        (``self._go``), and the counts' copy into pinned host memory, valid
+        after the returned event."""
+        n = len(layout)
+        self._count_buffers(n)
+        N.call("tgs_block_touch_check", rows.numel(), N.ptr(rows),
+               1 if rows.dtype == torch.int64 else 0, N.ptr(layout.d_starts),
+               N.ptr(layout.d_stops), n, N.ptr(self._counts_dev), N.ptr(self._go),
+               N.stream_handle(self.device))
+        self._counts_host[:n].copy_(self._counts_dev[:n], non_blocking=True)
+        ready = torch.cuda.Event()
+        ready.record(torch.cuda.current_stream(self.device))
+        return ready
+
     def _apply_counts(self, layout: _Layout, counts: np.ndarray, n_rows: int, beta1: float,
-                      beta2: float) -> Dict[str, Any]:
+                      beta2: float, upload: bool = True) -> Dict[str, Any]:
         """Advance the slots of the touched blocks and refresh their bias
-        terms (``gpu_resident_optimizer.py:302-337`` behaviour); returns the
-        step's stats dictionary."""
+        terms (``gpu_resident_optimizer.py:302-337`` behaviour; uploaded unless
+        the caller has); returns the step's stats dictionary."""
         if counts.shape[0] != len(layout) or int(counts.sum()) != int(n_rows):
             raise RuntimeError(
                 "[GPUResidentAdam] a touched row lies outside every resident block of the layout")
@@ -372,8 +402,10 @@ class GPUResidentAdam:
         slots = layout.slots[hit]
         cold_slots, cold_rows = self.slots.advance(
             slots, layout.stops[hit] - layout.starts[hit], counts[hit])
-        if slots.size:
+        if slots.size and upload:
             self._upload_bias_terms(slots, beta1, beta2)
+        elif slots.size:
+            self._set_bias_terms(self._bias_host, slots, self.slots.steps[slots], beta1, beta2)
         self._counters["cold_restarts"] += cold_slots
         self._counters["cold_restarted_rows_touched_total"] += cold_rows
         self._counters["optimizer_rows_touched_total"] += int(n_rows)
@@ -424,7 +456,7 @@ class GPUResidentAdam:
         ptrs, widths, strides, lrs = self._component_tables(gaussians, grads)
         head = (N.ptr(self._bias_terms[0]), N.ptr(self._bias_terms[1]))
         tail = (beta1, beta2, eps, float(self.batch_size))
-        return "tgs_resident_adam_step", head, (len(self._LAUNCH_ORDER), *ptrs, widths, strides,
+        return "tgs_resident_adam_step_checked", head, (len(self._LAUNCH_ORDER), *ptrs, widths, strides,
                                                  lrs), tail
 
     def step(self, iteration: int, gaussians, sparse_grad_local_ids: torch.Tensor,
@@ -449,19 +481,28 @@ class GPUResidentAdam:
         beta1, beta2, eps = self._hyper(gaussians)
         kernel, head, comps, tail = self._kernel_args(gaussians, sparse_grad_components, beta1,
                                                       beta2, eps, iteration)
-        counts = self._count_touches(layout, rows)
-        torch.cuda.current_stream(self.device).synchronize()
-        stats = self._apply_counts(layout, counts.numpy(), rows.numel(), beta1, beta2)
+        # The GPU does not wait for the host: the update is queued behind the
+        # counts and their check, with bias terms of one more step for every
+        # block of the layout (the kernel reads those of touched blocks only),
+        # and the host advances the touched slots while it runs.
+        ready = self._check_touches(layout, rows)
+        if self._bias_corrected:
+            table = self._bias_host.copy()
+            self._set_bias_terms(table, layout.slots, self.slots.steps[layout.slots] + 1, beta1,
+                                 beta2)
+            self._upload_bias_table(table)
         hooks = self.kernel_hooks
         if hooks:
             hooks[0]()
         N.call(kernel, rows.numel(), N.ptr(rows), 1 if rows.dtype == torch.int64 else 0,
                N.ptr(layout.d_starts), N.ptr(layout.d_stops), N.ptr(layout.d_slots), len(layout),
-               self.block_size, *head, *comps, *tail, N.ptr(self._error_flag),
+               self.block_size, *head, *comps, *tail, N.ptr(self._error_flag), N.ptr(self._go),
                N.stream_handle(self.device))
         if hooks:
             hooks[1]()
-        return stats
+        ready.synchronize()
+        return self._apply_counts(layout, self._counts_host[:len(layout)].numpy(), rows.numel(),
+                                  beta1, beta2, upload=False)
 
     # ---- update fused into the gradient launch ------------------------------
     # A caller that computes the touched rows' gradients on the GPU applies the
@@ -561,6 +602,8 @@ class GPUResidentSophia(GPUResidentAdam):
     ``g`` is the gradient divided by the batch size, as in GPUResidentAdam.
     """
 
+    _bias_corrected = False
+
     def __init__(self, batch_size: int = 1, block_size: int = 4096, capacity_blocks: int = 0,
                  device: str = "cuda", rho: float = 0.04, hessian_interval: int = 1):
         super().__init__(batch_size, block_size, capacity_blocks, device)
@@ -577,5 +620,5 @@ class GPUResidentSophia(GPUResidentAdam):
         ptrs, widths, strides, lrs = self._component_tables(gaussians, grads)
         tail = (beta1, beta2, eps, self.rho, float(self.batch_size),
                 self._update_hessian(iteration))
-        return "tgs_resident_sophia_step", (), (len(self._LAUNCH_ORDER), *ptrs, widths, strides,
+        return "tgs_resident_sophia_step_checked", (), (len(self._LAUNCH_ORDER), *ptrs, widths, strides,
                                                  lrs), tail

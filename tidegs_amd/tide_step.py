@@ -296,7 +296,17 @@ class TideStep:
         Ks = Ks.to(self.device, torch.float32).contiguous()
         campos = self._buf("campos", 3 * C, torch.float32).view(C, 3)
         self._begin("camera_centers")
-        N.call("tgs_tide_camera_centers", C, N.ptr(viewmats), N.ptr(campos), s)
+        # totals [C+3+128]: V_c..., T, sum V, visits (compaction), then 64
+        # {min, max} pairs of the depth keys' range (visibility)
+        totals = self._buf("totals", C + 3 + 2 * RANGE_SLOTS, torch.int32)
+        # the projection sums the per-camera intersection counts (the rectangles'
+        # areas, [C]) and the range of the depth keys it writes (64 pairs), to
+        # check the depth sort's range (taken from the visibility pass) against;
+        # both go to the host in one copy while the depth sort runs
+        proj = self._buf("proj_totals", C + RANGE_SLOTS, torch.int64)
+        visible_range, projected_range = N.ptr(totals) + 4 * (C + 3), N.ptr(proj) + 8 * C
+        N.call("tgs_tide_begin", C, N.ptr(viewmats), N.ptr(campos), visible_range,
+               projected_range, N.ptr(proj), s)
         self._end()
         gt = gt.to(self.device, torch.float32).contiguous()
         lib = N.load()
@@ -306,13 +316,10 @@ class TideStep:
         masks = self._buf("masks", n, torch.int32)
         counts = self._buf("counts", (C + 2) * nb, torch.int32)
         self._begin("visibility")
-        # totals [C+3+128]: V_c..., T, sum V, visits (compaction), then 64
-        # {min, max} pairs of the depth keys' range (visibility)
-        totals = self._buf("totals", C + 3 + 2 * RANGE_SLOTS, torch.int32)
-        N.call("tgs_tide_visibility", n, N.ptr(P), self.row_stride, C, N.ptr(viewmats), N.ptr(Ks),
+        N.call("tgs_tide_visibility_begun", n, N.ptr(P), self.row_stride, C, N.ptr(viewmats), N.ptr(Ks),
                N.ptr(campos),
                W, H, self.eps2d, self.near, self.far, self.radius_clip, N.ptr(masks),
-               N.ptr(counts), N.ptr(totals) + 4 * (C + 3), s)
+               N.ptr(counts), visible_range, s)
         offs = self._buf("offs", (C + 2) * nb, torch.int32)
         ws = self._buf("scan_ws", lib.tgs_scan_workspace_size((C + 2) * nb), torch.uint8)
         N.call("tgs_exclusive_scan_u32", N.ptr(counts), N.ptr(offs), (C + 2) * nb, N.ptr(ws),
@@ -340,23 +347,15 @@ class TideStep:
         splats = self._buf("splats", cap_v * 12, torch.float32)
         dkeys = self._buf("depth_keys", cap_v, torch.int32)
         rects = self._buf("entry_rects", cap_v, torch.int64)
-        # the projection also sums the per-camera intersection counts (the
-        # rectangles' areas); they go to the host while the depth sort runs
-        isect_tot = self._buf("isect_totals", C, torch.int64)
-        # and the range of the depth keys it writes, to check the depth sort's
-        # range (taken from the visibility pass) against
-        proj_range = self._buf("proj_range", 2 * RANGE_SLOTS, torch.int32)
         self._begin("project_fwd")
-        N.call("tgs_tide_project_fwd", n, N.ptr(totals) + 4 * C, N.ptr(touched),
+        N.call("tgs_tide_project_fwd_begun", n, N.ptr(totals) + 4 * C, N.ptr(touched),
                N.ptr(visit_base), N.ptr(visits), N.ptr(masks), C, N.ptr(P), self.row_stride,
                N.ptr(viewmats), N.ptr(Ks), N.ptr(campos), W, H, self.eps2d, self.near, self.far,
                0.0, self.sh_degree, self.TILE, tw, th, N.ptr(splats), N.ptr(dkeys), N.ptr(rects),
-               N.ptr(isect_tot), N.ptr(proj_range), s)
+               N.ptr(proj), projected_range, s)
         self._end()
-        isect_host = self._pinned("isect_totals", C, torch.int64)
-        isect_host.copy_(isect_tot, non_blocking=True)
-        range_host = self._pinned("proj_range", 2 * RANGE_SLOTS, torch.int32)
-        range_host.copy_(proj_range, non_blocking=True)
+        proj_host = self._pinned("proj_totals", C + RANGE_SLOTS, torch.int64)
+        proj_host.copy_(proj, non_blocking=True)
         isects_ready = self._record()
 
         totals_ready.synchronize()  # host read 1: the projection keeps the GPU busy
@@ -405,7 +404,8 @@ class TideStep:
         self._end()
         self.last_depth_key_bits = key_bits
         isects_ready.synchronize()  # host read 2: the depth sort keeps the GPU busy
-        if V and not depth_range_holds(range_host.tolist(), key_base, key_bits):
+        if V and not depth_range_holds(proj_host[C:].view(torch.int32).tolist(), key_base,
+                                       key_bits):
             # a projected key outside the visibility pass's range (plus slack)
             # tied with its neighbours in the ranked sort; a stable sort on all
             # 32 bits of the ranked result restores the (depth, entry) order,
@@ -423,7 +423,7 @@ class TideStep:
             N.call("tgs_exclusive_scan_u32", N.ptr(fe_hist), N.ptr(fe_scan), hist_words,
                    N.ptr(ws), ws.numel(), s)
             self._end()
-        per_cam = isect_host.tolist()
+        per_cam = proj_host[:C].tolist()
         isect_segs = [0]
         for k in per_cam:
             isect_segs.append(isect_segs[-1] + int(k))
