@@ -243,6 +243,42 @@ def test_isect_tiles_paths_bit_exact(gpu, case):
     np.testing.assert_array_equal(to_np(flat), o_flat)
 
 
+@pytest.mark.parametrize("C,n,tw,th,depth", [
+    (1, 1, 1, 1, (2.0, 2.0)),             # one key without a bit to sort on
+    (1, 255, 1, 1, (2.0, 2.0)), (1, 256, 7, 3, (2.0, 2.0)),  # no depth bits
+    (2, 257, 7, 3, (0.0, 1.0)),           # ids of 2 cameras in 1 bit, depths from zero
+    (3, 8191, 16, 16, (1.0, 2.0 - 2.0 ** -23)),  # 256 tiles: 9 bits, depths of one binade
+    (1, 256 * 1024 + 1, 31, 17, (0.2, 500.0)),   # one block past a chunk of the sums' scan
+])
+@pytest.mark.parametrize("packed", [False, True])
+def test_isect_tiles_blocks_and_key_bits(gpu, C, n, tw, th, depth, packed):
+    """The plan's blocks of 256 Gaussians at their edges and keys sorted on the
+    bits that depths and ids can differ in: bit-exact with the oracle, offsets too."""
+    announce(f"isect blocks C={C} n={n} {tw}x{th} packed={packed}")
+    rng = np.random.default_rng(n)
+    m2d = rng.uniform(-8, [tw * 16 + 8, th * 16 + 8], size=(C, n, 2)).astype(np.float32)
+    radii = rng.integers(-2, 14, size=(C, n)).astype(np.int32)
+    m2d[0, 0], radii[0, 0] = 1.0, 3
+    depths = rng.uniform(*depth, size=(C, n)).astype(np.float32)
+    kw, okw = {}, {}
+    if packed:
+        cam = rng.integers(0, C, size=C * n)
+        m2d, radii, depths = m2d.reshape(-1, 2), radii.reshape(-1), depths.reshape(-1)
+        d_cam = torch.from_numpy(cam).to(gpu)
+        kw = dict(packed=True, n_cameras=C, camera_ids=d_cam, gaussian_ids=d_cam)
+        okw = dict(camera_ids=cam)
+    args = [torch.from_numpy(a).to(gpu) for a in (m2d, radii, depths)]
+    tiles, ids, flat = ops.isect_tiles(*args, 16, tw, th, **kw)
+    if packed and C > 1:  # the oracle takes the camera count from its ids
+        assert cam.max() == C - 1
+    o_tiles, o_ids, o_flat = R.isect_tiles(m2d, radii, depths, 16, tw, th, **okw)
+    np.testing.assert_array_equal(to_np(tiles), o_tiles)
+    np.testing.assert_array_equal(to_np(ids), o_ids)
+    np.testing.assert_array_equal(to_np(flat), o_flat)
+    offs = ops.isect_offset_encode(ids, C, tw, th)
+    np.testing.assert_array_equal(to_np(offs), R.isect_offset_encode(o_ids, C, tw, th))
+
+
 @pytest.mark.parametrize("n,shift", [(1, 0), (7, 0), (9, 1), (4096 + 5, 3), (200_003, 1)])
 def test_isect_offset_encode_ragged(gpu, n, shift):
     """Offsets from sorted keys of every length class of the eight-keys-per-

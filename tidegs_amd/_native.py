@@ -61,6 +61,15 @@ SIGNATURES = {
         ctypes.c_int,
         [U64, U32, P, P, P, P, P, U32, U32, U32, U32, P, P, P],
     ),
+    "tgs_isect_tiles_plan_size": (U64, [U64]),
+    "tgs_isect_tiles_plan": (
+        ctypes.c_int, [U64, P, P, P, U32, U32, U32, P, P, SZ, P, P]),
+    "tgs_isect_tiles_emit_plan": (
+        ctypes.c_int, [U64, U32, P, P, P, P, P, P, U32, U32, U32, U32, P, P, P]),
+    "tgs_radix_sort_pairs_range": (
+        ctypes.c_int,
+        [P, P, P, P, U64, U32, ctypes.c_int, ctypes.c_int, P, SZ, ctypes.POINTER(ctypes.c_int), P],
+    ),
     "tgs_radix_sort_workspace_size": (SZ, [U64]),
     "tgs_radix_sort_pairs": (
         ctypes.c_int,

@@ -284,6 +284,10 @@ struct RadixSegs {
   // base as 0): an order-preserving map of a key range onto its low bits, with
   // every key past the range tied at key_cap.  (0, ~0) ranks the keys as they are.
   uint32_t key_base = 0, key_cap = 0xffffffffu;
+  // 64-bit keys are ranked as (high word << low_bits) | (low word - key_base): low
+  // words known to lie in [key_base, key_base + 2^low_bits) take no more bits
+  // than their range.  (0, 32) ranks the keys as they are.
+  uint32_t low_bits = 32;
 };
 
 struct TileRange {
@@ -319,7 +323,8 @@ __device__ __forceinline__ uint32_t digit_of(K key, const RadixSegs& sg, int shi
     const uint32_t r = min(max((uint32_t)key, sg.key_base) - sg.key_base, sg.key_cap);
     return (r >> shift) & mask;
   } else {
-    return (uint32_t)(key >> shift) & mask;
+    const uint64_t r = ((uint64_t)key >> 32 << sg.low_bits) | ((uint32_t)key - sg.key_base);
+    return (uint32_t)(r >> shift) & mask;
   }
 }
 
@@ -692,10 +697,10 @@ static int radix_passes(K* keys, V* vals, K* keys_alt, V* vals_alt, RadixSegs& s
 // Data ping-pongs between (keys, vals) and (keys_alt, vals_alt); *selector is
 // set to 0 if the result is in keys/vals and 1 if in keys_alt/vals_alt
 // (the cub::DoubleBuffer convention used at isect_tiles.cu:196-217).
-extern "C" int tgs_radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
-                                    uint32_t* vals_alt, uint64_t n, int begin_bit, int end_bit,
-                                    void* workspace, size_t workspace_bytes, int* selector,
-                                    hipStream_t stream) {
+static int radix_sort_u64(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
+                          uint64_t n, uint32_t key_base, uint32_t low_bits, int begin_bit,
+                          int end_bit, void* workspace, size_t workspace_bytes, int* selector,
+                          hipStream_t stream) {
   TGS_CHECK_ARG(selector != nullptr, "radix_sort: null selector");
   *selector = 0;
   if (n <= 1 || end_bit <= begin_bit) return TGS_OK;
@@ -709,10 +714,35 @@ extern "C" int tgs_radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* ke
   }
   RadixSegs sg{};
   sg.n = 1;
+  sg.key_base = key_base;
+  sg.low_bits = low_bits;
   sg.key_off[0] = 0;
   sg.key_off[1] = (uint32_t)n;
   return radix_passes<uint64_t, uint32_t>(keys, vals, keys_alt, vals_alt, sg, begin_bit, end_bit,
                                           workspace, selector, stream);
+}
+
+extern "C" int tgs_radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
+                                    uint32_t* vals_alt, uint64_t n, int begin_bit, int end_bit,
+                                    void* workspace, size_t workspace_bytes, int* selector,
+                                    hipStream_t stream) {
+  return radix_sort_u64(keys, vals, keys_alt, vals_alt, n, 0u, 32u, begin_bit, end_bit, workspace,
+                        workspace_bytes, selector, stream);
+}
+
+// The same sort on the keys' order when every low word is known to lie in
+// [low_base, low_base + 2^low_bits) and every high word below 2^high_bits: low_bits
+// + high_bits bits instead of 32 + high_bits (the tile intersections' depth bits:
+// 25 to 27 of 32 for depths within a factor of 4 to 30, so five passes, not six).
+extern "C" int tgs_radix_sort_pairs_range(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
+                                          uint32_t* vals_alt, uint64_t n, uint32_t low_base,
+                                          int low_bits, int high_bits, void* workspace,
+                                          size_t workspace_bytes, int* selector,
+                                          hipStream_t stream) {
+  TGS_CHECK_ARG(low_bits >= 0 && low_bits <= 32 && high_bits >= 0 && high_bits <= 32,
+                "radix_sort_range: low_bits and high_bits in [0, 32]");
+  return radix_sort_u64(keys, vals, keys_alt, vals_alt, n, low_base, (uint32_t)low_bits, 0,
+                        low_bits + high_bits, workspace, workspace_bytes, selector, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -370,36 +370,50 @@ def isect_tiles(
     if total == 0:
         return (tiles_per_gauss, torch.empty(0, dtype=torch.int64, device=dev),
                 torch.empty(0, dtype=torch.int32, device=dev))
-    N.call("tgs_isect_tiles_count", total, N.ptr(means2d), N.ptr(radii), tile_size, tile_width,
-           tile_height, N.ptr(tiles_per_gauss), s)
-    cum = torch.empty(total, dtype=torch.int64, device=dev)
-    ws = torch.empty(N.load().tgs_scan_workspace_size(total), dtype=torch.uint8, device=dev)
-    N.call("tgs_inclusive_scan_i32_i64", N.ptr(tiles_per_gauss), N.ptr(cum), total, N.ptr(ws),
-           ws.numel(), s)
-    n_isects = int(cum[-1].item())
+    lib = N.load()
+    plan = torch.empty(lib.tgs_isect_tiles_plan_size(total), dtype=torch.uint8, device=dev)
+    summary = torch.empty(2, dtype=torch.int64, device=dev)
+    N.call("tgs_isect_tiles_plan", total, N.ptr(means2d), N.ptr(radii), N.ptr(depths), tile_size,
+           tile_width, tile_height, N.ptr(tiles_per_gauss), N.ptr(plan), plan.numel(),
+           N.ptr(summary), s)
+    n_isects, key_range = summary.tolist()
     isect_ids = torch.empty(n_isects, dtype=torch.int64, device=dev)
     flatten_ids = torch.empty(n_isects, dtype=torch.int32, device=dev)
     if n_isects:
-        N.call("tgs_isect_tiles_emit", total, Nn, N.ptr(cam_ids), N.ptr(means2d), N.ptr(radii),
-               N.ptr(depths), N.ptr(cum), tile_size, tile_width, tile_height, tile_n_bits,
-               N.ptr(isect_ids), N.ptr(flatten_ids), s)
+        N.call("tgs_isect_tiles_emit_plan", total, Nn, N.ptr(cam_ids), N.ptr(means2d),
+               N.ptr(radii), N.ptr(depths), N.ptr(tiles_per_gauss), N.ptr(plan), tile_size,
+               tile_width, tile_height, tile_n_bits, N.ptr(isect_ids), N.ptr(flatten_ids), s)
     if n_isects and sort:
-        isect_ids, flatten_ids = radix_sort_pairs(isect_ids, flatten_ids,
-                                                  end_bit=32 + tile_n_bits + cam_n_bits)
+        kmin, kmax = key_range & 0xFFFFFFFF, (key_range >> 32) & 0xFFFFFFFF
+        if kmax >> 31:  # a negative depth's sign fills the high word, as in the reference
+            isect_ids, flatten_ids = radix_sort_pairs(isect_ids, flatten_ids,
+                                                      end_bit=32 + tile_n_bits + cam_n_bits)
+        else:
+            # the depth bits take no more key bits than their range, and the ids
+            # no more than the largest one (packed camera ids: any of cam_n_bits)
+            high = tile_n_bits + cam_n_bits if packed else \
+                _bit_width(((C - 1) << tile_n_bits) | (n_tiles - 1))
+            isect_ids, flatten_ids = _radix_sort(
+                isect_ids, flatten_ids, "tgs_radix_sort_pairs_range", kmin,
+                _bit_width(kmax - kmin), high)
     return tiles_per_gauss, isect_ids, flatten_ids
 
 
 def radix_sort_pairs(keys: Tensor, values: Tensor, begin_bit: int = 0,
                      end_bit: int = 64) -> Tuple[Tensor, Tensor]:
     """Stable ascending sort of int64 keys (on bits [begin_bit, end_bit)) with int32 values."""
+    return _radix_sort(keys, values, "tgs_radix_sort_pairs", begin_bit, end_bit)
+
+
+def _radix_sort(keys: Tensor, values: Tensor, entry: str, *bits: int) -> Tuple[Tensor, Tensor]:
     n = keys.numel()
     dev = keys.device
     k_alt = torch.empty_like(keys)
     v_alt = torch.empty_like(values)
     ws = torch.empty(max(1, N.load().tgs_radix_sort_workspace_size(n)), dtype=torch.uint8, device=dev)
     sel = ctypes.c_int(0)
-    N.call("tgs_radix_sort_pairs", N.ptr(keys), N.ptr(values), N.ptr(k_alt), N.ptr(v_alt), n,
-           begin_bit, end_bit, N.ptr(ws), ws.numel(), ctypes.byref(sel), _stream())
+    N.call(entry, N.ptr(keys), N.ptr(values), N.ptr(k_alt), N.ptr(v_alt), n, *bits, N.ptr(ws),
+           ws.numel(), ctypes.byref(sel), _stream())
     return (k_alt, v_alt) if sel.value else (keys, values)
 
 
