@@ -203,22 +203,33 @@ int tgs_segmented_sort_pairs_u32_range(uint32_t* keys, void* vals, uint32_t* key
                                        uint32_t key_base, int key_bits, void* workspace,
                                        size_t workspace_bytes, int* selector,
                                        tgs_stream_t stream);
-/* Counts, offsets and depth range without a scan of every Gaussian's count: the
- * plan (tgs_isect_tiles_plan_size bytes, 16-byte aligned) holds one record per 256
- * Gaussians; summary = {intersections, kmin | kmax << 32}, kmin and kmax the least
- * and greatest depth bits (unsigned) of Gaussians with any (0xffffffff, 0: none).
- * The emission then writes what tgs_isect_tiles_emit does. */
-uint64_t tgs_isect_tiles_plan_size(uint64_t total);
-int tgs_isect_tiles_plan(uint64_t total, const float* means2d, const int32_t* radii,
+/* Counts, offsets and depth range without a scan of every Gaussian's count, for C
+ * cameras of N Gaussians (packed: one of nnz).  The plan (tgs_isect_tiles_plan_size
+ * bytes) holds one record per 256 Gaussians.  summary [2 + 2 C] = {intersections,
+ * kmin | kmax << 32} with the least and greatest depth bits (unsigned; 0xffffffff, 0
+ * where none) of the Gaussians that meet a tile, then per camera {such Gaussians,
+ * intersections} up to its end.  tgs_isect_tiles_emit_plan writes what
+ * tgs_isect_tiles_emit does; tgs_isect_tiles_sorted writes the sorted ids and
+ * flatten ids at once (summary: a host copy), where its workspace size is not 0:
+ * up to 32 cameras, tiles up to 255 x 255, no negative depth. */
+uint64_t tgs_isect_tiles_plan_size(uint32_t C, uint64_t N);
+int tgs_isect_tiles_plan(uint32_t C, uint64_t N, const float* means2d, const int32_t* radii,
                          const float* depths, uint32_t tile_size, uint32_t tile_width,
                          uint32_t tile_height, int32_t* tiles_per_gauss, void* plan,
                          size_t plan_bytes, uint64_t* summary, tgs_stream_t stream);
-int tgs_isect_tiles_emit_plan(uint64_t total, uint32_t N, const int64_t* camera_ids,
+int tgs_isect_tiles_emit_plan(uint32_t C, uint64_t N, const int64_t* camera_ids,
                               const float* means2d, const int32_t* radii, const float* depths,
                               const int32_t* tiles_per_gauss, const void* plan,
                               uint32_t tile_size, uint32_t tile_width, uint32_t tile_height,
                               uint32_t tile_n_bits, int64_t* isect_ids, int32_t* flatten_ids,
                               tgs_stream_t stream);
+uint64_t tgs_isect_tiles_sorted_workspace_size(uint32_t C, const uint64_t* summary,
+                                               uint32_t tile_width, uint32_t tile_height);
+int tgs_isect_tiles_sorted(uint32_t C, uint64_t N, const float* means2d, const int32_t* radii,
+                           const float* depths, const void* plan, const uint64_t* summary,
+                           uint32_t tile_size, uint32_t tile_width, uint32_t tile_height,
+                           int64_t* isect_ids, int32_t* flatten_ids, void* workspace,
+                           size_t workspace_bytes, tgs_stream_t stream);
 /* tgs_radix_sort_pairs on all bits of keys whose low words lie in [low_base, low_base
  * + 2^low_bits) and whose high words are below 2^high_bits. */
 int tgs_radix_sort_pairs_range(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,

@@ -248,12 +248,16 @@ def test_isect_tiles_paths_bit_exact(gpu, case):
     (1, 255, 1, 1, (2.0, 2.0)), (1, 256, 7, 3, (2.0, 2.0)),  # no depth bits
     (2, 257, 7, 3, (0.0, 1.0)),           # ids of 2 cameras in 1 bit, depths from zero
     (3, 8191, 16, 16, (1.0, 2.0 - 2.0 ** -23)),  # 256 tiles: 9 bits, depths of one binade
-    (1, 256 * 1024 + 1, 31, 17, (0.2, 500.0)),   # one block past a chunk of the sums' scan
+    (1, 4 * 256 * 1024 + 1, 31, 17, (0.2, 500.0)),  # one block past a chunk of the sums' scan
+    (2, 70_001, 255, 2, (0.2, 500.0)),    # the widest grid of the two sorts
+    (2, 70_001, 256, 2, (0.2, 500.0)),    # and one past it: a single sort
+    (32, 1001, 9, 9, (0.2, 500.0)), (33, 1001, 9, 9, (0.2, 500.0)),  # cameras, likewise
 ])
 @pytest.mark.parametrize("packed", [False, True])
 def test_isect_tiles_blocks_and_key_bits(gpu, C, n, tw, th, depth, packed):
-    """The plan's blocks of 256 Gaussians at their edges and keys sorted on the
-    bits that depths and ids can differ in: bit-exact with the oracle, offsets too."""
+    """The plan's blocks of 256 Gaussians at their edges, the two sorts and (packed
+    inputs, wide grids, many cameras) the single sort on the bits that depths and
+    ids can differ in: bit-exact with the oracle, offsets too."""
     announce(f"isect blocks C={C} n={n} {tw}x{th} packed={packed}")
     rng = np.random.default_rng(n)
     m2d = rng.uniform(-8, [tw * 16 + 8, th * 16 + 8], size=(C, n, 2)).astype(np.float32)

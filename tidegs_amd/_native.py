@@ -61,11 +61,14 @@ SIGNATURES = {
         ctypes.c_int,
         [U64, U32, P, P, P, P, P, U32, U32, U32, U32, P, P, P],
     ),
-    "tgs_isect_tiles_plan_size": (U64, [U64]),
+    "tgs_isect_tiles_plan_size": (U64, [U32, U64]),
     "tgs_isect_tiles_plan": (
-        ctypes.c_int, [U64, P, P, P, U32, U32, U32, P, P, SZ, P, P]),
+        ctypes.c_int, [U32, U64, P, P, P, U32, U32, U32, P, P, SZ, P, P]),
     "tgs_isect_tiles_emit_plan": (
-        ctypes.c_int, [U64, U32, P, P, P, P, P, P, U32, U32, U32, U32, P, P, P]),
+        ctypes.c_int, [U32, U64, P, P, P, P, P, P, U32, U32, U32, U32, P, P, P]),
+    "tgs_isect_tiles_sorted_workspace_size": (U64, [U32, P, U32, U32]),
+    "tgs_isect_tiles_sorted": (
+        ctypes.c_int, [U32, U64, P, P, P, P, P, U32, U32, U32, P, P, P, SZ, P]),
     "tgs_radix_sort_pairs_range": (
         ctypes.c_int,
         [P, P, P, P, U64, U32, ctypes.c_int, ctypes.c_int, P, SZ, ctypes.POINTER(ctypes.c_int), P],

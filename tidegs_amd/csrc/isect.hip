@@ -11,6 +11,42 @@
 //              empty tiles take the next run's start; trailing tiles take n.
 #include "tgs_common.cuh"
 
+#include <algorithm>
+
+// scan_sort.hip
+extern "C" size_t tgs_scan_workspace_size(uint64_t n);
+extern "C" int tgs_exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint64_t n,
+                                      void* workspace, size_t workspace_bytes,
+                                      hipStream_t stream);
+extern "C" size_t tgs_segmented_sort_workspace_size(uint64_t n, uint32_t n_segments);
+extern "C" int tgs_segmented_sort_pairs_u32(uint32_t* keys, void* vals, uint32_t* keys_alt,
+                                            void* vals_alt, uint32_t value_bytes, uint64_t n,
+                                            uint32_t n_segments, const uint32_t* seg_offsets,
+                                            int begin_bit, int end_bit, void* workspace,
+                                            size_t workspace_bytes, int* selector,
+                                            hipStream_t stream);
+extern "C" int tgs_segmented_sort_pairs_u32_range(uint32_t* keys, void* vals, uint32_t* keys_alt,
+                                                  void* vals_alt, uint32_t value_bytes, uint64_t n,
+                                                  uint32_t n_segments,
+                                                  const uint32_t* seg_offsets, uint32_t key_base,
+                                                  int key_bits, void* workspace,
+                                                  size_t workspace_bytes, int* selector,
+                                                  hipStream_t stream);
+// tide_step.hip
+extern "C" uint32_t tgs_tide_isect_fused_digit_bits(uint32_t tile_n_bits);
+extern "C" uint64_t tgs_tide_isect_fused_hist_words(uint32_t C, const uint32_t* cam_offsets,
+                                                    uint32_t tile_n_bits);
+extern "C" int tgs_tide_isect_fused_count(uint32_t C, const uint32_t* cam_offsets,
+                                          const uint64_t* entry_rects, uint32_t tile_width,
+                                          uint32_t tile_n_bits, uint32_t* hist,
+                                          uint64_t hist_words, hipStream_t stream);
+extern "C" int tgs_tide_isect_fused_scatter(uint32_t C, const uint32_t* cam_offsets,
+                                            const uint64_t* entry_rects, uint32_t tile_width,
+                                            uint32_t tile_n_bits, const uint32_t* hist_scan,
+                                            uint64_t hist_words, uint32_t n_isects,
+                                            uint32_t* keys, int32_t* flatten_ids,
+                                            hipStream_t stream);
+
 struct TileRect {
   uint32_t x0, y0, x1, y1;
 };
@@ -123,19 +159,32 @@ __global__ void __launch_bounds__(256) isect_offset_search_kernel(
 #define IB_ENTRIES 256
 
 struct IsectBlock {
-  int64_t sum;    // intersections; after the scan, those of the blocks before
-  uint32_t kmin;  // depth bits of the Gaussians with any: the least ...
-  uint32_t kmax;  // ... and greatest, as unsigned (0xffffffff, 0 where none)
+  int64_t sum;       // intersections; after the scan, those of the blocks before
+  uint32_t entries;  // Gaussians with any; after the scan, those of the blocks before
+  uint32_t kmin;     // their depth bits: the least ...
+  uint32_t kmax;     // ... and greatest, as unsigned (0xffffffff, 0 where none)
+  uint32_t pad;
 };
 
+// The Gaussian of this thread: each camera takes blocks_per_cam blocks, so that no block spans
+// two cameras.  False past the camera's last.
+__device__ __forceinline__ bool isect_block_entry(uint64_t N, uint32_t blocks_per_cam,
+                                                  uint64_t& idx) {
+  const uint32_t cam = blockIdx.x / blocks_per_cam;
+  const uint64_t local = (uint64_t)(blockIdx.x - cam * blocks_per_cam) * IB_ENTRIES + threadIdx.x;
+  idx = (uint64_t)cam * N + local;
+  return local < N;
+}
+
 __global__ void __launch_bounds__(IB_ENTRIES) isect_plan_kernel(
-    uint64_t total, const float* __restrict__ means2d, const int32_t* __restrict__ radii,
-    const float* __restrict__ depths, uint32_t tile_size, uint32_t tw, uint32_t th,
-    int32_t* __restrict__ tiles_per_gauss, IsectBlock* __restrict__ blocks) {
+    uint64_t N, uint32_t blocks_per_cam, const float* __restrict__ means2d,
+    const int32_t* __restrict__ radii, const float* __restrict__ depths, uint32_t tile_size,
+    uint32_t tw, uint32_t th, int32_t* __restrict__ tiles_per_gauss,
+    IsectBlock* __restrict__ blocks) {
   __shared__ IsectBlock s_w[IB_ENTRIES / 64];
-  const uint64_t idx = (uint64_t)blockIdx.x * IB_ENTRIES + threadIdx.x;
+  uint64_t idx;
   uint32_t n = 0u, key = 0u;
-  if (idx < total) {
+  if (isect_block_entry(N, blocks_per_cam, idx)) {
     const int32_t radius = radii[idx];
     if (radius > 0) {
       n = tile_count(
@@ -146,19 +195,21 @@ __global__ void __launch_bounds__(IB_ENTRIES) isect_plan_kernel(
   }
   int64_t sum = (int32_t)n;
   uint32_t kmin = n ? key : 0xffffffffu, kmax = n ? key : 0u;
+  const uint32_t any = (uint32_t)__popcll(tgs_ballot(n != 0u));
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     sum += __shfl_xor(sum, off, 64);
     kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, off, 64));
     kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, off, 64));
   }
-  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = IsectBlock{sum, kmin, kmax};
+  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = IsectBlock{sum, any, kmin, kmax, 0u};
   __syncthreads();
   if (threadIdx.x == 0) {
     IsectBlock b = s_w[0];
 #pragma unroll
     for (int w = 1; w < IB_ENTRIES / 64; ++w) {
       b.sum += s_w[w].sum;
+      b.entries += s_w[w].entries;
       b.kmin = min(b.kmin, s_w[w].kmin);
       b.kmax = max(b.kmax, s_w[w].kmax);
     }
@@ -166,37 +217,73 @@ __global__ void __launch_bounds__(IB_ENTRIES) isect_plan_kernel(
   }
 }
 
-// Exclusive scan of the blocks' sums in place by one workgroup, and the whole
-// range: summary = {intersections, kmin | kmax << 32}.
+// Exclusive scan of the blocks' sums in place by one workgroup, and the whole:
+// summary = {intersections, kmin | kmax << 32} and, for every camera, {entries,
+// intersections} up to its end.
 #define IB_SCAN_THREADS 1024
+#define IB_SCAN_ITEMS 4
 __global__ void __launch_bounds__(IB_SCAN_THREADS) isect_plan_scan_kernel(
-    uint32_t n_blocks, IsectBlock* __restrict__ blocks, uint64_t* __restrict__ summary) {
+    uint32_t n_blocks, uint32_t blocks_per_cam, IsectBlock* __restrict__ blocks,
+    uint64_t* __restrict__ summary) {
   constexpr int WAVES = IB_SCAN_THREADS / 64;
   __shared__ int64_t s_sum[WAVES];
-  __shared__ uint32_t s_min[WAVES], s_max[WAVES];
+  __shared__ uint32_t s_ent[WAVES], s_min[WAVES], s_max[WAVES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int64_t carry = 0;
-  uint32_t kmin = 0xffffffffu, kmax = 0u;
-  for (uint32_t base = 0; base < n_blocks; base += IB_SCAN_THREADS) {
-    const uint32_t i = base + threadIdx.x;
-    const IsectBlock b = i < n_blocks ? blocks[i] : IsectBlock{0, 0xffffffffu, 0u};
-    kmin = min(kmin, b.kmin);
-    kmax = max(kmax, b.kmax);
-    int64_t inc = b.sum;
+  int64_t sum_carry = 0;
+  uint32_t ent_carry = 0u, kmin = 0xffffffffu, kmax = 0u;
+  for (uint32_t base = 0; base < n_blocks; base += IB_SCAN_THREADS * IB_SCAN_ITEMS) {
+    const uint32_t i0 = base + threadIdx.x * IB_SCAN_ITEMS;
+    IsectBlock b[IB_SCAN_ITEMS];
+    int64_t sum = 0;
+    uint32_t ent = 0u;
+#pragma unroll
+    for (int k = 0; k < IB_SCAN_ITEMS; ++k) {
+      b[k] = i0 + k < n_blocks ? blocks[i0 + k] : IsectBlock{0, 0u, 0xffffffffu, 0u, 0u};
+      kmin = min(kmin, b[k].kmin);
+      kmax = max(kmax, b[k].kmax);
+      sum += b[k].sum;
+      ent += b[k].entries;
+    }
+    int64_t sum_inc = sum;
+    uint32_t ent_inc = ent;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
-      const int64_t o = __shfl_up(inc, off, 64);
-      if (lane >= off) inc += o;
+      const int64_t o = __shfl_up(sum_inc, off, 64);
+      const uint32_t e = __shfl_up(ent_inc, off, 64);
+      if (lane >= off) {
+        sum_inc += o;
+        ent_inc += e;
+      }
     }
-    if (lane == 63) s_sum[wave] = inc;
+    if (lane == 63) {
+      s_sum[wave] = sum_inc;
+      s_ent[wave] = ent_inc;
+    }
     __syncthreads();
-    int64_t before = carry;
+    int64_t sum_run = sum_carry + sum_inc - sum;
+    uint32_t ent_run = ent_carry + ent_inc - ent;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      if (w < wave) before += s_sum[w];
-      carry += s_sum[w];
+      if (w < wave) {
+        sum_run += s_sum[w];
+        ent_run += s_ent[w];
+      }
+      sum_carry += s_sum[w];
+      ent_carry += s_ent[w];
     }
-    if (i < n_blocks) blocks[i].sum = before + inc - b.sum;
+#pragma unroll
+    for (int k = 0; k < IB_SCAN_ITEMS; ++k) {
+      if (i0 + k >= n_blocks) break;
+      blocks[i0 + k].sum = sum_run;
+      blocks[i0 + k].entries = ent_run;
+      sum_run += b[k].sum;
+      ent_run += b[k].entries;
+      const uint32_t cam = (i0 + k) / blocks_per_cam;
+      if (i0 + k + 1 == (cam + 1) * blocks_per_cam) {
+        summary[2 + 2 * cam] = ent_run;
+        summary[3 + 2 * cam] = (uint64_t)sum_run;
+      }
+    }
     __syncthreads();
   }
 #pragma unroll
@@ -215,21 +302,21 @@ __global__ void __launch_bounds__(IB_SCAN_THREADS) isect_plan_scan_kernel(
       kmin = min(kmin, s_min[w]);
       kmax = max(kmax, s_max[w]);
     }
-    summary[0] = (uint64_t)carry;
+    summary[0] = (uint64_t)sum_carry;
     summary[1] = (uint64_t)kmin | ((uint64_t)kmax << 32);
   }
 }
 
 __global__ void __launch_bounds__(IB_ENTRIES) isect_emit_blocks_kernel(
-    uint64_t total, uint32_t N, const int64_t* __restrict__ camera_ids,
+    uint64_t plan_n, uint32_t blocks_per_cam, uint64_t N, const int64_t* __restrict__ camera_ids,
     const float* __restrict__ means2d, const int32_t* __restrict__ radii,
     const float* __restrict__ depths, const int32_t* __restrict__ tiles_per_gauss,
     const IsectBlock* __restrict__ blocks, uint32_t tile_size, uint32_t tw, uint32_t th,
     uint32_t tile_n_bits, int64_t* __restrict__ isect_ids, int32_t* __restrict__ flatten_ids) {
   __shared__ int64_t s_w[IB_ENTRIES / 64];
-  const uint64_t idx = (uint64_t)blockIdx.x * IB_ENTRIES + threadIdx.x;
+  uint64_t idx;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int32_t n = idx < total ? tiles_per_gauss[idx] : 0;
+  const int32_t n = isect_block_entry(plan_n, blocks_per_cam, idx) ? tiles_per_gauss[idx] : 0;
   int64_t inc = n;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -246,49 +333,76 @@ __global__ void __launch_bounds__(IB_ENTRIES) isect_emit_blocks_kernel(
             isect_ids, flatten_ids);
 }
 
-extern "C" uint64_t tgs_isect_tiles_plan_size(uint64_t total) {
-  return (total + IB_ENTRIES - 1) / IB_ENTRIES * sizeof(IsectBlock);
+// The cameras the two sorts take (one segment of the sorts and of the fused
+// emission each); a plan for more is laid out as one camera of them all, so that
+// many small cameras still fill their blocks.
+#define IB_MAX_CAMS 32
+
+struct IsectGrid {
+  uint32_t cams, per_cam;
+  uint64_t n;
+};
+
+static IsectGrid isect_grid(uint32_t C, uint64_t N) {
+  const uint32_t cams = C <= IB_MAX_CAMS ? C : 1u;
+  const uint64_t n = C <= IB_MAX_CAMS ? N : (uint64_t)C * N;
+  return IsectGrid{cams, tgs_blocks(n, IB_ENTRIES), n};
 }
 
-extern "C" int tgs_isect_tiles_plan(uint64_t total, const float* means2d, const int32_t* radii,
-                                    const float* depths, uint32_t tile_size, uint32_t tile_width,
-                                    uint32_t tile_height, int32_t* tiles_per_gauss, void* plan,
-                                    size_t plan_bytes, uint64_t* summary, hipStream_t stream) {
-  TGS_CHECK_ARG(total > 0, "isect_tiles_plan: nothing to plan");
+static int isect_plan_check(const char* who, uint32_t C, uint64_t N) {
+  TGS_CHECK_ARG(C > 0 && N > 0, "%s: nothing to plan", who);
+  TGS_CHECK_ARG((uint64_t)C * N < (1ull << 31),
+                "isect_tiles: C*N (or nnz) must fit int32 flatten ids");
+  return TGS_OK;
+}
+
+extern "C" uint64_t tgs_isect_tiles_plan_size(uint32_t C, uint64_t N) {
+  const IsectGrid g = isect_grid(C, N);
+  return (uint64_t)g.cams * g.per_cam * sizeof(IsectBlock);
+}
+
+extern "C" int tgs_isect_tiles_plan(uint32_t C, uint64_t N, const float* means2d,
+                                    const int32_t* radii, const float* depths, uint32_t tile_size,
+                                    uint32_t tile_width, uint32_t tile_height,
+                                    int32_t* tiles_per_gauss, void* plan, size_t plan_bytes,
+                                    uint64_t* summary, hipStream_t stream) {
+  int rc = isect_plan_check("isect_tiles_plan", C, N);
+  if (rc) return rc;
   TGS_CHECK_ARG(means2d && radii && depths && tiles_per_gauss && plan && summary &&
-                    ((uintptr_t)plan & 15u) == 0,
-                "isect_tiles_plan: null pointer (or a plan not 16-byte aligned)");
+                    ((uintptr_t)plan & 7u) == 0,
+                "isect_tiles_plan: null pointer (or a plan not 8-byte aligned)");
   TGS_CHECK_ARG(tile_size > 0, "tile_size must be > 0");
-  TGS_CHECK_ARG(total < (1ull << 31), "isect_tiles: C*N (or nnz) must fit int32 flatten ids");
-  if (plan_bytes < tgs_isect_tiles_plan_size(total)) {
+  if (plan_bytes < tgs_isect_tiles_plan_size(C, N)) {
     tgs_set_error("isect_tiles_plan: plan buffer too small");
     return TGS_ERR_WORKSPACE;
   }
-  const uint32_t nb = tgs_blocks(total, IB_ENTRIES);
-  hipLaunchKernelGGL(isect_plan_kernel, dim3(nb), dim3(IB_ENTRIES), 0, stream, total, means2d,
-                     radii, depths, tile_size, tile_width, tile_height, tiles_per_gauss,
+  const IsectGrid g = isect_grid(C, N);
+  hipLaunchKernelGGL(isect_plan_kernel, dim3(g.cams * g.per_cam), dim3(IB_ENTRIES), 0, stream, g.n,
+                     g.per_cam, means2d, radii, depths, tile_size, tile_width, tile_height, tiles_per_gauss,
                      (IsectBlock*)plan);
   TGS_LAUNCH_CHECK("isect_plan");
-  hipLaunchKernelGGL(isect_plan_scan_kernel, dim3(1), dim3(IB_SCAN_THREADS), 0, stream, nb,
-                     (IsectBlock*)plan, summary);
+  hipLaunchKernelGGL(isect_plan_scan_kernel, dim3(1), dim3(IB_SCAN_THREADS), 0, stream,
+                     g.cams * g.per_cam, g.per_cam, (IsectBlock*)plan, summary);
   TGS_RETURN_LAUNCH("tgs_isect_tiles_plan");
 }
 
-extern "C" int tgs_isect_tiles_emit_plan(uint64_t total, uint32_t N, const int64_t* camera_ids,
+extern "C" int tgs_isect_tiles_emit_plan(uint32_t C, uint64_t N, const int64_t* camera_ids,
                                          const float* means2d, const int32_t* radii,
                                          const float* depths, const int32_t* tiles_per_gauss,
                                          const void* plan, uint32_t tile_size,
                                          uint32_t tile_width, uint32_t tile_height,
                                          uint32_t tile_n_bits, int64_t* isect_ids,
                                          int32_t* flatten_ids, hipStream_t stream) {
-  if (total == 0) return TGS_OK;
+  int rc = isect_plan_check("isect_tiles_emit_plan", C, N);
+  if (rc) return rc;
   TGS_CHECK_ARG(means2d && radii && depths && tiles_per_gauss && plan && isect_ids && flatten_ids,
                 "isect_tiles_emit_plan: null pointer");
-  TGS_CHECK_ARG(camera_ids || N > 0, "isect_tiles_emit_plan: need camera_ids or N");
-  hipLaunchKernelGGL(isect_emit_blocks_kernel, dim3(tgs_blocks(total, IB_ENTRIES)),
-                     dim3(IB_ENTRIES), 0, stream, total, N, camera_ids, means2d, radii, depths,
-                     tiles_per_gauss, (const IsectBlock*)plan, tile_size, tile_width, tile_height,
-                     tile_n_bits, isect_ids, flatten_ids);
+  TGS_CHECK_ARG(tile_size > 0, "tile_size must be > 0");
+  const IsectGrid g = isect_grid(C, N);
+  hipLaunchKernelGGL(isect_emit_blocks_kernel, dim3(g.cams * g.per_cam), dim3(IB_ENTRIES), 0, stream, g.n,
+                     g.per_cam, N, camera_ids, means2d, radii, depths, tiles_per_gauss,
+                     (const IsectBlock*)plan, tile_size, tile_width, tile_height, tile_n_bits,
+                     isect_ids, flatten_ids);
   TGS_RETURN_LAUNCH("tgs_isect_tiles_emit_plan");
 }
 
@@ -299,6 +413,170 @@ extern "C" uint32_t tgs_bit_width(uint32_t v) {
     v >>= 1;
   }
   return b;
+}
+
+// ---------------------------------------------------------------------------
+// The reference's order in two sorts: Gaussians by depth (32-bit keys), then the
+// intersections they emit in that order by tile, stably, gives (camera, tile,
+// depth, Gaussian) with two 8-byte moves per intersection instead of the single
+// sort's five 12-byte ones.  isect_tiles and offsets, single sort and two: 1.2M
+// Gaussians, 2.7M intersections 240 and 232 us; a 500k-Gaussian 1237x822 image with
+// its backward 807 and 786 us.  The single sort takes what this does not: packed
+// camera ids (in any order), grids past 255 tiles a side (8-bit rectangles), more
+// cameras than the emission's segments, negative depths (their sign fills the id).
+// ---------------------------------------------------------------------------
+// Depth keys and tile rectangles (x0 | x1 << 8 | y0 << 16 | y1 << 24, above the
+// index) of the Gaussians that meet any tile, in order.
+__global__ void __launch_bounds__(IB_ENTRIES) isect_entries_kernel(
+    uint64_t N, uint32_t blocks_per_cam, const float* __restrict__ means2d,
+    const int32_t* __restrict__ radii, const float* __restrict__ depths, uint32_t tile_size,
+    uint32_t tw, uint32_t th, const IsectBlock* __restrict__ blocks, uint32_t* __restrict__ keys,
+    uint64_t* __restrict__ rects) {
+  __shared__ uint32_t s_w[IB_ENTRIES / 64];
+  uint64_t idx;
+  TileRect r{0u, 0u, 0u, 0u};
+  if (isect_block_entry(N, blocks_per_cam, idx)) {
+    const int32_t radius = radii[idx];
+    if (radius > 0)
+      r = tile_rect(means2d[idx * 2], means2d[idx * 2 + 1], radius, tile_size, tw, th);
+  }
+  const bool any = tile_count(r) != 0u;
+  const uint64_t m = tgs_ballot(any);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) s_w[wave] = (uint32_t)__popcll(m);
+  __syncthreads();
+  if (!any) return;
+  uint32_t pos = blocks[blockIdx.x].entries + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+  for (int w = 0; w < wave; ++w) pos += s_w[w];
+  keys[pos] = (uint32_t)__float_as_int(depths[idx]);
+  rects[pos] = (uint64_t)(r.x0 | (r.x1 << 8) | (r.y0 << 16) | (r.y1 << 24)) << 32 | (uint32_t)idx;
+}
+
+// The 64-bit ids of sorted camera | tile keys; the flatten ids too where the sort
+// left them in scratch.
+__global__ void __launch_bounds__(256) isect_rebuild_ids_kernel(
+    uint32_t n, const uint32_t* __restrict__ keys, const int32_t* fids,
+    const float* __restrict__ depths, int64_t* __restrict__ isect_ids, int32_t* flatten_ids) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int32_t f = fids[i];
+  isect_ids[i] = ((int64_t)keys[i] << 32) | (int64_t)__float_as_int(depths[f]);
+  if (flatten_ids != fids) flatten_ids[i] = f;
+}
+
+struct IsectSorted {
+  uint32_t V, n, tile_bits;  // entries, intersections, bit width of the tile count
+  uint32_t ent[IB_MAX_CAMS + 1], isect[IB_MAX_CAMS + 1];
+  uint64_t hist_words, dkeys, dkeys2, rects, hist, scan, keys, keys2, fids2, sort_ws, scan_ws, end;
+  size_t sort_bytes, scan_bytes;
+};
+
+// False where the two sorts do not apply.
+static bool isect_sorted_layout(uint32_t C, const uint64_t* summary, uint32_t tile_width,
+                                uint32_t tile_height, IsectSorted& o) {
+  if (!summary || C == 0 || C > IB_MAX_CAMS || tile_width == 0 || tile_height == 0 || tile_width > 255 ||
+      tile_height > 255 || summary[0] == 0 || summary[0] >= (1ull << 31) || summary[1] >> 63)
+    return false;
+  o = IsectSorted{};
+  o.tile_bits = tgs_bit_width(tile_width * tile_height);
+  for (uint32_t c = 0; c < C; ++c) {
+    o.ent[c + 1] = (uint32_t)summary[2 + 2 * c];
+    o.isect[c + 1] = (uint32_t)summary[3 + 2 * c];
+  }
+  o.V = o.ent[C];
+  o.n = o.isect[C];
+  o.hist_words = tgs_tide_isect_fused_hist_words(C, o.ent, o.tile_bits);
+  if (o.hist_words == 0 || o.n != summary[0]) return false;
+  o.sort_bytes = std::max(tgs_segmented_sort_workspace_size(o.V, C),
+                          tgs_segmented_sort_workspace_size(o.n, C));
+  o.scan_bytes = tgs_scan_workspace_size(o.hist_words);
+  uint64_t at = 0;
+  auto take = [&](uint64_t bytes) {
+    const uint64_t a = at;
+    at += (bytes + 255) & ~255ull;
+    return a;
+  };
+  o.dkeys = take(4ull * o.V);
+  o.dkeys2 = take(4ull * o.V);
+  o.rects = take(8ull * o.V);
+  o.hist = take(4 * o.hist_words);
+  o.scan = take(4 * o.hist_words);
+  o.keys = take(4ull * o.n);
+  o.keys2 = take(4ull * o.n);
+  o.fids2 = take(4ull * o.n);
+  o.sort_ws = take(o.sort_bytes);
+  o.scan_ws = take(o.scan_bytes);
+  o.end = at;
+  return true;
+}
+
+extern "C" uint64_t tgs_isect_tiles_sorted_workspace_size(uint32_t C, const uint64_t* summary,
+                                                          uint32_t tile_width,
+                                                          uint32_t tile_height) {
+  IsectSorted o;
+  return isect_sorted_layout(C, summary, tile_width, tile_height, o) ? o.end : 0;
+}
+
+extern "C" int tgs_isect_tiles_sorted(uint32_t C, uint64_t N, const float* means2d,
+                                      const int32_t* radii, const float* depths, const void* plan,
+                                      const uint64_t* summary, uint32_t tile_size,
+                                      uint32_t tile_width, uint32_t tile_height,
+                                      int64_t* isect_ids, int32_t* flatten_ids, void* workspace,
+                                      size_t workspace_bytes, hipStream_t stream) {
+  int rc = isect_plan_check("isect_tiles_sorted", C, N);
+  if (rc) return rc;
+  IsectSorted o;
+  TGS_CHECK_ARG(isect_sorted_layout(C, summary, tile_width, tile_height, o),
+                "isect_tiles_sorted: not for these cameras, tiles or depths");
+  TGS_CHECK_ARG(means2d && radii && depths && plan && isect_ids && flatten_ids && workspace,
+                "isect_tiles_sorted: null pointer");
+  TGS_CHECK_ARG(tile_size > 0, "tile_size must be > 0");
+  TGS_CHECK_ARG((uint64_t)o.V <= (uint64_t)C * N, "isect_tiles_sorted: not this plan's summary");
+  if (workspace_bytes < o.end) {
+    tgs_set_error("isect_tiles_sorted: workspace %zu < %llu", workspace_bytes,
+                  (unsigned long long)o.end);
+    return TGS_ERR_WORKSPACE;
+  }
+  char* w = (char*)workspace;
+  uint32_t *dkeys = (uint32_t*)(w + o.dkeys), *dkeys2 = (uint32_t*)(w + o.dkeys2);
+  uint64_t *rects = (uint64_t*)(w + o.rects), *rects2 = (uint64_t*)isect_ids;  // V <= n
+  uint32_t *hist = (uint32_t*)(w + o.hist), *scan = (uint32_t*)(w + o.scan);
+  uint32_t *keys = (uint32_t*)(w + o.keys), *keys2 = (uint32_t*)(w + o.keys2);
+  int32_t *fids = (int32_t*)(w + o.fids2), *fids2 = flatten_ids;
+  const IsectGrid g = isect_grid(C, N);
+  hipLaunchKernelGGL(isect_entries_kernel, dim3(g.cams * g.per_cam), dim3(IB_ENTRIES), 0, stream, g.n,
+                     g.per_cam, means2d, radii, depths, tile_size, tile_width, tile_height,
+                     (const IsectBlock*)plan, dkeys, rects);
+  TGS_LAUNCH_CHECK("isect_entries");
+  const uint32_t kmin = (uint32_t)summary[1], kmax = (uint32_t)(summary[1] >> 32);
+  int sel = 0;
+  rc = tgs_segmented_sort_pairs_u32_range(dkeys, rects, dkeys2, rects2, 8, o.V, C, o.ent, kmin,
+                                          (int)std::max(1u, tgs_bit_width(kmax - kmin)),
+                                          w + o.sort_ws, o.sort_bytes, &sel, stream);
+  if (rc) return rc;
+  if (sel) rects = rects2;
+  if ((rc = tgs_tide_isect_fused_count(C, o.ent, rects, tile_width, o.tile_bits, hist,
+                                       o.hist_words, stream)))
+    return rc;
+  if ((rc = tgs_exclusive_scan_u32(hist, scan, o.hist_words, w + o.scan_ws, o.scan_bytes, stream)))
+    return rc;
+  if ((rc = tgs_tide_isect_fused_scatter(C, o.ent, rects, tile_width, o.tile_bits, scan,
+                                         o.hist_words, o.n, keys, fids, stream)))
+    return rc;
+  const int first = (int)tgs_tide_isect_fused_digit_bits(o.tile_bits);
+  if ((int)o.tile_bits > first) {
+    sel = 0;
+    rc = tgs_segmented_sort_pairs_u32(keys, fids, keys2, fids2, 4, o.n, C, o.isect, first,
+                                      (int)o.tile_bits, w + o.sort_ws, o.sort_bytes, &sel, stream);
+    if (rc) return rc;
+    if (sel) {
+      keys = keys2;
+      fids = fids2;
+    }
+  }
+  hipLaunchKernelGGL(isect_rebuild_ids_kernel, dim3(tgs_blocks(o.n, 256)), dim3(256), 0, stream,
+                     o.n, keys, fids, depths, isect_ids, flatten_ids);
+  TGS_RETURN_LAUNCH("tgs_isect_tiles_sorted");
 }
 
 extern "C" int tgs_isect_tiles_count(uint64_t total, const float* means2d, const int32_t* radii,

@@ -371,19 +371,30 @@ def isect_tiles(
         return (tiles_per_gauss, torch.empty(0, dtype=torch.int64, device=dev),
                 torch.empty(0, dtype=torch.int32, device=dev))
     lib = N.load()
-    plan = torch.empty(lib.tgs_isect_tiles_plan_size(total), dtype=torch.uint8, device=dev)
-    summary = torch.empty(2, dtype=torch.int64, device=dev)
-    N.call("tgs_isect_tiles_plan", total, N.ptr(means2d), N.ptr(radii), N.ptr(depths), tile_size,
-           tile_width, tile_height, N.ptr(tiles_per_gauss), N.ptr(plan), plan.numel(),
+    plan_c, plan_n = (1, total) if packed else (C, Nn)
+    plan = torch.empty(lib.tgs_isect_tiles_plan_size(plan_c, plan_n), dtype=torch.uint8, device=dev)
+    summary = torch.empty(2 + 2 * plan_c, dtype=torch.int64, device=dev)
+    N.call("tgs_isect_tiles_plan", plan_c, plan_n, N.ptr(means2d), N.ptr(radii), N.ptr(depths),
+           tile_size, tile_width, tile_height, N.ptr(tiles_per_gauss), N.ptr(plan), plan.numel(),
            N.ptr(summary), s)
-    n_isects, key_range = summary.tolist()
+    summary = summary.cpu()
+    n_isects, key_range = summary[:2].tolist()
     isect_ids = torch.empty(n_isects, dtype=torch.int64, device=dev)
     flatten_ids = torch.empty(n_isects, dtype=torch.int32, device=dev)
-    if n_isects:
-        N.call("tgs_isect_tiles_emit_plan", total, Nn, N.ptr(cam_ids), N.ptr(means2d),
-               N.ptr(radii), N.ptr(depths), N.ptr(tiles_per_gauss), N.ptr(plan), tile_size,
-               tile_width, tile_height, tile_n_bits, N.ptr(isect_ids), N.ptr(flatten_ids), s)
-    if n_isects and sort:
+    if n_isects == 0:
+        return tiles_per_gauss, isect_ids, flatten_ids
+    ws_bytes = 0 if packed or not sort else lib.tgs_isect_tiles_sorted_workspace_size(
+        C, N.ptr(summary), tile_width, tile_height)
+    if ws_bytes:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        N.call("tgs_isect_tiles_sorted", C, Nn, N.ptr(means2d), N.ptr(radii), N.ptr(depths),
+               N.ptr(plan), N.ptr(summary), tile_size, tile_width, tile_height, N.ptr(isect_ids),
+               N.ptr(flatten_ids), N.ptr(ws), ws_bytes, s)
+        return tiles_per_gauss, isect_ids, flatten_ids
+    N.call("tgs_isect_tiles_emit_plan", plan_c, plan_n, N.ptr(cam_ids), N.ptr(means2d),
+           N.ptr(radii), N.ptr(depths), N.ptr(tiles_per_gauss), N.ptr(plan), tile_size,
+           tile_width, tile_height, tile_n_bits, N.ptr(isect_ids), N.ptr(flatten_ids), s)
+    if sort:
         kmin, kmax = key_range & 0xFFFFFFFF, (key_range >> 32) & 0xFFFFFFFF
         if kmax >> 31:  # a negative depth's sign fills the high word, as in the reference
             isect_ids, flatten_ids = radix_sort_pairs(isect_ids, flatten_ids,
