@@ -721,6 +721,14 @@ __global__ void __launch_bounds__(256) tide_isect_emit_blocked_kernel(
 // ---------------------------------------------------------------------------
 #define FE_CHUNK 2048
 #define FE_KEYS (FE_CHUNK / 256)
+// A rectangle of more tiles than this is walked by its whole wave: one thread
+// took a launch's tail for a splat of a thousand tiles.  Count and scan, emission
+// and tile pass, in us, one thread and the wave: 463k entries of a 1237x822 image
+// 102 and 84, 58 and 51; 37k of 640x400 77 and 69, 40 and 35; 9.6k of 256x256
+// 60 and 55, 31 and 31.  16 and 64 measured the same, 8 slower.  The emission's
+// blocks of 1024 entries keep one thread: with two million entries or more other
+// blocks fill the tail, and the ballots cost 1432 -> 1517 us at 58M.
+#define FE_WIDE 32u
 
 struct FusedEmit {
   uint32_t C;
@@ -751,6 +759,7 @@ template <int FE_ITEMS>  // entries per thread: fe.entries = 256 * FE_ITEMS
 __global__ void __launch_bounds__(256) tide_isect_fused_count_kernel(
     FusedEmit fe, const uint64_t* __restrict__ rects, uint32_t* __restrict__ hist) {
   __shared__ uint32_t s_cnt[256];
+  const int lane = threadIdx.x & 63;
   uint32_t c, bl, e0, e1;
   fe_block(fe, blockIdx.x, c, bl, e0, e1);
   s_cnt[threadIdx.x] = 0u;
@@ -764,10 +773,20 @@ __global__ void __launch_bounds__(256) tide_isect_fused_count_kernel(
   }
 #pragma unroll
   for (int k = 0; k < FE_ITEMS; ++k) {
-    const uint32_t x0 = rc[k] & 255u, x1 = (rc[k] >> 8) & 255u, y0 = (rc[k] >> 16) & 255u,
-                   y1 = rc[k] >> 24;
-    for (uint32_t y = y0; y < y1; ++y)
-      for (uint32_t x = x0; x < x1; ++x) atomicAdd(&s_cnt[(y * fe.tw + x) & fe.mask], 1u);
+    const bool wide = rect_tiles(rc[k]) > FE_WIDE;
+    if (!wide) {
+      const uint32_t x0 = rc[k] & 255u, x1 = (rc[k] >> 8) & 255u, y0 = (rc[k] >> 16) & 255u,
+                     y1 = rc[k] >> 24;
+      for (uint32_t y = y0; y < y1; ++y)
+        for (uint32_t x = x0; x < x1; ++x) atomicAdd(&s_cnt[(y * fe.tw + x) & fe.mask], 1u);
+    }
+    for (uint64_t m = tgs_ballot(wide); m; m &= m - 1) {
+      const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)rc[k], __builtin_ctzll(m));
+      const uint32_t x1 = (r >> 8) & 255u, y1 = r >> 24;
+      for (uint32_t y = ((r >> 16) & 255u) + (lane >> 3); y < y1; y += 8)
+        for (uint32_t x = (r & 255u) + (lane & 7); x < x1; x += 8)
+          atomicAdd(&s_cnt[(y * fe.tw + x) & fe.mask], 1u);
+    }
   }
   __syncthreads();
   if (threadIdx.x <= fe.mask) hist[fe_hist_index(fe, c, threadIdx.x, bl)] = s_cnt[threadIdx.x];
@@ -833,7 +852,22 @@ __global__ void __launch_bounds__(256) tide_isect_fused_scatter_kernel(
     for (int k = 0; k < FE_ITEMS; ++k) {
       const uint32_t a = rect_tiles(rc[k]);
       const uint32_t lo = max(p[k], q0), hi = min(p[k] + a, q0 + FE_CHUNK);
-      if (lo < hi) {
+      const bool wide = FE_ITEMS == 1 && a > FE_WIDE && lo < hi;
+      for (uint64_t m = tgs_ballot(wide); m; m &= m - 1) {
+        const int src = __builtin_ctzll(m);
+        const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)rc[k], src);
+        const uint32_t pr = (uint32_t)__builtin_amdgcn_readlane((int)p[k], src);
+        const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)hi, src);
+        const int32_t f = __builtin_amdgcn_readlane(id[k], src);
+        const uint32_t x0 = r & 255u, w = ((r >> 8) & 255u) - x0;
+        const uint32_t first = ((r >> 16) & 255u) * fe.tw + x0;
+        for (uint32_t i = max(pr, q0) + lane; i < end; i += 64) {
+          const uint32_t o = i - pr, y = o / w;
+          s_k[i - q0] = cam_enc | (first + y * fe.tw + (o - y * w));
+          s_v[i - q0] = f;
+        }
+      }
+      if (lo < hi && !wide) {
         const uint32_t x0 = rc[k] & 255u, x1 = (rc[k] >> 8) & 255u, y0 = (rc[k] >> 16) & 255u;
         const uint32_t w = x1 - x0;
         const uint32_t o = lo - p[k];  // nonzero only for an entry spanning chunks
