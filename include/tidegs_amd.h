@@ -570,6 +570,30 @@ int tgs_tide_rasterize_bwd(uint32_t C, const float* splats, const float* backgro
                            uint32_t n_isects, const float* alphas, const int32_t* last_ids,
                            const float* v_images, const float* v_alphas, float* splat_grads,
                            tgs_stream_t stream);
+/* The same two calls with the tiles of the longest lists first, for launches of a
+ * few rounds of workgroups.  tgs_tide_raster_order_tiles: the int32 words of the
+ * order (0: this size is not ordered, order = null); tgs_tide_raster_order writes
+ * it, and any permutation of the C * tile_height * tile_width tiles is one. */
+uint64_t tgs_tide_raster_order_tiles(uint32_t C, uint32_t tile_width, uint32_t tile_height,
+                                     uint32_t n_isects);
+int tgs_tide_raster_order(uint32_t C, uint32_t tile_width, uint32_t tile_height,
+                          const int32_t* tile_offsets, uint32_t n_isects, int32_t* order,
+                          tgs_stream_t stream);
+int tgs_tide_rasterize_fwd_ordered(uint32_t C, const float* splats, const float* backgrounds,
+                                   uint32_t W, uint32_t H, uint32_t tile_width,
+                                   uint32_t tile_height, const int32_t* tile_offsets,
+                                   const int32_t* flatten_ids, uint32_t n_isects, float* images,
+                                   float* alphas, int32_t* last_ids, const int32_t* order,
+                                   int32_t* n_contrib, float* clear, uint64_t clear_words,
+                                   tgs_stream_t stream);
+int tgs_tide_rasterize_bwd_ordered(uint32_t C, const float* splats, const float* backgrounds,
+                                   uint32_t W, uint32_t H, uint32_t tile_width,
+                                   uint32_t tile_height, const int32_t* tile_offsets,
+                                   const int32_t* flatten_ids, uint32_t n_isects,
+                                   const float* alphas, const int32_t* last_ids,
+                                   const float* v_images, const float* v_alphas,
+                                   float* splat_grads, const int32_t* order,
+                                   tgs_stream_t stream);
 /* The same two calls with the backward split along the tiles' lists, for images
  * of few tiles: the forward leaves each pixel's state at the end of every
  * segment of a list, and the backward runs one workgroup per (tile, segment).
@@ -583,8 +607,8 @@ int tgs_tide_rasterize_fwd_split(uint32_t C, const float* splats, const float* b
                                  uint32_t tile_height, const int32_t* tile_offsets,
                                  const int32_t* flatten_ids, uint32_t n_isects, float* images,
                                  float* alphas, int32_t* last_ids, float* clear,
-                                 uint64_t clear_words, float* states, int32_t* item_tile,
-                                 tgs_stream_t stream);
+                                 uint64_t clear_words, const int32_t* order, float* states,
+                                 int32_t* item_tile, tgs_stream_t stream);
 int tgs_tide_rasterize_bwd_split(uint32_t C, const float* splats, const float* backgrounds,
                                  uint32_t W, uint32_t H, uint32_t tile_width,
                                  uint32_t tile_height, const int32_t* tile_offsets,

@@ -843,3 +843,38 @@ def test_rasterize_split_matches_whole_tiles(gpu, n, tw, th, crop, what):
         np.testing.assert_array_equal(np.isfinite(a), fine)
         np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
         assert rel_l2(a[fine], b[fine]) < 2e-5
+
+
+@pytest.mark.parametrize("C,tw,th", [(3, 23, 23),    # 1587 tiles: just past one round, split too
+                                     (7, 31, 30),    # 6510: the backward ordered as well
+                                     (2, 64, 64), (4, 64, 64)])  # the largest camera, the most tiles
+def test_raster_order_permutes_and_matches(gpu, C, tw, th):
+    """The longest-first tile order is a permutation by octaves of the lists'
+    lengths, each octave in tile order, and rendering in it matches the kernels
+    in tile order (the SoA ones, which absgrad selects): bit-identical images,
+    gradients to the order of the sums (float32, relative 2-norm 2e-5)."""
+    from tidegs_amd import _native as N
+    announce(f"raster order C={C} tiles={tw}x{th}")
+    n = C * tw * th
+    W, H = tw * 16 - 5, th * 16 - 3
+    m2d, conics, colors, opacs, offs, flat = _raster_case(gpu, seed=n, C=C, W=W, H=H)
+    assert N.load().tgs_tide_raster_order_tiles(C, tw, th, flat.numel()) == n
+    order = torch.full((n,), -1, dtype=torch.int32, device=gpu)
+    N.call("tgs_tide_raster_order", C, tw, th, N.ptr(offs), flat.numel(), N.ptr(order),
+           N.stream_handle(gpu))
+    lengths = np.diff(to_np(offs).reshape(-1), append=flat.numel())
+    bits = np.frexp(lengths.astype(np.float64))[1]  # bit length, 0 for an empty list
+    top = max(flat.numel() // n, 1).bit_length() + 2
+    cls = np.clip(top - bits, 0, 7)
+    np.testing.assert_array_equal(to_np(order), np.argsort(cls, kind="stable"))
+    g = torch.Generator(device=gpu).manual_seed(1)
+    v = [torch.randn((C, H, W, k), generator=g, device=gpu) for k in (3, 1)]
+    out = []
+    for absgrad in (False, True):
+        leaves = [t.clone().requires_grad_() for t in (m2d, conics, colors, opacs)]
+        rc, ra = ops.rasterize_to_pixels(*leaves, W, H, 16, offs, flat, absgrad=absgrad)
+        out.append((rc, ra, torch.autograd.grad((rc, ra), leaves, v)))
+    (rc, ra, grads), (rc2, ra2, grads2) = out
+    assert torch.equal(rc, rc2) and torch.equal(ra, ra2)
+    for a, b in zip(grads, grads2):
+        assert rel_l2(to_np(a), to_np(b)) < 2e-5

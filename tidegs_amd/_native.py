@@ -155,10 +155,16 @@ SIGNATURES = {
         ctypes.c_int, [U32, P, P, U32, U32, U32, U32, P, P, U32, P, P, P, P, P, U64, P]),
     "tgs_tide_rasterize_bwd": (
         ctypes.c_int, [U32, P, P, U32, U32, U32, U32, P, P, U32, P, P, P, P, P, P]),
+    "tgs_tide_raster_order_tiles": (U64, [U32, U32, U32, U32]),
+    "tgs_tide_raster_order": (ctypes.c_int, [U32, U32, U32, P, U32, P, P]),
+    "tgs_tide_rasterize_fwd_ordered": (
+        ctypes.c_int, [U32, P, P, U32, U32, U32, U32, P, P, U32, P, P, P, P, P, P, U64, P]),
+    "tgs_tide_rasterize_bwd_ordered": (
+        ctypes.c_int, [U32, P, P, U32, U32, U32, U32, P, P, U32, P, P, P, P, P, P, P]),
     "tgs_tide_raster_split_items": (U64, [U32, U32, U32, U32]),
     "tgs_tide_rasterize_fwd_split": (
         ctypes.c_int,
-        [U32, P, P, U32, U32, U32, U32, P, P, U32, P, P, P, P, U64, P, P, P]),
+        [U32, P, P, U32, U32, U32, U32, P, P, U32, P, P, P, P, U64, P, P, P, P]),
     "tgs_tide_rasterize_bwd_split": (
         ctypes.c_int,
         [U32, P, P, U32, U32, U32, U32, P, P, U32, P, P, P, P, P, P, P, P]),

@@ -131,6 +131,7 @@ struct RasterGeom {
   uint32_t W, H;
   uint32_t tile_w, tile_h;
   uint32_t n_isects;
+  const int32_t* order = nullptr;  // tiles in launch order (raster_order_kernel)
 };
 
 // ---------------------------------------------------------------------------
@@ -478,6 +479,17 @@ __device__ __forceinline__ void xcd_line_order(uint32_t lin, uint32_t n_lines, u
   }
 }
 
+// Camera, row and column of camera-major tile t (one past the last: the last).
+__device__ __forceinline__ void raster_tile(const RasterGeom& G, uint32_t t, uint32_t& cam,
+                                            uint32_t& ty, uint32_t& tx) {
+  const uint32_t per_cam = G.tile_h * G.tile_w;
+  t = min(t, G.C * per_cam - 1u);
+  cam = t / per_cam;
+  t -= cam * per_cam;
+  ty = t / G.tile_w;
+  tx = t - ty * G.tile_w;
+}
+
 // ---------------------------------------------------------------------------
 // Split tiles.  A tile's list is one serial chain per pixel, so a small image
 // (256 tiles on 256 CUs) runs one workgroup per CU and waits for the deepest
@@ -548,8 +560,8 @@ __global__ void __launch_bounds__(TILE* TILE, SPLIT ? 6 : CDIM <= 4 ? 8 : 1) ras
   constexpr int EMH = TILE == 16 ? 1 : BATCH;
   __shared__ __align__(16) uint32_t s_emh[WAVES][2][EMH];
 
-  const uint32_t cam = blockIdx.z;
-  const uint32_t ty = blockIdx.y, tx = blockIdx.x;
+  uint32_t cam = blockIdx.z, ty = blockIdx.y, tx = blockIdx.x;
+  if (G.order) raster_tile(G, (uint32_t)G.order[(cam * G.tile_h + ty) * G.tile_w + tx], cam, ty, tx);
   const uint32_t tile_id = ty * G.tile_w + tx;
   const uint32_t tr = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane((int)(tr >> 6));  // wave-uniform
@@ -843,12 +855,10 @@ __global__ void __launch_bounds__(TILE* TILE, CDIM <= 4 ? 6 : 1) raster_bwd_kern
   if (SPLIT) {
     // an item that no tile has (offsets that do not start at 0) holds anything:
     // the range test below refuses what is not this tile's
-    const uint32_t tile_lin =
-        min((uint32_t)split.item_tile[blockIdx.x], G.C * G.tile_h * G.tile_w - 1u);
-    cam = tile_lin / (G.tile_h * G.tile_w);
-    const uint32_t t = tile_lin - cam * (G.tile_h * G.tile_w);
-    ty = t / G.tile_w;
-    tx = t - ty * G.tile_w;
+    raster_tile(G, (uint32_t)split.item_tile[blockIdx.x], cam, ty, tx);
+  } else if (G.order) {
+    raster_tile(G, (uint32_t)G.order[(blockIdx.z * G.tile_w + blockIdx.y) * G.tile_h + blockIdx.x],
+                cam, ty, tx);
   } else {
     cam = blockIdx.z;
     xcd_line_order(blockIdx.y * G.tile_h + blockIdx.x, G.tile_w, G.tile_h, tx, ty);

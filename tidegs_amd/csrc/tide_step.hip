@@ -1821,13 +1821,119 @@ extern "C" int tgs_tide_isect_ids(uint32_t n_isects, const uint32_t* keys,
   TGS_RETURN_LAUNCH("tgs_tide_isect_ids");
 }
 
-extern "C" int tgs_tide_rasterize_fwd(uint32_t C, const float* splats, const float* backgrounds,
-                                      uint32_t W, uint32_t H, uint32_t tile_width,
-                                      uint32_t tile_height, const int32_t* tile_offsets,
-                                      const int32_t* flatten_ids, uint32_t n_isects,
-                                      float* images, float* alphas, int32_t* last_ids,
-                                      int32_t* n_contrib, float* clear, uint64_t clear_words,
-                                      hipStream_t stream) {
+// Longest lists first.  Several cameras of few tiles end on the last camera's long
+// lists, each a serial chain per pixel, with the rest of the card idle: at 4
+// cameras of 2170 tiles the forward issued 73% of the instructions per time it
+// does at 130k tiles.  Forward (this launch included) and backward in tile order
+// and ordered, in us:
+//   4 cameras of 979x546   300k rows 168 and 480 -> 144 and 430,
+//                          1M rows 330 and 825 -> 256 and 759
+//   2 of 1237x822          137 and 412 -> 126 and 387
+//   32 of 256x256          244 and 607 -> 168 and 418
+//   16 of 256x256 (split)  195 and 256 -> 143 and 256
+// The order is by the octave of the list's length relative to the mean (8 classes,
+// from 4 times it down), so that within a class neighbouring tiles still follow
+// each other (by length alone: the same).  One workgroup, every tile's class in
+// registers: a stable counting sort with three ballots per 64 tiles, about 6 us
+// (one ballot per class: 14).
+#define RASTER_ORDER_THREADS 1024
+#define RASTER_ORDER_ITEMS 16
+#define RASTER_ORDER_TILES (RASTER_ORDER_THREADS * RASTER_ORDER_ITEMS)
+
+__global__ void __launch_bounds__(RASTER_ORDER_THREADS) raster_order_kernel(
+    uint32_t n_tiles, uint32_t n_isects, const int32_t* __restrict__ tile_offsets,
+    int32_t* __restrict__ order) {
+  constexpr int WAVES = RASTER_ORDER_THREADS / 64, CLASSES = 8;
+  // tiles of class c in 64 tiles q (tile / 64): [c][q], then those before them
+  __shared__ uint32_t s_n[CLASSES * RASTER_ORDER_ITEMS * WAVES];
+  __shared__ uint32_t s_wave[WAVES];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t lt = (1ull << lane) - 1ull;
+  const int top = __clz((int)max(n_isects / n_tiles, 1u)) - 2;  // 4 times the mean
+  constexpr int PER = CLASSES * RASTER_ORDER_ITEMS * WAVES / RASTER_ORDER_THREADS;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) s_n[j * RASTER_ORDER_THREADS + threadIdx.x] = 0u;
+  uint32_t cls[RASTER_ORDER_ITEMS], rank[RASTER_ORDER_ITEMS];
+#pragma unroll
+  for (int k = 0; k < RASTER_ORDER_ITEMS; ++k) {
+    const uint32_t t = (uint32_t)k * RASTER_ORDER_THREADS + threadIdx.x;
+    cls[k] = CLASSES - 1;  // past the last tile: last of the last class
+    if (t < n_tiles) {
+      const int32_t end = t + 1 < n_tiles ? tile_offsets[t + 1] : (int32_t)n_isects;
+      cls[k] = (uint32_t)min(max(__clz(max(end - tile_offsets[t], 0)) - top, 0), CLASSES - 1);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < RASTER_ORDER_ITEMS; ++k) {
+    if ((uint32_t)k * RASTER_ORDER_THREADS >= n_tiles) break;
+    uint64_t peers = ~0ull;
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      const bool bit = (cls[k] >> b) & 1u;
+      const uint64_t m = tgs_ballot(bit);
+      peers &= bit ? m : ~m;
+    }
+    rank[k] = (uint32_t)__popcll(peers & lt);
+    if (rank[k] == 0u)
+      s_n[(cls[k] * RASTER_ORDER_ITEMS + k) * WAVES + wave] = (uint32_t)__popcll(peers);
+  }
+  __syncthreads();
+  uint32_t n[PER], sum = 0u;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    n[j] = s_n[threadIdx.x * PER + j];
+    sum += n[j];
+  }
+  const uint32_t inc = wave_incl_scan(sum);
+  if (lane == 63) s_wave[wave] = inc;
+  __syncthreads();
+  uint32_t at = inc - sum;
+  for (int w = 0; w < wave; ++w) at += s_wave[w];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    s_n[threadIdx.x * PER + j] = at;
+    at += n[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < RASTER_ORDER_ITEMS; ++k) {
+    const uint32_t t = (uint32_t)k * RASTER_ORDER_THREADS + threadIdx.x;
+    if (t < n_tiles)
+      order[s_n[(cls[k] * RASTER_ORDER_ITEMS + k) * WAVES + wave] + rank[k]] = (int32_t)t;
+  }
+}
+
+// The sizes ordered: more than one round of the forward's resident workgroups, up
+// to what one workgroup orders; cameras of up to 4096 tiles.  A camera of more ends
+// on its own short border lists, and the neighbours that the order parts cost
+// more: 1 camera of 1920x1080 124 and 401 -> 130 and 398 us, 2 of 1600x900 146 and
+// 500 -> 153 and 491, 2 of 1920x1080 232 and 757 -> 241 and 768.
+extern "C" uint64_t tgs_tide_raster_order_tiles(uint32_t C, uint32_t tile_width,
+                                                uint32_t tile_height, uint32_t n_isects) {
+  const uint64_t per_cam = (uint64_t)tile_width * tile_height, n = C * per_cam;
+  return n_isects && C > 1 && per_cam <= 4096 && n > 1536 && n <= RASTER_ORDER_TILES ? n : 0;
+}
+
+extern "C" int tgs_tide_raster_order(uint32_t C, uint32_t tile_width, uint32_t tile_height,
+                                     const int32_t* tile_offsets, uint32_t n_isects,
+                                     int32_t* order, hipStream_t stream) {
+  const uint64_t n = tgs_tide_raster_order_tiles(C, tile_width, tile_height, n_isects);
+  TGS_CHECK_ARG(n, "tide_raster_order: this size is not ordered");
+  TGS_CHECK_ARG(tile_offsets && order, "tide_raster_order: null");
+  hipLaunchKernelGGL(raster_order_kernel, dim3(1), dim3(RASTER_ORDER_THREADS), 0, stream,
+                     (uint32_t)n, n_isects, tile_offsets, order);
+  TGS_RETURN_LAUNCH("tgs_tide_raster_order");
+}
+
+extern "C" int tgs_tide_rasterize_fwd_ordered(uint32_t C, const float* splats, const float* backgrounds,
+                                              uint32_t W, uint32_t H, uint32_t tile_width,
+                                              uint32_t tile_height, const int32_t* tile_offsets,
+                                              const int32_t* flatten_ids, uint32_t n_isects,
+                                              float* images, float* alphas, int32_t* last_ids,
+                                              const int32_t* order, int32_t* n_contrib,
+                                              float* clear, uint64_t clear_words,
+                                              hipStream_t stream) {
   TGS_CHECK_ARG(clear_words % 4 == 0 && (clear_words == 0 || clear) &&
                     ((uintptr_t)clear & 15u) == 0,
                 "tide_rasterize_fwd: clear needs a 16-byte aligned buffer of 4k words");
@@ -1838,7 +1944,7 @@ extern "C" int tgs_tide_rasterize_fwd(uint32_t C, const float* splats, const flo
   TGS_CHECK_ARG(tile_width * 16 >= W && tile_height * 16 >= H, "tide_rasterize_fwd: tile grid");
   TGS_CHECK_ARG(C <= 65535 && tile_width <= 65535 && tile_height <= 65535,
                 "tide_rasterize_fwd: at most 65535 cameras and tiles per image side");
-  const RasterGeom G{C, W, H, tile_width, tile_height, n_isects};
+  const RasterGeom G{C, W, H, tile_width, tile_height, n_isects, order};
   if (n_contrib)
     hipLaunchKernelGGL((raster_fwd_kernel<3, 16, PackedSplats, true>), raster_fwd_grid(G),
                        dim3(256), 0, stream, G, PackedSplats{(const float4*)splats}, backgrounds,
@@ -1850,6 +1956,18 @@ extern "C" int tgs_tide_rasterize_fwd(uint32_t C, const float* splats, const flo
                        tile_offsets, flatten_ids, images, alphas, last_ids, (float4*)clear,
                        (uint64_t)clear_words / 4, nullptr);
   TGS_RETURN_LAUNCH("tgs_tide_rasterize_fwd");
+}
+
+extern "C" int tgs_tide_rasterize_fwd(uint32_t C, const float* splats, const float* backgrounds,
+                                      uint32_t W, uint32_t H, uint32_t tile_width,
+                                      uint32_t tile_height, const int32_t* tile_offsets,
+                                      const int32_t* flatten_ids, uint32_t n_isects,
+                                      float* images, float* alphas, int32_t* last_ids,
+                                      int32_t* n_contrib, float* clear, uint64_t clear_words,
+                                      hipStream_t stream) {
+  return tgs_tide_rasterize_fwd_ordered(C, splats, backgrounds, W, H, tile_width, tile_height,
+                                        tile_offsets, flatten_ids, n_isects, images, alphas,
+                                        last_ids, nullptr, n_contrib, clear, clear_words, stream);
 }
 
 // Segment size of a split rasterization (raster.cuh, RasterSplit) as a shift, 0
@@ -1896,8 +2014,8 @@ extern "C" int tgs_tide_rasterize_fwd_split(
     uint32_t C, const float* splats, const float* backgrounds, uint32_t W, uint32_t H,
     uint32_t tile_width, uint32_t tile_height, const int32_t* tile_offsets,
     const int32_t* flatten_ids, uint32_t n_isects, float* images, float* alphas,
-    int32_t* last_ids, float* clear, uint64_t clear_words, float* states, int32_t* item_tile,
-    hipStream_t stream) {
+    int32_t* last_ids, float* clear, uint64_t clear_words, const int32_t* order, float* states,
+    int32_t* item_tile, hipStream_t stream) {
   TGS_CHECK_ARG(clear_words % 4 == 0 && (clear_words == 0 || clear) &&
                     ((uintptr_t)clear & 15u) == 0,
                 "tide_rasterize_fwd: clear needs a 16-byte aligned buffer of 4k words");
@@ -1910,7 +2028,7 @@ extern "C" int tgs_tide_rasterize_fwd_split(
   RasterSplit sp;
   const int rc = raster_split_args(C, tile_width, tile_height, n_isects, states, item_tile, sp);
   if (rc) return rc;
-  const RasterGeom G{C, W, H, tile_width, tile_height, n_isects};
+  const RasterGeom G{C, W, H, tile_width, tile_height, n_isects, order};
   hipLaunchKernelGGL((raster_fwd_kernel<3, 16, PackedSplats, false, true>), raster_fwd_grid(G),
                      dim3(256), 0, stream, G, PackedSplats{(const float4*)splats}, backgrounds,
                      tile_offsets, flatten_ids, images, alphas, last_ids, (float4*)clear,
@@ -1941,13 +2059,14 @@ extern "C" int tgs_tide_rasterize_bwd_split(
   TGS_RETURN_LAUNCH("tgs_tide_rasterize_bwd_split");
 }
 
-extern "C" int tgs_tide_rasterize_bwd(uint32_t C, const float* splats, const float* backgrounds,
-                                      uint32_t W, uint32_t H, uint32_t tile_width,
-                                      uint32_t tile_height, const int32_t* tile_offsets,
-                                      const int32_t* flatten_ids, uint32_t n_isects,
-                                      const float* alphas, const int32_t* last_ids,
-                                      const float* v_images, const float* v_alphas,
-                                      float* splat_grads, hipStream_t stream) {
+extern "C" int tgs_tide_rasterize_bwd_ordered(uint32_t C, const float* splats, const float* backgrounds,
+                                              uint32_t W, uint32_t H, uint32_t tile_width,
+                                              uint32_t tile_height, const int32_t* tile_offsets,
+                                              const int32_t* flatten_ids, uint32_t n_isects,
+                                              const float* alphas, const int32_t* last_ids,
+                                              const float* v_images, const float* v_alphas,
+                                              float* splat_grads, const int32_t* order,
+                                              hipStream_t stream) {
   if (C == 0 || W == 0 || H == 0 || n_isects == 0) return TGS_OK;
   TGS_CHECK_ARG(splats && tile_offsets && flatten_ids && alphas && last_ids && v_images &&
                     splat_grads,
@@ -1955,12 +2074,24 @@ extern "C" int tgs_tide_rasterize_bwd(uint32_t C, const float* splats, const flo
   TGS_CHECK_ARG(tile_width * 16 >= W && tile_height * 16 >= H, "tide_rasterize_bwd: tile grid");
   TGS_CHECK_ARG(C <= 65535 && tile_width <= 65535 && tile_height <= 65535,
                 "tide_rasterize_bwd: at most 65535 cameras and tiles per image side");
-  const RasterGeom G{C, W, H, tile_width, tile_height, n_isects};
+  const RasterGeom G{C, W, H, tile_width, tile_height, n_isects, order};
   hipLaunchKernelGGL((raster_bwd_kernel<3, 16, PackedSplats, PackedGrads>), raster_bwd_grid(G),
                      dim3(256), 0, stream, G,
                      PackedSplats{(const float4*)splats}, PackedGrads{splat_grads}, backgrounds,
                      tile_offsets, flatten_ids, alphas, last_ids, v_images, v_alphas);
   TGS_RETURN_LAUNCH("tgs_tide_rasterize_bwd");
+}
+
+extern "C" int tgs_tide_rasterize_bwd(uint32_t C, const float* splats, const float* backgrounds,
+                                      uint32_t W, uint32_t H, uint32_t tile_width,
+                                      uint32_t tile_height, const int32_t* tile_offsets,
+                                      const int32_t* flatten_ids, uint32_t n_isects,
+                                      const float* alphas, const int32_t* last_ids,
+                                      const float* v_images, const float* v_alphas,
+                                      float* splat_grads, hipStream_t stream) {
+  return tgs_tide_rasterize_bwd_ordered(C, splats, backgrounds, W, H, tile_width, tile_height,
+                                        tile_offsets, flatten_ids, n_isects, alphas, last_ids,
+                                        v_images, v_alphas, splat_grads, nullptr, stream);
 }
 
 extern "C" int tgs_tide_project_bwd_update(

@@ -477,7 +477,7 @@ class _RasterizeToPixels(torch.autograd.Function):
         dev = means2d.device
         render_alphas = torch.empty((C, height, width, 1), dtype=torch.float32, device=dev)
         last_ids = torch.empty((C, height, width), dtype=torch.int32, device=dev)
-        records = states = item_tile = None
+        records = states = item_tile = order = None
         if ch == 3 and tile_size == 16 and not absgrad:
             render_colors = torch.empty((C, height, width, ch), dtype=torch.float32, device=dev)
             records = _packed_splats(means2d, conics, colors, opacities)
@@ -487,13 +487,20 @@ class _RasterizeToPixels(torch.autograd.Function):
             # few tiles: split the backward along the tiles' lists
             items = (N.load().tgs_tide_raster_split_items(C, tw, th, flatten_ids.numel())
                      if any(ctx.needs_input_grad[:4]) and C * width * height else 0)
+            # a few rounds of workgroups: the longest lists first
+            if C * width * height and N.load().tgs_tide_raster_order_tiles(
+                    C, tw, th, flatten_ids.numel()):
+                order = torch.empty(C * th * tw, dtype=torch.int32, device=dev)
+                N.call("tgs_tide_raster_order", C, tw, th, N.ptr(isect_offsets),
+                       flatten_ids.numel(), N.ptr(order), _stream())
             if items:
                 states = torch.empty((items, 1024), dtype=torch.float32, device=dev)
                 item_tile = torch.empty(items, dtype=torch.int32, device=dev)
-                N.call("tgs_tide_rasterize_fwd_split", *args, None, 0, N.ptr(states),
-                       N.ptr(item_tile), _stream())
+                N.call("tgs_tide_rasterize_fwd_split", *args, None, 0, N.ptr(order),
+                       N.ptr(states), N.ptr(item_tile), _stream())
             else:
-                N.call("tgs_tide_rasterize_fwd", *args, None, None, 0, _stream())
+                N.call("tgs_tide_rasterize_fwd_ordered", *args, N.ptr(order), None, None, 0,
+                       _stream())
         else:
             outs = []
             for s0, w, cw in _channel_chunks(ch):
@@ -518,7 +525,7 @@ class _RasterizeToPixels(torch.autograd.Function):
                                         torch.zeros((), dtype=torch.float32, device=dev))
         ctx.save_for_backward(means2d, conics, colors, opacities, backgrounds, isect_offsets,
                               flatten_ids, kernel_alphas, render_alphas, last_ids, records, pmask,
-                              states, item_tile)
+                              states, item_tile, order)
         ctx.width, ctx.height, ctx.tile_size, ctx.absgrad = width, height, tile_size, absgrad
         ctx.set_materialize_grads(False)
         return render_colors, render_alphas
@@ -526,8 +533,8 @@ class _RasterizeToPixels(torch.autograd.Function):
     @staticmethod
     def backward(ctx, v_render_colors, v_render_alphas):
         (means2d, conics, colors, opacities, backgrounds, isect_offsets, flatten_ids,
-         render_alphas, out_alphas, last_ids, records, pmask, states,
-         item_tile) = ctx.saved_tensors
+         render_alphas, out_alphas, last_ids, records, pmask, states, item_tile,
+         order) = ctx.saved_tensors
         C = isect_offsets.shape[0]
         th, tw = isect_offsets.shape[1], isect_offsets.shape[2]
         ch = colors.shape[-1]
@@ -556,7 +563,7 @@ class _RasterizeToPixels(torch.autograd.Function):
                 N.call("tgs_tide_rasterize_bwd_split", *args, N.ptr(states), N.ptr(item_tile),
                        _stream())
             else:
-                N.call("tgs_tide_rasterize_bwd", *args, _stream())
+                N.call("tgs_tide_rasterize_bwd_ordered", *args, N.ptr(order), _stream())
             N.call("tgs_unpack_splat_grads", n, N.ptr(grads), N.ptr(v_means2d), N.ptr(v_conics),
                    N.ptr(v_colors), N.ptr(v_opacities), _stream())
         else:

@@ -474,16 +474,22 @@ class TideStep:
         n_contrib = self._buf("n_contrib", C * H * W, torch.int32) if self._count_pairs else None
         # batches of few tiles split the backward along the tiles' lists
         items = 0 if self._count_pairs else lib.tgs_tide_raster_split_items(C, tw, th, n_isects)
+        # a few rounds of workgroups: the longest lists first
+        order = None
+        if lib.tgs_tide_raster_order_tiles(C, tw, th, n_isects):
+            order = self._buf("raster_order", n_buckets, torch.int32)
+            N.call("tgs_tide_raster_order", C, tw, th, N.ptr(offsets), n_isects, N.ptr(order), s)
         if items:
             states = self._buf("raster_states", items * 1024, torch.float32)
             item_tile = self._buf("raster_items", items, torch.int32)
             N.call("tgs_tide_rasterize_fwd_split", C, N.ptr(splats), N.ptr(bg), W, H, tw, th,
                    N.ptr(offsets), N.ptr(fids), n_isects, N.ptr(images), N.ptr(alphas),
-                   N.ptr(last_ids), N.ptr(sgrads), sg_words, N.ptr(states), N.ptr(item_tile), s)
+                   N.ptr(last_ids), N.ptr(sgrads), sg_words, N.ptr(order), N.ptr(states),
+                   N.ptr(item_tile), s)
         else:
-            N.call("tgs_tide_rasterize_fwd", C, N.ptr(splats), N.ptr(bg), W, H, tw, th,
+            N.call("tgs_tide_rasterize_fwd_ordered", C, N.ptr(splats), N.ptr(bg), W, H, tw, th,
                    N.ptr(offsets), N.ptr(fids), n_isects, N.ptr(images), N.ptr(alphas),
-                   N.ptr(last_ids), N.ptr(n_contrib), N.ptr(sgrads), sg_words, s)
+                   N.ptr(last_ids), N.ptr(order), N.ptr(n_contrib), N.ptr(sgrads), sg_words, s)
         self._end()
         sums = self._buf("loss_sums", 2 * C, torch.float64)
         v_images = self._buf("v_images", C * H * W * 3, torch.float32)
@@ -499,7 +505,7 @@ class TideStep:
         if items:
             N.call("tgs_tide_rasterize_bwd_split", *bwd_args, N.ptr(states), N.ptr(item_tile), s)
         else:
-            N.call("tgs_tide_rasterize_bwd", *bwd_args, s)
+            N.call("tgs_tide_rasterize_bwd_ordered", *bwd_args, N.ptr(order), s)
         self._end()
 
         # 5. per touched row: projection + SH + activation backward (and, with
