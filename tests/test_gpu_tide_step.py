@@ -513,3 +513,41 @@ def test_fused_emission_block_sizes(gpu, V, C, big):
     """The fused emission with 256- and with 1024-entry blocks: one entry, one
     past a block, and either side of the line between the two forms."""
     test_fused_emission_sort_matches_stable_tile_sort(gpu, V, C, big, 40, 30)
+
+
+@pytest.mark.parametrize("T", [1, 15, 17, (1 << 15) - 1, 1 << 15, (1 << 16) - 1, 1 << 16])
+def test_fused_update_rows_per_wavefront(gpu, T):
+    """The fused update of the first T touched rows, in wavefronts of 16, 32 and
+    64 rows, against the update of all of them: the same bits in those rows (a
+    row's update depends on nothing else), and every other row untouched."""
+    announce(f"fused update rows per wavefront T={T}")
+    from tidegs_amd import _native as N
+    sc = scenes.small(seed=8, n=80_000, n_cams=1, W=96, H=64, log_scale_mu=-4.0)
+    base = sc.params.to(gpu).contiguous()
+    ts = TideStep(base.clone(), sc.width, sc.height, batch_size=1, block_size=1000)
+    touched, _, _ = ts.forward_backward(sc.viewmats, sc.Ks, sc.gt)
+    L = ts.last
+    assert touched.numel() > 1 << 16
+    vm = sc.viewmats.to(gpu, torch.float32).contiguous()
+    Ks = sc.Ks.to(gpu, torch.float32).contiguous()
+    out = []
+    for n in (touched.numel(), T):
+        o = TideStep(base.clone(), sc.width, sc.height, batch_size=1, block_size=1000)
+        counts = o.optimizer.launch_touch_counts(o.gaussians, touched[:n])
+        torch.cuda.synchronize()
+        args, _ = o.optimizer.fused_update_args(1, o.gaussians, n, counts)
+        N.call("tgs_tide_project_bwd_update", n, N.ptr(touched), N.ptr(L["visit_base"]),
+               N.ptr(L["visits"]), N.ptr(L["masks"]), 1, N.ptr(o.params), o.row_stride, N.ptr(vm),
+               N.ptr(Ks), N.ptr(L["campos"]), sc.width, sc.height, o.eps2d, o.near, o.far, 0.0,
+               o.sh_degree, N.ptr(L["splat_grads"]), *args, N.stream_handle(gpu))
+        out.append((o.params, o.optimizer._exp_avg, o.optimizer._exp_avg_sq))
+    rows = touched[:T].long()
+    (pa, ma, va), (pb, mb, vb) = out
+    assert torch.equal(pa[rows], pb[rows]) and bool((pb[rows] != base[rows]).any())
+    rest = torch.ones(base.shape[0], dtype=torch.bool, device=gpu)
+    rest[rows] = False
+    assert torch.equal(pb[rest], base[rest])
+    for a, b in ((ma, mb), (va, vb)):  # slots of whole blocks: the touched rows' sums
+        assert int((b != 0).any(1).sum()) <= T
+        hit = (b != 0).any(1)
+        assert torch.equal(a[hit], b[hit])

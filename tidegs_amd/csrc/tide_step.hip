@@ -1260,21 +1260,20 @@ struct TideOptim {
 
 template <bool SOPHIA, bool POW2_BS>
 __global__ void __launch_bounds__(FUSED_THREADS) tide_project_bwd_optim_kernel(
-    uint32_t n_touched, const int32_t* __restrict__ touched,
+    uint32_t n_touched, uint32_t rows, const int32_t* __restrict__ touched,
     const int32_t* __restrict__ visit_base, const int32_t* __restrict__ visits,
     const uint32_t* __restrict__ masks, TideCams tc, float* __restrict__ params,
     uint32_t row_stride, int W, int H, float eps2d, float near_plane, float far_plane,
     float radius_clip, int sh_degree, const float* __restrict__ splat_grads, TideOptim O) {
   __shared__ CamLDS s_cam;
-  __shared__ float s_g[FUSED_THREADS / 64][64 * ROW_PITCH];
+  __shared__ float sg[64 * ROW_PITCH];
   load_cams_lds(tc, s_cam, W, H);
   const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t t0 = blockIdx.x * blockDim.x + (uint32_t)wv * 64u;  // the wavefront's first row
+  static_assert(FUSED_THREADS == 64, "one wavefront takes the workgroup's rows");
+  const uint32_t t0 = blockIdx.x * rows;  // the wavefront's first row
   const uint32_t t = t0 + (uint32_t)lane;
-  float* sg = s_g[wv];
   int32_t my_row = 0;
-  if (t < n_touched) {
+  if ((uint32_t)lane < rows && t < n_touched) {
     my_row = touched[t];
     tide_row_grads(t, my_row, visit_base, visits, masks, s_cam, tc.C, params, row_stride, W, H,
                    eps2d, near_plane, far_plane, radius_clip, sh_degree, splat_grads,
@@ -1284,7 +1283,7 @@ __global__ void __launch_bounds__(FUSED_THREADS) tide_project_bwd_optim_kernel(
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (t0 >= n_touched) return;
-  const int n_w = n_touched - t0 < 64u ? (int)(n_touched - t0) : 64;
+  const int n_w = (int)min(n_touched - t0, rows);
 
   const bool act = lane < TIDE_ROW;
   const int PW = (int)row_stride, SW = O.state_pitch;
@@ -2094,6 +2093,15 @@ extern "C" int tgs_tide_rasterize_bwd(uint32_t C, const float* splats, const flo
                                         v_images, v_alphas, splat_grads, nullptr, stream);
 }
 
+// Touched rows per wavefront of the fused update: a wavefront's second phase is a
+// chain over its rows, so few rows are spread over more wavefronts until those no
+// longer run at once.  With 64, 32 and 16 rows, in us: 10k rows 28, 20 and 17; 40k
+// 32, 25 and 28; 70k 37, 32 and 36; 100k of 4 cameras 50, 53 and 61; 500k 148, 150
+// and 188.
+static uint32_t fused_rows(uint32_t n_touched) {
+  return n_touched < (1u << 15) ? 16u : n_touched < (1u << 16) ? 32u : 64u;
+}
+
 extern "C" int tgs_tide_project_bwd_update(
     uint32_t n_touched, const int32_t* touched, const int32_t* visit_base, const int32_t* visits,
     const uint32_t* masks, uint32_t C, float* params, uint32_t row_stride, const float* viewmats,
@@ -2144,9 +2152,10 @@ extern "C" int tgs_tide_project_bwd_update(
   O.error_flag = error_flag;
 #define TIDE_FUSED_LAUNCH(SOPHIA, POW2)                                                          \
   hipLaunchKernelGGL((tide_project_bwd_optim_kernel<SOPHIA, POW2>),                              \
-                     dim3(tgs_blocks(n_touched, FUSED_THREADS)), dim3(FUSED_THREADS), 0, stream, \
-                     n_touched, touched, visit_base, visits, masks, tc, params, row_stride, W, H, \
+                     dim3(tgs_blocks(n_touched, rows)), dim3(FUSED_THREADS), 0, stream, n_touched, \
+                     rows, touched, visit_base, visits, masks, tc, params, row_stride, W, H, \
                      eps2d, near_plane, far_plane, radius_clip, sh_degree, splat_grads, O)
+  const uint32_t rows = fused_rows(n_touched);
   int bs_exp = 0;
   const bool pow2 = batch_size > 0.f && std::frexp(batch_size, &bs_exp) == 0.5f;
   if (optimizer == 1) {
