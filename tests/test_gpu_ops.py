@@ -247,6 +247,8 @@ def test_isect_tiles_paths_bit_exact(gpu, case):
     (1, 1, 1, 1, (2.0, 2.0)),             # one key without a bit to sort on
     (1, 255, 1, 1, (2.0, 2.0)), (1, 256, 7, 3, (2.0, 2.0)),  # no depth bits
     (2, 257, 7, 3, (0.0, 1.0)),           # ids of 2 cameras in 1 bit, depths from zero
+    (1, 4000, 1, 1, (2.0, 2.0)),          # two sorts without a bit, a single tile pass
+    (1, 2520, 5, 5, (0.2, 500.0)), (1, 2100, 5, 5, (0.2, 500.0)),  # about 2048 with any tile
     (3, 8191, 16, 16, (1.0, 2.0 - 2.0 ** -23)),  # 256 tiles: 9 bits, depths of one binade
     (1, 4 * 256 * 1024 + 1, 31, 17, (0.2, 500.0)),  # one block past a chunk of the sums' scan
     (2, 70_001, 255, 2, (0.2, 500.0)),    # the widest grid of the two sorts

@@ -485,6 +485,13 @@ static bool isect_sorted_layout(uint32_t C, const uint64_t* summary, uint32_t ti
   }
   o.V = o.ent[C];
   o.n = o.isect[C];
+  // Few Gaussians make few blocks of the fused emission, each a serial chain over
+  // its tiles, and a single sort of few keys is launches either way.  Two sorts and
+  // one, in us, by Gaussians and tiles of each: 300 of 4 99 and 95, of 62 170 and
+  // 106; 2000 of 16 99 and 113, of 61 196 and 138; 10k of 16 109 and 124, of 61 200
+  // and 169, of 233 386 and 269; 40k of 61 239 and 255, of 858 1493 and 1785; 100k
+  // of 61 290 and 454; 400k of 16 236 and 426, of 61 688 and 1572.
+  if (o.V < (1u << 15) && (o.V < 2048u || o.n > 32ull * o.V)) return false;
   o.hist_words = tgs_tide_isect_fused_hist_words(C, o.ent, o.tile_bits);
   if (o.hist_words == 0 || o.n != summary[0]) return false;
   o.sort_bytes = std::max(tgs_segmented_sort_workspace_size(o.V, C),
