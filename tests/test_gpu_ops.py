@@ -306,6 +306,28 @@ def test_isect_offset_encode_ragged(gpu, n, shift):
     np.testing.assert_array_equal(to_np(offs), R.isect_offset_encode(keys, C, tw, th))
 
 
+@pytest.mark.parametrize("C,tw,th", [(1, 5, 5), (1, 1, 1), (3, 7, 3), (2, 16, 16)])
+def test_isect_negative_depths(gpu, C, tw, th):
+    """A negative depth's sign fills the id's high word: ids, order and the bucket
+    the offsets count such an id in are the formula's (oracle), for all of one
+    sign and, ids only, for both signs."""
+    announce(f"isect negative depths C={C} {tw}x{th}")
+    rng = np.random.default_rng(C + tw)
+    n = 3001
+    m2d = rng.uniform(0, [tw * 16, th * 16], size=(C, n, 2)).astype(np.float32)
+    radii = rng.integers(0, 14, size=(C, n)).astype(np.int32)
+    for lo, hi in ((-50.0, -0.5), (-50.0, 50.0)):
+        depths = rng.uniform(lo, hi, size=(C, n)).astype(np.float32)
+        args = [torch.from_numpy(a).to(gpu) for a in (m2d, radii, depths)]
+        _, ids, flat = ops.isect_tiles(*args, 16, tw, th)
+        _, o_ids, o_flat = R.isect_tiles(m2d, radii, depths, 16, tw, th)
+        np.testing.assert_array_equal(to_np(ids), o_ids)
+        np.testing.assert_array_equal(to_np(flat), o_flat)
+        if hi < 0:
+            offs = ops.isect_offset_encode(ids, C, tw, th)
+            np.testing.assert_array_equal(to_np(offs), R.isect_offset_encode(o_ids, C, tw, th))
+
+
 def test_isect_tiles_packed_and_empty(gpu):
     announce("isect packed + empty")
     sc, radii, m2d, depths, _, _ = _projected(gpu, seed=4, C=2)

@@ -125,24 +125,27 @@ __global__ void __launch_bounds__(256) isect_emit_kernel(
 }
 
 // Offsets by search: bucket b = (camera, tile) gets the index of the first sorted
-// key whose high word is >= its own (camera << tile_n_bits | tile), i.e. an empty
-// bucket takes the next occupied one's start and buckets after the last key take
-// n_isects, as the reference's scatter from the run starts writes them.  One
-// thread per bucket, a branch-free binary search with a uniform trip count.  One
-// thread per key, writing the run of empty buckets before its own, took 9 us for
-// 2.7M keys of 4293 tiles and 31 us for 1.4M where one thread met a long run
-// (the empty rows above a scene): 6 us in both here.
+// key of its own or a later bucket, i.e. an empty bucket takes the next occupied
+// one's start and buckets after the last key take n_isects, as the reference's
+// scatter from the run starts writes them.  A key's bucket is computed from its
+// signed high word as there: a negative depth's sign fills the word, and such a
+// key counts where the formula puts it, not past the last bucket.  One thread per
+// bucket, a branch-free binary search with a uniform trip count.  One thread per
+// key, writing the run of empty buckets before its own, took 9 us for 2.7M keys of
+// 4293 tiles and 31 us for 1.4M where one thread met a long run (the empty rows
+// above a scene): 6 us in both here.
 __global__ void __launch_bounds__(256) isect_offset_search_kernel(
-    uint64_t n_isects, const uint64_t* __restrict__ isect_ids, uint64_t n_buckets, uint32_t n_tiles,
+    uint64_t n_isects, const int64_t* __restrict__ isect_ids, uint64_t n_buckets, uint32_t n_tiles,
     uint32_t tile_n_bits, uint64_t top, int32_t* __restrict__ offsets) {
   const uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= n_buckets) return;
-  const uint64_t cam = b / n_tiles;
-  const uint64_t kb = (cam << tile_n_bits) | (b - cam * n_tiles);
+  const int64_t tmask = ((int64_t)1 << tile_n_bits) - 1;
   uint64_t pos = 0;  // keys [0, pos) lie in buckets before b
   for (uint64_t step = top; step != 0u; step >>= 1) {
     const uint64_t p = pos + step;
-    if (p <= n_isects && (isect_ids[p - 1] >> 32) < kb) pos = p;
+    if (p > n_isects) continue;
+    const int64_t hi = isect_ids[p - 1] >> 32;
+    if ((hi >> tile_n_bits) * n_tiles + (hi & tmask) < (int64_t)b) pos = p;
   }
   offsets[b] = (int32_t)pos;
 }
@@ -633,7 +636,7 @@ extern "C" int tgs_isect_offset_encode(uint64_t n_isects, const int64_t* isect_i
   uint64_t top = 1;
   while (top <= n_isects / 2) top <<= 1;
   hipLaunchKernelGGL(isect_offset_search_kernel, dim3(tgs_blocks(total, 256)), dim3(256), 0, stream,
-                     n_isects, (const uint64_t*)isect_ids, total, n_tiles, tile_n_bits, top,
+                     n_isects, isect_ids, total, n_tiles, tile_n_bits, top,
                      offsets);
   TGS_RETURN_LAUNCH("tgs_isect_offset_encode");
 }
