@@ -72,6 +72,39 @@ def test_projection_fwd_bwd(gpu, calc_comp):
     assert rel_l2(to_np(dv.grad)[:, :3], to_np(v_vm)[:, :3]) < 1e-4
 
 
+class _NoGradient(torch.autograd.Function):
+    """A consumer that passes no gradient back (None, not zeros)."""
+
+    @staticmethod
+    def forward(ctx, *ts):
+        return sum(t.sum() for t in ts)
+
+    @staticmethod
+    def backward(ctx, g):
+        return (None,) * 3
+
+
+@pytest.mark.parametrize("used", [(), (0,), (1,), (2,), (0, 2)])
+def test_projection_missing_cotangents(gpu, used):
+    """Outputs that no gradient reaches count as zeros: the leaves get tensors
+    (zeros where nothing reaches any output), equal to those under explicit zeros."""
+    announce(f"projection cotangents of outputs {used}")
+    sc, means, quats, scales = _proj_inputs(n=500)
+    leaves = [t.to(gpu).requires_grad_() for t in (means, quats, scales)]
+    radii, m2d, depths, conics, _ = ops.fully_fused_projection(
+        leaves[0], None, *leaves[1:], sc.viewmats.to(gpu), sc.Ks.to(gpu), sc.width, sc.height)
+    outs = (m2d, depths, conics)
+    g = torch.Generator().manual_seed(2)
+    v = [torch.randn(o.shape, generator=g).to(gpu) * (radii > 0).view(*radii.shape, *[1] * (o.dim() - 2))
+         if i in used else torch.zeros_like(o) for i, o in enumerate(outs)]
+    ref = torch.autograd.grad(outs, leaves, v, retain_graph=True)
+    loss = _NoGradient.apply(*outs) if not used else sum((outs[i] * v[i]).sum() for i in used)
+    got = torch.autograd.grad(loss, leaves)
+    for a, b in zip(got, ref):
+        np.testing.assert_array_equal(to_np(a), to_np(b))
+    assert bool(got[0].abs().sum() > 0) == bool(used)  # every output depends on the means
+
+
 @pytest.mark.parametrize("calc_comp,sparse", [(False, False), (True, False), (False, True)])
 def test_projection_packed(gpu, calc_comp, sparse):
     """fully_fused_projection(packed=True): entries camera-major and Gaussian-

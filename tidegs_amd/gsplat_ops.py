@@ -97,9 +97,6 @@ class _FullyFusedProjection(torch.autograd.Function):
         means, covars, quats, scales, viewmats, Ks, radii, conics, comps = ctx.saved_tensors
         C, Nn = viewmats.shape[0], means.shape[0]
 
-        if v_means2d is None and v_depths is None and v_conics is None and v_comps is None:
-            return (None,) * 13
-
         def _c(t, shape):
             return torch.zeros(shape, dtype=torch.float32, device=means.device) if t is None \
                 else t.contiguous()
