@@ -103,3 +103,21 @@ def test_hist0_sort_refuses_offset_first_pass():
     rc = lib.tgs_segmented_sort_pairs_u32_hist0(None, None, None, None, 16, 1, segs, 1, 13,
                                                 None, 0, ctypes.byref(sel), None)
     assert rc != 0 and "bit 0" in N.last_error()
+
+
+def test_stream_handle_refuses_other_devices():
+    """A host device has no stream: a launch asking for one would hand host
+    addresses to a kernel, so it is refused before any GPU is looked for."""
+    import torch
+    from tidegs_amd import _native as N
+    for device in ("cpu", torch.device("cpu"), "meta"):
+        with pytest.raises(ValueError, match="Expected a cuda device"):
+            N.stream_handle(device)
+
+
+def test_resident_optimizer_on_the_host_refused():
+    """An optimizer built for the host raises where its first launch would be."""
+    from tidegs_amd.resident_optim import GPUResidentAdam
+    opt = GPUResidentAdam(block_size=4, device="cpu")
+    with pytest.raises(ValueError, match="Expected a cuda device"):
+        opt.set_resident_blocks([0, 1])

@@ -271,9 +271,13 @@ def ptr(t) -> int | None:
 
 def stream_handle(device=None) -> int:
     """The current stream's raw handle (without building a torch stream object:
-    every launch asks for it)."""
+    every launch asks for it).  Only of a GPU: the launch that asks would hand
+    a host tensor's address to a kernel."""
     if device is not None and not isinstance(device, int):
-        device = torch.device(device).index
+        device = torch.device(device)
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        device = device.index
     if device is None:
         device = torch.cuda.current_device()
     return torch._C._cuda_getCurrentRawStream(device)
