@@ -205,7 +205,7 @@ int tgs_segmented_sort_pairs_u32_range(uint32_t* keys, void* vals, uint32_t* key
                                        tgs_stream_t stream);
 /* Counts, offsets and depth range without a scan of every Gaussian's count, for C
  * cameras of N Gaussians (packed: one of nnz).  The plan (tgs_isect_tiles_plan_size
- * bytes) holds one record per 256 Gaussians.  summary [2 + 2 C] = {intersections,
+ * bytes, no fewer than for any smaller C, N) holds one record per 256 Gaussians.  summary [2 + 2 C] = {intersections,
  * kmin | kmax << 32} with the least and greatest depth bits (unsigned; 0xffffffff, 0
  * where none) of the Gaussians that meet a tile, then per camera {such Gaussians,
  * intersections} up to its end.  tgs_isect_tiles_emit_plan writes what
@@ -285,7 +285,7 @@ int tgs_fused_ssim_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1, fl
 /* Mean SSIM without the map (clm_kernels/__init__.py:23-61's fused_ssim):
  * mean = mean of the map over [crop, H - crop) x [crop, W - crop).  img1 is
  * NCHW, or NHWC with channels_last; img2 NCHW.  partials: scratch of
- * tgs_fused_ssim_mean_partials doubles.  img1_copy (optional): img1 in NCHW, for
+ * tgs_fused_ssim_mean_partials doubles (no fewer than any smaller B, CH, H, W take).  img1_copy (optional): img1 in NCHW, for
  * the backward.  The partial maps (NCHW) are all set or all null. */
 uint64_t tgs_fused_ssim_mean_partials(int32_t B, int32_t CH, int32_t H, int32_t W);
 int tgs_fused_ssim_mean_fwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1, float C2,
@@ -310,7 +310,8 @@ int tgs_tide_loss(int32_t B, int32_t H, int32_t W, const float* images_hwc, cons
                   float gt_div, float lambda_dssim, double* sums, float* v_images_hwc,
                   tgs_stream_t stream);
 /* The same, with sums written instead of added to (no clear needed): partials is
- * scratch of tgs_tide_loss_partials doubles, added up in a fixed order. */
+ * scratch of tgs_tide_loss_partials doubles (no fewer than any smaller B, H, W
+ * take), added up in a fixed order. */
 uint64_t tgs_tide_loss_partials(int32_t B, int32_t H, int32_t W);
 int tgs_tide_loss_summed(int32_t B, int32_t H, int32_t W, const float* images_hwc,
                          const float* gt_chw, float gt_div, float lambda_dssim, double* partials,
@@ -600,7 +601,9 @@ int tgs_tide_rasterize_bwd_ordered(uint32_t C, const float* splats, const float*
  * segment of a list, and the backward runs one workgroup per (tile, segment).
  * tgs_tide_raster_split_items: the items of this size (0: not split, use the
  * calls above).  states: 1024 floats per item, 16-byte aligned; item_tile: one
- * int32 per item; neither needs clearing.  Both calls take the same sizes. */
+ * int32 per item; neither needs clearing.  Both calls take the same sizes.  The
+ * items are no fewer than those of any fewer intersections or tiles, so buffers
+ * sized for the largest batch that is split hold the smaller ones. */
 uint64_t tgs_tide_raster_split_items(uint32_t C, uint32_t tile_width, uint32_t tile_height,
                                      uint32_t n_isects);
 int tgs_tide_rasterize_fwd_split(uint32_t C, const float* splats, const float* backgrounds,

@@ -128,3 +128,40 @@ def test_fused_update_argument_checks_without_a_gpu():
     assert call(5, optimizer=1, bias=None, row_stride=65) == -1  # Sophia needs no bias tables
     assert "row_stride" in _native.last_error()
     assert call(5, block_size=1 << 23) == -1 and "block_size" in _native.last_error()
+
+
+def _never_smaller(query, sizes, what):
+    """A buffer sized by ``query`` for one size holds every size before it."""
+    got = [query(*s) for s in sizes]
+    for (a, x), (b, y) in zip(zip(sizes, got), zip(sizes[1:], got[1:])):
+        assert x <= y, f"{what}: {a} takes {x}, {b} only {y}"
+
+
+def test_scratch_sizes_never_shrink_with_the_problem():
+    """The calls that take no buffer length rely on it: a caller that sizes its
+    scratch once, for its largest problem, reuses it for every smaller one."""
+    from tidegs_amd import _native
+
+    lib = _native.load()
+    near = sorted({max(1, (1 << k) + d) for k in range(28) for d in (-1, 0, 1, 63)})
+    for tiles in ((16, 16), (64, 64), (96, 64), (1, 1)):
+        _never_smaller(lambda n: lib.tgs_tide_raster_split_items(1, *tiles, n), [(n,) for n in near],
+                       f"split items of {tiles} tiles")
+    assert lib.tgs_tide_raster_split_items(1, 16, 16, 300_000) >= 256 + (262_207 >> 6)
+    dims = sorted({1, 5, 10, 11, 12, 13, 22, 44, 45, 54, 55, 78, 79, 123, 124, 546, 979, 1080, 1920,
+                   4096, *range(14, 120, 7)})
+    counts = sorted({1, 2, 3, 4, 5, 6, 7, 16, 17, 48, 64, 255, 256, 257, 4096})
+    for a in (1, 3, 16):
+        for d in (1, 60, 546, 1920):
+            for query, what in ((lambda b, h, w: lib.tgs_tide_loss_partials(b, h, w), "loss"),
+                                (lambda b, h, w: lib.tgs_fused_ssim_mean_partials(b, 3, h, w), "ssim"),
+                                (lambda b, h, w: lib.tgs_fused_ssim_mean_partials(a, b, h, w),
+                                 "ssim channels")):
+                _never_smaller(query, [(a, h, d) for h in dims], f"{what} partials by height")
+                _never_smaller(query, [(a, d, w) for w in dims], f"{what} partials by width")
+                _never_smaller(query, [(b, d, 979) for b in counts], f"{what} partials by images")
+    for n in (1, 10, 255, 256, 257, 100_000):
+        _never_smaller(lib.tgs_isect_tiles_plan_size, [(c, n) for c in range(1, 70)], "plan by cameras")
+    for c in (1, 32, 33, 100):
+        _never_smaller(lib.tgs_isect_tiles_plan_size, [(c, n) for n in near if n < 1 << 24],
+                       "plan by Gaussians")

@@ -839,6 +839,63 @@ def test_tide_loss_bands(gpu, B, H, W):
     test_tide_loss_kernel(gpu, B, H, W)
 
 
+def _guarded(n, dtype, gpu):
+    """n values with a sentinel behind them: (buffer, check that it is untouched)."""
+    pad = 4096
+    t = torch.full((n + pad,), 7, dtype=dtype, device=gpu)
+    return t[:n], lambda: bool((t[n:] == 7).all())
+
+
+@pytest.mark.parametrize("B,CH,H,W", [(1, 1, 1, 1), (1, 3, 12, 44), (1, 3, 300, 200), (40, 3, 20, 50),
+                                      (1, 4, 546, 979), (9, 3, 200, 300)])
+def test_scratch_queries_cover_the_launch(gpu, B, CH, H, W):
+    """The buffers of exactly the queried sizes hold what the launches write."""
+    from tidegs_amd import _native as N
+    announce(f"scratch queries {B}x{CH}x{H}x{W}")
+    lib, s = N.load(), N.stream_handle(gpu)
+    a, b = torch.rand((2, B, CH, H, W), device=gpu)
+    part, whole = _guarded(lib.tgs_fused_ssim_mean_partials(B, CH, H, W), torch.float64, gpu)
+    mean = torch.empty((), device=gpu)
+    N.call("tgs_fused_ssim_mean_fwd", B, CH, H, W, 1e-4, 9e-4, N.ptr(a), 0, N.ptr(b), 0, N.ptr(part),
+           N.ptr(mean), None, None, None, None, s)
+    assert whole() and abs(float(mean) - float(fused_ssim(a, b))) < 1e-6
+    if CH == 3:
+        part, whole = _guarded(lib.tgs_tide_loss_partials(B, H, W), torch.float64, gpu)
+        sums = torch.full((2 * B,), float("nan"), dtype=torch.float64, device=gpu)
+        v = torch.empty((B, H, W, 3), device=gpu)
+        img = a.permute(0, 2, 3, 1).contiguous()
+        N.call("tgs_tide_loss_summed", B, H, W, N.ptr(img), N.ptr(b), 1.0, 0.2, N.ptr(part),
+               N.ptr(sums), N.ptr(v), s)
+        assert whole()
+        l1 = (a - b).abs().double().sum((1, 2, 3))
+        assert torch.allclose(sums.view(B, 2)[:, 0], l1, rtol=1e-5)
+
+
+@pytest.mark.parametrize("n", [1, 63, 1000, 1100, 2100])
+def test_split_buffers_of_a_larger_batch(gpu, n):
+    """States and items sized once, for 600k intersections of 256 tiles, hold the
+    split raster's smaller batches too."""
+    from tidegs_amd import _native as N
+    announce(f"split buffers of a larger batch n={n}")
+    lib, s = N.load(), N.stream_handle(gpu)
+    items = lib.tgs_tide_raster_split_items(1, 16, 16, 600_000)
+    states, states_whole = _guarded(items * 1024, torch.float32, gpu)
+    item_tile, items_whole = _guarded(items, torch.int32, gpu)
+    tensors = _dense_tiles(gpu, n, 16, 16, n)
+    offs, flat = tensors[4:]
+    need = lib.tgs_tide_raster_split_items(1, 16, 16, flat.numel())
+    assert 0 < need <= items  # else the launch below would write past them
+    img, alpha = ops.rasterize_to_pixels(*tensors[:4], 256, 256, 16, offs, flat)
+    out, out_a = torch.empty_like(img), torch.empty_like(alpha)
+    last = torch.empty((1, 256, 256), dtype=torch.int32, device=gpu)
+    rec = ops._packed_splats(*tensors[:4])
+    N.call("tgs_tide_rasterize_fwd_split", 1, N.ptr(rec), None, 256, 256, 16, 16, N.ptr(offs),
+           N.ptr(flat), flat.numel(), N.ptr(out), N.ptr(out_a), N.ptr(last), None, 0, None,
+           N.ptr(states), N.ptr(item_tile), s)
+    assert states_whole() and items_whole()
+    np.testing.assert_array_equal(to_np(out), to_np(img))
+
+
 def _dense_tiles(gpu, n, tw, th, seed, opacity=(0.02, 0.9)):
     """n Gaussians in every tile of a tw x th image, in list order: (means2d,
     conics, colors, opacities, offsets, flatten ids), [1, N] splats."""

@@ -359,9 +359,12 @@ static int isect_plan_check(const char* who, uint32_t C, uint64_t N) {
   return TGS_OK;
 }
 
+// No less than for fewer cameras or Gaussians (up to IB_MAX_CAMS cameras each end on
+// a block of their own).
 extern "C" uint64_t tgs_isect_tiles_plan_size(uint32_t C, uint64_t N) {
   const IsectGrid g = isect_grid(C, N);
-  return (uint64_t)g.cams * g.per_cam * sizeof(IsectBlock);
+  const uint64_t own = (uint64_t)std::min(C, (uint32_t)IB_MAX_CAMS) * tgs_blocks(N, IB_ENTRIES);
+  return std::max((uint64_t)g.cams * g.per_cam, own) * sizeof(IsectBlock);
 }
 
 extern "C" int tgs_isect_tiles_plan(uint32_t C, uint64_t N, const float* means2d,

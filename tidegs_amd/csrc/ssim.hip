@@ -16,6 +16,8 @@
 // strategies/base_engine.py:472-488.
 #include "tgs_common.cuh"
 
+#include <algorithm>
+
 #define SS_R 5  // window radius
 
 // Normalised Gaussian window, w_i = exp(-(i-5)^2 / 4.5) / sum_j exp(-(j-5)^2 / 4.5).
@@ -89,6 +91,19 @@ static int band_input_rows(int H, int64_t strips_planes, int halo, float lone, i
     }
   }
   return best;
+}
+
+// Most workgroups that band_input_rows can lead to, for planes and sizes up to
+// these: every row a band of its own at the least rows, or what the cost allows (no
+// more than the longest bands', whose cost the choice never exceeds).
+static int64_t band_workgroups_max(int H, int64_t strips_planes, int halo, float lone,
+                                   int max_periods) {
+  const int least = (halo + LR_RING) / LR_RING * LR_RING, longest = max_periods * LR_RING;
+  const int64_t by_rows = strips_planes * ((H + least - halo - 1) / (least - halo));
+  const int64_t wgs = strips_planes * ((H + longest - halo - 1) / (longest - halo));
+  const double per_cu = std::max((double)((wgs + 255) / 256), (double)lone);
+  // (the slack and the 1: the costs are compared in float)
+  return std::min(by_rows, 256 * ((int64_t)(longest * per_cu / least * (1 + 1e-6)) + 1));
 }
 
 struct Plane {
@@ -330,12 +345,14 @@ struct SsimGrid {
 // three times a busy CU's.  Bands of more than 78 rows gain nothing (sixteen
 // 1080p images, 45-, 78- and 133-row bands: forward 780, 758, 766 us, backward
 // 664, 633, 734); one 256x256 image in 12-, 23- and 78-row bands: 15, 20, 49 us.
+#define SSIM_LONE 3.f
+#define SSIM_PERIODS 8
 static SsimGrid ssim_grid(int64_t B, int64_t CH, int H, int W) {
   const int nw = CH % 3 == 0 ? 3 : 1;
   const int64_t planes = B * (CH / nw);
   const int strips = (W + SR_OUT - 1) / SR_OUT;
   SsimGrid g;
-  g.rows = band_input_rows(H, planes * strips, 2 * SS_R, 3.f, 8);
+  g.rows = band_input_rows(H, planes * strips, 2 * SS_R, SSIM_LONE, SSIM_PERIODS);
   const int band = g.rows - 2 * SS_R;
   g.grid = dim3((unsigned)(planes * strips), (H + band - 1) / band);
   g.block = dim3(64 * nw);
@@ -381,10 +398,16 @@ extern "C" int tgs_fused_ssim_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, f
   TGS_RETURN_LAUNCH("tgs_fused_ssim_bwd");
 }
 
+// One sum per wavefront of the launch; the buffer's size is no less than any
+// smaller image's or batch's (of whatever channel count), so that one sized for the
+// largest holds them all.
 extern "C" uint64_t tgs_fused_ssim_mean_partials(int32_t B, int32_t CH, int32_t H, int32_t W) {
-  if ((int64_t)B * CH * H * W == 0) return 0;
-  const SsimGrid g = ssim_grid(B, CH, H, W);
-  return (uint64_t)g.grid.x * g.grid.y * (g.block.x / 64);
+  if (B <= 0 || CH <= 0 || H <= 0 || W <= 0) return 0;
+  const int64_t planes = (int64_t)B * CH, strips = (W + SR_OUT - 1) / SR_OUT;
+  const auto most = [&](int64_t n) {
+    return band_workgroups_max(H, n * strips, 2 * SS_R, SSIM_LONE, SSIM_PERIODS);
+  };
+  return (uint64_t)std::max(most(planes), 3 * most((planes + 2) / 3));
 }
 
 extern "C" int tgs_fused_ssim_mean_fwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1,
@@ -406,7 +429,7 @@ extern "C" int tgs_fused_ssim_mean_fwd(int32_t B, int32_t CH, int32_t H, int32_t
   TGS_LAUNCH_CHECK("tgs_fused_ssim_mean_fwd");
   const double count = (double)B * CH * (H - 2 * crop) * (W - 2 * crop);
   hipLaunchKernelGGL(ssim_mean_kernel, dim3(1), dim3(256), 0, stream, partials,
-                     (int64_t)tgs_fused_ssim_mean_partials(B, CH, H, W), count, mean);
+                     (int64_t)g.grid.x * g.grid.y * (g.block.x / 64), count, mean);
   TGS_RETURN_LAUNCH("tgs_fused_ssim_mean_fwd");
 }
 
@@ -678,10 +701,12 @@ struct LossGrid {
 // before, left small batches to a few long-running wavefronts: one 256x256 image
 // 102 -> 25 us, four 979x546 132 -> 91, one 1080p 126 -> 94; sixteen 1080p images
 // keep the 123 rows (1.10 ms; in 13-row bands 1.86).
+#define LOSS_LONE 2.4f
+#define LOSS_PERIODS 13
 static LossGrid loss_grid(int B, int H, int W) {
   LossGrid g;
   const int strips = (W + LR_OUT - 1) / LR_OUT;
-  g.rows = band_input_rows(H, (int64_t)strips * B, 4 * SS_R, 2.4f, 13);
+  g.rows = band_input_rows(H, (int64_t)strips * B, 4 * SS_R, LOSS_LONE, LOSS_PERIODS);
   const int band = g.rows - 4 * SS_R;
   g.grid = dim3(strips, (H + band - 1) / band, B);
   return g;
@@ -718,10 +743,12 @@ extern "C" int tgs_tide_loss(int32_t B, int32_t H, int32_t W, const float* image
 // in `partials` and a small launch adds them in a fixed order.  The atomics of
 // the other form queue on one image's two addresses (one 979x546 image in 33-row
 // bands: 966 workgroups, 95 us with one atomic per wavefront).
+// (Two sums per workgroup; the buffer's size is no less than any smaller image's or
+// batch's.)
 extern "C" uint64_t tgs_tide_loss_partials(int32_t B, int32_t H, int32_t W) {
-  if ((int64_t)B * H * W == 0) return 0;
-  const LossGrid g = loss_grid(B, H, W);
-  return 2ull * g.grid.x * g.grid.y * g.grid.z;
+  if (B <= 0 || H <= 0 || W <= 0) return 0;
+  return 2ull * (uint64_t)band_workgroups_max(H, (int64_t)((W + LR_OUT - 1) / LR_OUT) * B, 4 * SS_R,
+                                              LOSS_LONE, LOSS_PERIODS);
 }
 
 extern "C" int tgs_tide_loss_summed(int32_t B, int32_t H, int32_t W, const float* images_hwc,

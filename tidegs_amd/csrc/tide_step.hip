@@ -1988,11 +1988,16 @@ static uint32_t raster_split_shift(uint64_t n_tiles, uint64_t n_isects) {
   return shift;
 }
 
+// The launch's items are n_tiles + (n_isects >> shift); the buffers' are the most
+// that any fewer intersections take as well (shorter segments: up to 4096 of them),
+// so that buffers sized for the largest batch hold every smaller one.
 extern "C" uint64_t tgs_tide_raster_split_items(uint32_t C, uint32_t tile_width,
                                                 uint32_t tile_height, uint32_t n_isects) {
   const uint64_t n_tiles = (uint64_t)C * tile_width * tile_height;
   const uint32_t shift = raster_split_shift(n_tiles, n_isects);
-  return shift ? n_tiles + (n_isects >> shift) : 0;
+  if (!shift) return 0;
+  const uint32_t shortest = n_isects >> 6 < 4096u ? n_isects >> 6 : 4096u;
+  return n_tiles + (n_isects >> shift > shortest ? n_isects >> shift : shortest);
 }
 
 static int raster_split_args(uint32_t C, uint32_t tile_width, uint32_t tile_height,
@@ -2002,8 +2007,8 @@ static int raster_split_args(uint32_t C, uint32_t tile_width, uint32_t tile_heig
   sp.states = (float4*)states;
   sp.item_tile = item_tile;
   sp.shift = raster_split_shift(n_tiles, n_isects);
-  sp.items = (uint32_t)tgs_tide_raster_split_items(C, tile_width, tile_height, n_isects);
   TGS_CHECK_ARG(sp.shift, "tide_rasterize_split: this size is not split");
+  sp.items = (uint32_t)(n_tiles + (n_isects >> sp.shift));
   TGS_CHECK_ARG(states && item_tile && ((uintptr_t)states & 15u) == 0,
                 "tide_rasterize_split: states (16-byte aligned) and item_tile are needed");
   return TGS_OK;
