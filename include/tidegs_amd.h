@@ -152,7 +152,8 @@ int tgs_isect_tiles_emit(uint64_t total, uint32_t N, const int64_t* camera_ids,
                          int64_t* isect_ids, int32_t* flatten_ids, tgs_stream_t stream);
 /* cub::DeviceRadixSort::SortPairs replacement (isect_tiles.cu:189-227): stable
  * ascending sort on key bits [begin_bit, end_bit); double-buffered, *selector
- * (host int) = 0 if the result is in keys/vals, 1 if in keys_alt/vals_alt. */
+ * (host int) = 0 if the result is in keys/vals, 1 if in keys_alt/vals_alt.  A
+ * workspace sized for n keys serves every sort of fewer. */
 size_t tgs_radix_sort_workspace_size(uint64_t n);
 int tgs_radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
                          uint64_t n, int begin_bit, int end_bit, void* workspace,
@@ -173,7 +174,8 @@ int tgs_radix_sort_pairs_noalloc(uint64_t* keys, uint32_t* vals, uint64_t* keys_
  * segment [seg_offsets[s], seg_offsets[s+1]) is sorted on key bits
  * [begin_bit, end_bit) on its own.  seg_offsets is a HOST array of
  * n_segments+1 (<= 65) non-decreasing offsets from 0 to n.  Double-buffered
- * like tgs_radix_sort_pairs. */
+ * like tgs_radix_sort_pairs, with a workspace that serves fewer keys and segments
+ * too. */
 size_t tgs_segmented_sort_workspace_size(uint64_t n, uint32_t n_segments);
 /* Beside the reference's interface: tgs_segmented_sort_pairs_u32 with 4-byte
  * values whose first pass's per-tile digit counts are already at the start of

@@ -138,8 +138,8 @@ def _never_smaller(query, sizes, what):
 
 
 def test_scratch_sizes_never_shrink_with_the_problem():
-    """The calls that take no buffer length rely on it: a caller that sizes its
-    scratch once, for its largest problem, reuses it for every smaller one."""
+    """A caller that sizes its scratch once, for its largest problem, reuses it for
+    every smaller one; the calls that take no buffer length cannot even tell."""
     from tidegs_amd import _native
 
     lib = _native.load()
@@ -148,6 +148,14 @@ def test_scratch_sizes_never_shrink_with_the_problem():
         _never_smaller(lambda n: lib.tgs_tide_raster_split_items(1, *tiles, n), [(n,) for n in near],
                        f"split items of {tiles} tiles")
     assert lib.tgs_tide_raster_split_items(1, 16, 16, 300_000) >= 256 + (262_207 >> 6)
+    keys = sorted({*near, (3 << 19) - 1, 3 << 19, 1_500_000, 1_600_000})
+    _never_smaller(lib.tgs_radix_sort_workspace_size, [(n,) for n in keys], "sort workspace")
+    for segments in (1, 16, 64):
+        _never_smaller(lib.tgs_segmented_sort_workspace_size, [(n, segments) for n in keys],
+                       "segmented sort workspace by keys")
+    for n in (1, 1 << 20, (3 << 19) - 1, 3 << 19, 10_000_000):
+        _never_smaller(lib.tgs_segmented_sort_workspace_size, [(n, k) for k in range(1, 65)],
+                       "segmented sort workspace by segments")
     dims = sorted({1, 5, 10, 11, 12, 13, 22, 44, 45, 54, 55, 78, 79, 123, 124, 546, 979, 1080, 1920,
                    4096, *range(14, 120, 7)})
     counts = sorted({1, 2, 3, 4, 5, 6, 7, 16, 17, 48, 64, 255, 256, 257, 4096})

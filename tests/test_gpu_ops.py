@@ -441,6 +441,30 @@ def test_segmented_sort_size_rules(gpu, segs, vbytes):
     np.testing.assert_array_equal(to_np(rk).view(np.uint32), keys[order])
 
 
+@pytest.mark.parametrize("bits,n", [(64, (1 << 20) - 1), (64, 300_000), (32, (3 << 19) - 1), (32, 70_000)])
+def test_sort_workspace_of_a_larger_sort(gpu, bits, n):
+    """A workspace sized at the first size of whole tiles sorts fewer keys too."""
+    import ctypes
+    from tidegs_amd import _native as N
+    announce(f"workspace of a larger sort {bits} bits n={n}")
+    lib, s, sel = N.load(), N.stream_handle(gpu), ctypes.c_int(0)
+    keys = np.random.default_rng(n).integers(0, 2 ** 19, size=n)
+    k = torch.from_numpy(keys.astype(np.int64 if bits == 64 else np.int32)).to(gpu)
+    v = torch.arange(n, dtype=torch.int32, device=gpu)
+    k2, v2 = torch.empty_like(k), torch.empty_like(v)
+    if bits == 64:
+        size = lib.tgs_radix_sort_workspace_size(1 << 20)
+        ws = torch.empty(size, dtype=torch.uint8, device=gpu)
+        N.call("tgs_radix_sort_pairs", N.ptr(k), N.ptr(v), N.ptr(k2), N.ptr(v2), n, 0, 19,
+               N.ptr(ws), size, ctypes.byref(sel), s)
+    else:
+        size = lib.tgs_segmented_sort_workspace_size(3 << 19, 1)
+        ws = torch.empty(size, dtype=torch.uint8, device=gpu)
+        N.call("tgs_segmented_sort_pairs_u32", N.ptr(k), N.ptr(v), N.ptr(k2), N.ptr(v2), 4, n, 1,
+               (ctypes.c_uint32 * 2)(0, n), 0, 19, N.ptr(ws), size, ctypes.byref(sel), s)
+    np.testing.assert_array_equal(to_np(v2 if sel.value else v), np.argsort(keys, kind="stable"))
+
+
 @pytest.mark.parametrize("n", [1, 9, 8192, 8193, 16384, 16385])
 def test_scan_size_rules(gpu, n):
     """One-workgroup and three-kernel scans at the line between them."""

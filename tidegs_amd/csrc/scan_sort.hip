@@ -552,8 +552,9 @@ __global__ void __launch_bounds__(SORT_THREADS) __attribute__((amdgpu_waves_per_
 // of whole tiles win: with 64-bit keys at 1.2M (172 against 164 us), with
 // 32-bit ones later (1.2M 82 against 97, 2.7M 157 against 113).
 #define SORT_ITEMS_SMALL 4
+static uint64_t sort_small_line(uint32_t key_bytes) { return key_bytes == 8 ? 1u << 20 : 3u << 19; }
 static uint32_t sort_items(uint64_t n, uint32_t key_bytes) {
-  return n < (key_bytes == 8 ? 1u << 20 : 3u << 19) ? SORT_ITEMS_SMALL : SORT_ITEMS;
+  return n < sort_small_line(key_bytes) ? SORT_ITEMS_SMALL : SORT_ITEMS;
 }
 
 // Most tiles a sort of n keys in n_segments segments can have (a caller's
@@ -570,12 +571,24 @@ static size_t radix_workspace(uint64_t tiles) {
   return (size_t)(al(hist * 4) * 2 + al(tgs_scan_workspace_size(hist)));
 }
 
-extern "C" size_t tgs_radix_sort_workspace_size(uint64_t n) {
-  return radix_workspace(sort_tiles_max(n, 8, 0));
+// What a sort of n keys takes, and what it and every sort of fewer keys (in no more
+// segments) takes: a workspace sized once for the largest sort serves them all.  The
+// sorts below the line take quarter tiles, so the largest of them counts too (2 MB
+// of histograms with 64-bit keys, 3 MB with 32-bit ones).
+static size_t sort_workspace(uint64_t n, uint32_t key_bytes, uint64_t n_segments) {
+  return radix_workspace(sort_tiles_max(n, key_bytes, n_segments));
+}
+static size_t sort_workspace_up_to(uint64_t n, uint32_t key_bytes, uint64_t n_segments) {
+  const uint64_t line = sort_small_line(key_bytes);
+  const size_t own = sort_workspace(n, key_bytes, n_segments);
+  const size_t small = n < line ? 0 : sort_workspace(line - 1, key_bytes, n_segments);
+  return own > small ? own : small;
 }
 
+extern "C" size_t tgs_radix_sort_workspace_size(uint64_t n) { return sort_workspace_up_to(n, 8, 0); }
+
 extern "C" size_t tgs_segmented_sort_workspace_size(uint64_t n, uint32_t n_segments) {
-  return radix_workspace(sort_tiles_max(n, 4, n_segments));
+  return sort_workspace_up_to(n, 4, n_segments);
 }
 
 // Tile and group bases of the segments (key_off set) for tiles of `items` keys
@@ -707,9 +720,9 @@ static int radix_sort_u64(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, ui
   TGS_CHECK_ARG(keys && vals && keys_alt && vals_alt && workspace, "radix_sort: null pointer");
   TGS_CHECK_ARG(begin_bit >= 0 && end_bit <= 64, "radix_sort: bit range out of [0,64]");
   TGS_CHECK_ARG(n < (1ull << 32) - SORT_TILE, "radix_sort: n too large");
-  if (workspace_bytes < tgs_radix_sort_workspace_size(n)) {
+  if (workspace_bytes < sort_workspace(n, 8, 0)) {
     tgs_set_error("radix_sort: workspace %zu < %zu", workspace_bytes,
-                  tgs_radix_sort_workspace_size(n));
+                  sort_workspace(n, 8, 0));
     return TGS_ERR_WORKSPACE;
   }
   RadixSegs sg{};
@@ -816,9 +829,9 @@ extern "C" int tgs_radix_sort_pairs_noalloc(uint64_t* keys, uint32_t* vals, uint
                         TGS_ALIGN256((TGS_NOALLOC_SORT_HIST + SCAN_CHUNK - 1) / SCAN_CHUNK * 8ull +
                                      8ull),
                 "scratch smaller than the sort workspace");
-  if (tgs_radix_sort_workspace_size(n) > TGS_NOALLOC_SORT_BYTES) {
+  if (sort_workspace(n, 8, 0) > TGS_NOALLOC_SORT_BYTES) {
     tgs_set_error("radix_sort_noalloc: workspace %zu exceeds the scratch array",
-                  tgs_radix_sort_workspace_size(n));
+                  sort_workspace(n, 8, 0));
     return TGS_ERR_WORKSPACE;
   }
   void* ws = nullptr;
@@ -917,9 +930,9 @@ static int segmented_sort_u32(uint32_t* keys, void* vals, uint32_t* keys_alt, vo
     sg.key_off[s] = seg_offsets[s];
   }
   sg.key_off[n_segments] = (uint32_t)n;
-  if (workspace_bytes < tgs_segmented_sort_workspace_size(n, n_segments)) {
+  if (workspace_bytes < sort_workspace(n, 4, n_segments)) {
     tgs_set_error("segmented_sort: workspace %zu < %zu", workspace_bytes,
-                  tgs_segmented_sort_workspace_size(n, n_segments));
+                  sort_workspace(n, 4, n_segments));
     return TGS_ERR_WORKSPACE;
   }
   if (value_bytes == 4)
