@@ -523,7 +523,10 @@ int tgs_tide_isect_emit_blocked_hist(uint32_t n_entries, const int32_t* cam_offs
  *   tgs_tide_isect_fused_digit_bits  the first pass's width w over tile_n_bits
  *                                    bits (ceil(bits / 8) passes of
  *                                    ceil(bits / passes) bits);
- *   tgs_tide_isect_fused_hist_words  hist words: blocks * 2^w;
+ *   tgs_tide_isect_fused_hist_words  words that hist and hist_scan take, for
+ *                                    this batch and every one of fewer entries;
+ *   tgs_tide_isect_fused_used_words  the words of them this batch fills, the
+ *                                    scan's length: blocks * 2^w;
  *   tgs_tide_isect_fused_count       hist [camera][digit][block of the camera]
  *                                    = the block's intersections with tile &
  *                                    (2^w - 1) == digit;
@@ -537,6 +540,8 @@ int tgs_tide_isect_emit_blocked_hist(uint32_t n_entries, const int32_t* cam_offs
  *    tile_n_bits > w, completes the tile-bit sort). */
 uint32_t tgs_tide_isect_fused_digit_bits(uint32_t tile_n_bits);
 uint64_t tgs_tide_isect_fused_hist_words(uint32_t C, const uint32_t* cam_offsets,
+                                         uint32_t tile_n_bits);
+uint64_t tgs_tide_isect_fused_used_words(uint32_t C, const uint32_t* cam_offsets,
                                          uint32_t tile_n_bits);
 int tgs_tide_isect_fused_count(uint32_t C, const uint32_t* cam_offsets,
                                const uint64_t* entry_rects, uint32_t tile_width,

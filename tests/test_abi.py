@@ -156,6 +156,15 @@ def test_scratch_sizes_never_shrink_with_the_problem():
     for n in (1, 1 << 20, (3 << 19) - 1, 3 << 19, 10_000_000):
         _never_smaller(lib.tgs_segmented_sort_workspace_size, [(n, k) for k in range(1, 65)],
                        "segmented sort workspace by segments")
+    for cams in (1, 2, 16, 32):
+        def hist_words(n, query=lib.tgs_tide_isect_fused_hist_words):
+            offs = (ctypes.c_uint32 * (cams + 1))(*[n * c // cams for c in range(cams + 1)])
+            return query(cams, offs, 13)
+
+        sizes = [(n,) for n in keys + [5_000_000, 8_400_000, 9_000_000] if n >= cams]
+        _never_smaller(hist_words, sorted(sizes), f"fused histogram of {cams} cameras")
+        for n, in sizes:
+            assert hist_words(n, lib.tgs_tide_isect_fused_used_words) <= hist_words(n)
     dims = sorted({1, 5, 10, 11, 12, 13, 22, 44, 45, 54, 55, 78, 79, 123, 124, 546, 979, 1080, 1920,
                    4096, *range(14, 120, 7)})
     counts = sorted({1, 2, 3, 4, 5, 6, 7, 16, 17, 48, 64, 255, 256, 257, 4096})

@@ -146,6 +146,7 @@ SIGNATURES = {
          P]),
     "tgs_tide_isect_fused_digit_bits": (U32, [U32]),
     "tgs_tide_isect_fused_hist_words": (U64, [U32, P, U32]),
+    "tgs_tide_isect_fused_used_words": (U64, [U32, P, U32]),
     "tgs_tide_isect_fused_count": (ctypes.c_int, [U32, P, P, U32, U32, P, U64, P]),
     "tgs_tide_isect_fused_scatter": (
         ctypes.c_int, [U32, P, P, U32, U32, P, U64, U32, P, P, P]),

@@ -36,6 +36,8 @@ extern "C" int tgs_segmented_sort_pairs_u32_range(uint32_t* keys, void* vals, ui
 extern "C" uint32_t tgs_tide_isect_fused_digit_bits(uint32_t tile_n_bits);
 extern "C" uint64_t tgs_tide_isect_fused_hist_words(uint32_t C, const uint32_t* cam_offsets,
                                                     uint32_t tile_n_bits);
+extern "C" uint64_t tgs_tide_isect_fused_used_words(uint32_t C, const uint32_t* cam_offsets,
+                                                    uint32_t tile_n_bits);
 extern "C" int tgs_tide_isect_fused_count(uint32_t C, const uint32_t* cam_offsets,
                                           const uint64_t* entry_rects, uint32_t tile_width,
                                           uint32_t tile_n_bits, uint32_t* hist,
@@ -498,11 +500,13 @@ static bool isect_sorted_layout(uint32_t C, const uint64_t* summary, uint32_t ti
   // and 169, of 233 386 and 269; 40k of 61 239 and 255, of 858 1493 and 1785; 100k
   // of 61 290 and 454; 400k of 16 236 and 426, of 61 688 and 1572.
   if (o.V < (1u << 15) && (o.V < 2048u || o.n > 32ull * o.V)) return false;
-  o.hist_words = tgs_tide_isect_fused_hist_words(C, o.ent, o.tile_bits);
+  o.hist_words = tgs_tide_isect_fused_used_words(C, o.ent, o.tile_bits);
   if (o.hist_words == 0 || o.n != summary[0]) return false;
   o.sort_bytes = std::max(tgs_segmented_sort_workspace_size(o.V, C),
                           tgs_segmented_sort_workspace_size(o.n, C));
-  o.scan_bytes = tgs_scan_workspace_size(o.hist_words);
+  // (buffers that also hold every smaller call's)
+  const uint64_t hist_most = tgs_tide_isect_fused_hist_words(C, o.ent, o.tile_bits);
+  o.scan_bytes = tgs_scan_workspace_size(hist_most);
   uint64_t at = 0;
   auto take = [&](uint64_t bytes) {
     const uint64_t a = at;
@@ -512,8 +516,8 @@ static bool isect_sorted_layout(uint32_t C, const uint64_t* summary, uint32_t ti
   o.dkeys = take(4ull * o.V);
   o.dkeys2 = take(4ull * o.V);
   o.rects = take(8ull * o.V);
-  o.hist = take(4 * o.hist_words);
-  o.scan = take(4 * o.hist_words);
+  o.hist = take(4 * hist_most);
+  o.scan = take(4 * hist_most);
   o.keys = take(4ull * o.n);
   o.keys2 = take(4ull * o.n);
   o.fids2 = take(4ull * o.n);

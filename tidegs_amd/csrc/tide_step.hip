@@ -1705,7 +1705,8 @@ extern "C" uint32_t tgs_tide_isect_fused_digit_bits(uint32_t tile_n_bits) {
 // and tile pass with 256 and 1024, in us: 9.6k entries 34 and 52, 37k 41 and
 // 81, 0.46M 58 and 73, 1.1M 188 and 202 (with the depth sort), 3.6M 323 and 303;
 // 58M 1957 and 1418.
-static uint32_t fe_entries(uint32_t n_entries) { return n_entries < (1u << 21) ? 256 : 1024; }
+#define FE_SMALL (1u << 21)
+static uint32_t fe_entries(uint32_t n_entries) { return n_entries < FE_SMALL ? 256 : 1024; }
 
 #define FE_LAUNCH(kernel, entries, ...)                                                       \
   do {                                                                                        \
@@ -1742,13 +1743,29 @@ static int fused_emit_setup(uint32_t C, const uint32_t* cam_offsets, uint32_t ti
   return TGS_OK;
 }
 
+extern "C" uint64_t tgs_tide_isect_fused_used_words(uint32_t C, const uint32_t* cam_offsets,
+                                                    uint32_t tile_n_bits) {
+  FusedEmit fe;
+  uint32_t nb = 0;
+  if (fused_emit_setup(C, cam_offsets, 1, tile_n_bits, fe, nb, "tide_isect_fused_used_words"))
+    return 0;
+  return (uint64_t)nb * (fe.mask + 1u);
+}
+
+// The buffers' words also cover every batch of fewer entries: just below FE_SMALL a
+// batch takes more blocks than up to four times as many entries do.
 extern "C" uint64_t tgs_tide_isect_fused_hist_words(uint32_t C, const uint32_t* cam_offsets,
                                                     uint32_t tile_n_bits) {
   FusedEmit fe;
   uint32_t nb = 0;
   if (fused_emit_setup(C, cam_offsets, 1, tile_n_bits, fe, nb, "tide_isect_fused_hist_words"))
     return 0;
-  return (uint64_t)nb * (fe.mask + 1u);
+  uint32_t small = 0;
+  for (uint32_t c = 0; c < C; ++c)
+    small += (uint32_t)(((uint64_t)cam_offsets[c + 1] - cam_offsets[c] + 255) / 256);
+  const uint32_t most = (FE_SMALL - 1) / 256 + C;
+  small = small < most ? small : most;
+  return (uint64_t)(nb > small ? nb : small) * (fe.mask + 1u);
 }
 
 extern "C" int tgs_tide_isect_fused_count(uint32_t C, const uint32_t* cam_offsets,
