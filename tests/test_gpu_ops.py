@@ -1016,3 +1016,33 @@ def test_raster_order_permutes_and_matches(gpu, C, tw, th):
     assert torch.equal(rc, rc2) and torch.equal(ra, ra2)
     for a, b in zip(grads, grads2):
         assert rel_l2(to_np(a), to_np(b)) < 2e-5
+
+
+def test_rasterize_without_gradients_leaves_no_states(gpu, monkeypatch):
+    """A render whose backward cannot follow (no_grad, inference_mode, detached
+    inputs) takes the forward without segment states; the image is the same."""
+    announce("raster without gradients")
+    from tidegs_amd import _native as N
+    *tensors, offs, flat = _dense_tiles(gpu, 90, 4, 4, 3)
+    leaves = [t.requires_grad_() for t in tensors]
+    called = []
+    call = N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: (called.append(name), call(name, *a))[1])
+
+    def render(ts):
+        called.clear()
+        out = ops.rasterize_to_pixels(*ts, 64, 64, 16, offs, flat)
+        return out, "tgs_tide_rasterize_fwd_split" in called
+
+    (ref, _), split = render(leaves)
+    assert split and ref.requires_grad
+    with torch.no_grad():
+        (img, _), split = render(leaves)
+    assert not split and torch.equal(img, ref)
+    with torch.inference_mode():
+        (img, _), split = render(leaves)
+    assert not split and torch.equal(img, ref)
+    (img, _), split = render([t.detach() for t in leaves])
+    assert not split and torch.equal(img, ref)
+    (img, _), split = render([leaves[0].detach(), *leaves[1:]])
+    assert split and torch.equal(img, ref)

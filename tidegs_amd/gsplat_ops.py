@@ -467,7 +467,7 @@ class _RasterizeToPixels(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, means2d, conics, colors, opacities, backgrounds, width, height, tile_size,
-                isect_offsets, flatten_ids, absgrad, masks):
+                isect_offsets, flatten_ids, absgrad, masks, backward_follows):
         C = isect_offsets.shape[0]
         th, tw = isect_offsets.shape[1], isect_offsets.shape[2]
         ch = colors.shape[-1]
@@ -483,7 +483,7 @@ class _RasterizeToPixels(torch.autograd.Function):
                     N.ptr(render_colors), N.ptr(render_alphas), N.ptr(last_ids))
             # few tiles: split the backward along the tiles' lists
             items = (N.load().tgs_tide_raster_split_items(C, tw, th, flatten_ids.numel())
-                     if any(ctx.needs_input_grad[:4]) and C * width * height else 0)
+                     if backward_follows and C * width * height else 0)
             # a few rounds of workgroups: the longest lists first
             if C * width * height and N.load().tgs_tide_raster_order_tiles(
                     C, tw, th, flatten_ids.numel()):
@@ -585,7 +585,7 @@ class _RasterizeToPixels(torch.autograd.Function):
         if ctx.needs_input_grad[4]:
             v_backgrounds = (v_out_colors * (1.0 - out_alphas)).sum(dim=(1, 2))
         return (v_means2d, v_conics, v_colors, v_opacities, v_backgrounds, None, None, None,
-                None, None, None, None)
+                None, None, None, None, None)
 
 
 def rasterize_to_pixels(
@@ -637,6 +637,10 @@ def rasterize_to_pixels(
     N.require_cuda(means2d, conics, colors, opacities, backgrounds, isect_offsets, flatten_ids,
                    names=["means2d", "conics", "colors", "opacities", "backgrounds",
                           "isect_offsets", "flatten_ids"])
+    # asked here: inside the Function grad mode is off, and its needs_input_grad is set
+    # for inputs that require a gradient under torch.no_grad() too
+    backward_follows = torch.is_grad_enabled() and any(
+        t.requires_grad for t in (means2d, conics, colors, opacities))
     return _RasterizeToPixels.apply(
         means2d, conics, colors, opacities, backgrounds, int(image_width), int(image_height),
-        int(tile_size), isect_offsets, flatten_ids, absgrad, masks)
+        int(tile_size), isect_offsets, flatten_ids, absgrad, masks, backward_follows)
