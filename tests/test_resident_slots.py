@@ -94,3 +94,46 @@ def test_component_learning_rates():
         component_learning_rates(None, specs)
     with pytest.raises(RuntimeError, match="12 values"):
         component_learning_rates(np.ones(12), specs)
+
+
+def test_next_bias_terms_follow_the_step_counts(monkeypatch):
+    """The table uploaded ahead of a step holds every slot's terms after one more
+    step, whatever changed the counts; only changed counts are computed (a layout
+    of many blocks costs no powers of the untouched ones)."""
+    from tidegs_amd.resident_optim import GPUResidentAdam
+
+    computed = []
+    plain = GPUResidentAdam._set_bias_terms
+
+    def counted(table, slots, steps, beta1, beta2):
+        computed.append(len(slots))
+        plain(table, slots, steps, beta1, beta2)
+
+    monkeypatch.setattr(GPUResidentAdam, "_set_bias_terms", staticmethod(counted))
+    opt = GPUResidentAdam(block_size=4, device="cpu")
+    slots = opt.slots
+    slots.add_slots(1000)
+    rng = np.random.default_rng(0)
+
+    def check(betas, at_most):
+        computed.clear()
+        got = opt._next_bias_terms(*betas)
+        assert sum(computed) <= at_most
+        t = slots.steps.astype(np.float64) + 1
+        np.testing.assert_array_equal(got, np.stack(
+            [1.0 - betas[0] ** t, np.sqrt(1.0 - betas[1] ** t)]).astype(np.float32))
+
+    betas = (0.9, 0.999)
+    check(betas, 1000)
+    check(betas, 0)
+    for _ in range(5):
+        hit = np.sort(rng.choice(1000, 7, replace=False))
+        slots.advance(hit, np.full(7, 4), np.full(7, 2))
+        check(betas, 7)
+    slots.retarget(range(40), lambda n: None)   # admitted blocks start over
+    check(betas, 40)
+    slots.steps[100:200] = 500                  # a restored snapshot
+    check(betas, 100)
+    check((0.8, 0.99), 1000)
+    slots.add_slots(24)
+    check((0.8, 0.99), 1024)

@@ -240,6 +240,11 @@ class GPUResidentAdam:
         # each with the event of its last copy
         self._bias_host = np.zeros((2, 0), np.float32)
         self._bias_terms: Optional[torch.Tensor] = None
+        # every slot's bias terms after one more step, the step counts and the
+        # betas they were computed from
+        self._next_terms = np.zeros((2, 0), np.float32)
+        self._next_steps = np.zeros(0, np.int64)
+        self._next_betas = None
         self._staging = []
         self._staging_turn = 0
         self._counts_dev: Optional[torch.Tensor] = None
@@ -310,6 +315,22 @@ class GPUResidentAdam:
         t = steps.astype(np.float64)
         table[0, slots] = 1.0 - beta1 ** t
         table[1, slots] = np.sqrt(1.0 - beta2 ** t)
+
+    def _next_bias_terms(self, beta1: float, beta2: float) -> np.ndarray:
+        """Every slot's bias terms after one more step.  Computed for the slots
+        whose step count is not the one they were last computed from: those of
+        the last step's touched blocks, not the whole table at every step (two
+        float64 powers per block: a step on 1.1k rows of 100k blocks 1140 us,
+        170 so)."""
+        steps = self.slots.steps
+        if self._next_betas != (beta1, beta2) or self._next_steps.size != steps.size:
+            self._next_terms = np.zeros((2, steps.size), np.float32)
+            self._next_steps = np.full(steps.size, -1, np.int64)
+            self._next_betas = (beta1, beta2)
+        stale = np.flatnonzero(self._next_steps != steps)
+        self._set_bias_terms(self._next_terms, stale, steps[stale] + 1, beta1, beta2)
+        self._next_steps[stale] = steps[stale]
+        return self._next_terms
 
     def _upload_bias_table(self, table: np.ndarray) -> None:
         """Queue the upload of a whole bias table from the staging table whose
@@ -392,9 +413,9 @@ class GPUResidentAdam:
 
     def _apply_counts(self, layout: _Layout, counts: np.ndarray, n_rows: int, beta1: float,
                       beta2: float, upload: bool = True) -> Dict[str, Any]:
-        """Advance the slots of the touched blocks and refresh their bias
-        terms (``gpu_resident_optimizer.py:302-337`` behaviour; uploaded unless
-        the caller has); returns the step's stats dictionary."""
+        """Advance the slots of the touched blocks and, unless the caller has
+        uploaded them, refresh their bias terms (``gpu_resident_optimizer.py:
+        302-337`` behaviour); returns the step's stats dictionary."""
         if counts.shape[0] != len(layout) or int(counts.sum()) != int(n_rows):
             raise RuntimeError(
                 "[GPUResidentAdam] a touched row lies outside every resident block of the layout")
@@ -404,8 +425,6 @@ class GPUResidentAdam:
             slots, layout.stops[hit] - layout.starts[hit], counts[hit])
         if slots.size and upload:
             self._upload_bias_terms(slots, beta1, beta2)
-        elif slots.size:
-            self._set_bias_terms(self._bias_host, slots, self.slots.steps[slots], beta1, beta2)
         self._counters["cold_restarts"] += cold_slots
         self._counters["cold_restarted_rows_touched_total"] += cold_rows
         self._counters["optimizer_rows_touched_total"] += int(n_rows)
@@ -483,14 +502,11 @@ class GPUResidentAdam:
                                                       beta2, eps, iteration)
         # The GPU does not wait for the host: the update is queued behind the
         # counts and their check, with bias terms of one more step for every
-        # block of the layout (the kernel reads those of touched blocks only),
-        # and the host advances the touched slots while it runs.
+        # slot (the kernel reads those of touched blocks only), and the host
+        # advances the touched slots while it runs.
         ready = self._check_touches(layout, rows)
         if self._bias_corrected:
-            table = self._bias_host.copy()
-            self._set_bias_terms(table, layout.slots, self.slots.steps[layout.slots] + 1, beta1,
-                                 beta2)
-            self._upload_bias_table(table)
+            self._upload_bias_table(self._next_bias_terms(beta1, beta2))
         hooks = self.kernel_hooks
         if hooks:
             hooks[0]()
