@@ -385,7 +385,8 @@ def test_isect_tiles_packed_and_empty(gpu):
 
 @pytest.mark.parametrize("n,begin,end", [(1, 0, 64), (100, 0, 46), (4097, 3, 40),
                                          (1_000_003, 0, 46), (70_000, 0, 64),
-                                         ((1 << 20) - 1, 0, 46), (1 << 20, 0, 46)])
+                                         ((1 << 20) - 1, 0, 46), (1 << 20, 0, 46),
+                                         (3 << 20, 0, 40), ((3 << 20) + 1, 0, 40)])
 def test_radix_sort_pairs_stable(gpu, n, begin, end):
     announce(f"radix n={n} bits=[{begin},{end})")
     rng = np.random.default_rng(n)

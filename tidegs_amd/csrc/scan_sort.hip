@@ -264,15 +264,18 @@ extern "C" int tgs_exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint64_
 //   kernel's atomics) and the rows since.  A pass is two launches, not five:
 //   the scan's three kernels take 11-16 us of a pass whose histogram and
 //   scatter take 15 us at 10k keys and 25 us at 2.7M.  Above the line the
-//   scatters' row sums cost more than the scan.  Whole sorts, with the scan
-//   and without, in us:
-//     46 bits of 64-bit keys, 4-byte values  10k 134 -> 60, 300k 168 -> 108,
-//                                            2.7M 234 -> 202, 5M 334 -> 376
-//     25 bits of 32-bit keys, 8-byte values  10k 89 -> 39, 300k 112 -> 56,
-//                                            2.7M 147 -> 113, 5M 192 -> 187
+//   scatters' row sums cost more than the scan: with 64-bit keys as soon as the
+//   768 workgroups that the chip holds at once (3 per CU by their LDS) do not
+//   take every tile, with 32-bit ones later.  Whole sorts, with the scan and
+//   without, in us:
+//     46 bits of 64-bit keys, 4-byte values  10k 134 -> 58, 300k 169 -> 115,
+//                                            2.7M 235 -> 221, 3.14M 242 -> 228,
+//                                            3.3M 279 -> 305, 4.1M 303 -> 343
+//     25 bits of 32-bit keys, 8-byte values  10k 87 -> 34, 300k 112 -> 56,
+//                                            2.7M 148 -> 115, 4.1M 177 -> 164
 // ---------------------------------------------------------------------------
 #define RADIX_GROUP 32
-#define RADIX_LOCAL_KEYS (1u << 22)
+#define RADIX_LOCAL_KEYS(key_bytes) ((key_bytes) == 8 ? 3u << 20 : 1u << 22)
 
 struct RadixSegs {
   uint32_t n;                             // number of segments (>= 1)
@@ -661,7 +664,7 @@ static int radix_passes(K* keys, V* vals, K* keys_alt, V* vals_alt, RadixSegs& s
     most = nt > most ? nt : most;
   }
   const bool grouped = most > RADIX_GROUP;
-  const bool local = !first_hist_ready && sg.key_off[sg.n] <= RADIX_LOCAL_KEYS &&
+  const bool local = !first_hist_ready && sg.key_off[sg.n] <= RADIX_LOCAL_KEYS(sizeof(K)) &&
                      (!grouped || group_words * passes <= hist_max);
   if (local && grouped) {
     const int rc = tgs_fill_u32(hist_scan, group_words * passes, 0u, stream);
