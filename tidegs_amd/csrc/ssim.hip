@@ -342,17 +342,21 @@ struct SsimGrid {
 };
 
 // Bands: a lone workgroup's row takes 0.5 us forward and 0.6 us backward, about
-// three times a busy CU's.  Bands of more than 78 rows gain nothing (sixteen
-// 1080p images, 45-, 78- and 133-row bands: forward 780, 758, 766 us, backward
-// 664, 633, 734); one 256x256 image in 12-, 23- and 78-row bands: 15, 20, 49 us.
-#define SSIM_LONE 3.f
+// three times a busy CU's with the three wavefronts of an RGB workgroup and six
+// times with one (its share of the CU is a third; a CU with several is fuller): one
+// plane of 1080p in the bands of 3, 6 and 9 times 39, 24 and 23 us forward and 42,
+// 24 and 32 backward (16x16 tiles: 30 and 39), 979x546 of two planes 21, 17, 17
+// and 22, 17, 17.  Bands of more than 78 rows gain nothing (sixteen 1080p images,
+// 45-, 78- and 133-row bands: forward 780, 758, 766 us, backward 664, 633, 734);
+// one 256x256 image in 12-, 23- and 78-row bands: 15, 20, 49 us.
+#define SSIM_LONE(nw) ((nw) == 1 ? 6.f : 3.f)
 #define SSIM_PERIODS 8
 static SsimGrid ssim_grid(int64_t B, int64_t CH, int H, int W) {
   const int nw = CH % 3 == 0 ? 3 : 1;
   const int64_t planes = B * (CH / nw);
   const int strips = (W + SR_OUT - 1) / SR_OUT;
   SsimGrid g;
-  g.rows = band_input_rows(H, planes * strips, 2 * SS_R, SSIM_LONE, SSIM_PERIODS);
+  g.rows = band_input_rows(H, planes * strips, 2 * SS_R, SSIM_LONE(nw), SSIM_PERIODS);
   const int band = g.rows - 2 * SS_R;
   g.grid = dim3((unsigned)(planes * strips), (H + band - 1) / band);
   g.block = dim3(64 * nw);
@@ -404,10 +408,10 @@ extern "C" int tgs_fused_ssim_bwd(int32_t B, int32_t CH, int32_t H, int32_t W, f
 extern "C" uint64_t tgs_fused_ssim_mean_partials(int32_t B, int32_t CH, int32_t H, int32_t W) {
   if (B <= 0 || CH <= 0 || H <= 0 || W <= 0) return 0;
   const int64_t planes = (int64_t)B * CH, strips = (W + SR_OUT - 1) / SR_OUT;
-  const auto most = [&](int64_t n) {
-    return band_workgroups_max(H, n * strips, 2 * SS_R, SSIM_LONE, SSIM_PERIODS);
+  const auto most = [&](int64_t n, int nw) {
+    return nw * band_workgroups_max(H, n * strips, 2 * SS_R, SSIM_LONE(nw), SSIM_PERIODS);
   };
-  return (uint64_t)std::max(most(planes), 3 * most((planes + 2) / 3));
+  return (uint64_t)std::max(most(planes, 1), most((planes + 2) / 3, 3));
 }
 
 extern "C" int tgs_fused_ssim_mean_fwd(int32_t B, int32_t CH, int32_t H, int32_t W, float C1,
