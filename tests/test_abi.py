@@ -182,3 +182,17 @@ def test_scratch_sizes_never_shrink_with_the_problem():
     for c in (1, 32, 33, 100):
         _never_smaller(lib.tgs_isect_tiles_plan_size, [(c, n) for n in near if n < 1 << 24],
                        "plan by Gaussians")
+
+
+def test_split_and_order_lines():
+    """Which tile counts split the backward: up to 6144, or 3072 where the longest
+    lists go first (several cameras, more than 1536 tiles)."""
+    from tidegs_amd import _native
+
+    lib = _native.load()
+    for (c, w, h), split, order in (((1, 78, 78), 1, 0), ((1, 79, 78), 0, 0), ((3, 32, 16), 1, 0),
+                                    ((3, 23, 23), 1, 1), ((3, 32, 32), 1, 1), ((2, 41, 38), 0, 1),
+                                    ((2, 70, 60), 0, 0)):  # 4200 tiles a camera: not ordered
+        got = [lib.tgs_tide_raster_split_items(c, w, h, 500_000) > 0,
+               lib.tgs_tide_raster_order_tiles(c, w, h, 500_000) > 0]
+        assert got == [bool(split), bool(order)], (c, w, h)

@@ -985,6 +985,7 @@ def test_rasterize_split_matches_whole_tiles(gpu, n, tw, th, crop, what):
 
 
 @pytest.mark.parametrize("C,tw,th", [(3, 23, 23),    # 1587 tiles: just past one round, split too
+                                     (3, 32, 32), (2, 41, 38),  # 3072 the last split, 3116 not
                                      (7, 31, 30),    # 6510: the backward ordered as well
                                      (2, 64, 64), (4, 64, 64)])  # the largest camera, the most tiles
 def test_raster_order_permutes_and_matches(gpu, C, tw, th):

@@ -1846,8 +1846,10 @@ extern "C" int tgs_tide_isect_ids(uint32_t n_isects, const uint32_t* keys,
 //                          1M rows 330 and 825 -> 256 and 759
 //   2 of 1237x822          137 and 412 -> 126 and 387
 //   32 of 256x256          244 and 607 -> 168 and 418
-//   16 of 256x256 (split)  195 and 256 -> 143 and 256
-// The order is by the octave of the list's length relative to the mean (8 classes,
+//   16 of 256x256          forward and backward 310 -> 222
+// Lists that are all of one length gain nothing and take this launch, 5 to 10 us:
+// 2 cameras of 979x546, 1.5M intersections, forward 98 -> 103; 32 of 256x256, 757k,
+// 58 -> 67.  The order is by the octave of the list's length relative to the mean (8 classes,
 // from 4 times it down), so that within a class neighbouring tiles still follow
 // each other (by length alone: the same).  One workgroup, every tile's class in
 // registers: a stable counting sort with three ballots per 64 tiles, about 6 us
@@ -1994,12 +1996,26 @@ extern "C" int tgs_tide_rasterize_fwd(uint32_t C, const float* splats, const flo
 //   475, 87k 124 -> 41; 1000, 311k 162 -> 78; 1000, 4.8M 612 -> 226 (512)
 //   4056, 1.4M 264 -> 219 (512; 64: 251); 4096, 1.9M 398 -> 257
 //   8160, 2.9M 407 -> 420 (512); 32640, 11.6M 1487 -> 1593
-// (the forward takes 0-8% longer).  Shorter segments spread a short list over
-// more workgroups, longer ones spare states and per-workgroup set-up, so the
-// segments are the shortest with at most 4096 of them.
+// (the forward takes 0-8% longer).  Where the longest lists go first the finish is
+// even already, and the split's plain order takes that away, from 3072 tiles on.
+// Forward and backward ordered, and ordered and split, in us:
+//   1900 tiles of 4 cameras, 588k 263 -> 214; 2464 of 2, 675k 234 -> 222
+//   3000 of 3, 1.46M 358 -> 341; 3072 of 12, 741k 285 -> 247
+//   4096 of 16, 670k 222 -> 249, 1.87M 475 -> 420
+//   4340 of 2, 904k 255 -> 280, 1.66M 338 -> 361, 4.0M 643 -> 639; 4800 of 4 299 -> 330
+// Images whose lists are all of one length gain nothing from an even finish: 3000
+// tiles of 3 cameras, 1.45M 401 -> 443; 4056 of 1, 1.23M 348 -> 372.
+// Shorter segments spread a short list over more workgroups, longer ones spare
+// states and per-workgroup set-up, so the segments are the shortest with at most
+// 4096 of them.
 #define RASTER_SPLIT_TILES 6144
-static uint32_t raster_split_shift(uint64_t n_tiles, uint64_t n_isects) {
-  if (n_tiles > RASTER_SPLIT_TILES || n_isects == 0) return 0;
+#define RASTER_SPLIT_TILES_ORDERED 3072
+static uint32_t raster_split_shift(uint32_t C, uint32_t tile_width, uint32_t tile_height,
+                                   uint32_t n_isects) {
+  const uint64_t n_tiles = (uint64_t)C * tile_width * tile_height;
+  const bool ordered = tgs_tide_raster_order_tiles(C, tile_width, tile_height, n_isects) != 0;
+  if (n_tiles > (ordered ? RASTER_SPLIT_TILES_ORDERED : RASTER_SPLIT_TILES) || n_isects == 0)
+    return 0;
   uint32_t shift = 6;
   while (shift < 9 && (n_isects >> shift) > 4096) ++shift;
   return shift;
@@ -2011,7 +2027,7 @@ static uint32_t raster_split_shift(uint64_t n_tiles, uint64_t n_isects) {
 extern "C" uint64_t tgs_tide_raster_split_items(uint32_t C, uint32_t tile_width,
                                                 uint32_t tile_height, uint32_t n_isects) {
   const uint64_t n_tiles = (uint64_t)C * tile_width * tile_height;
-  const uint32_t shift = raster_split_shift(n_tiles, n_isects);
+  const uint32_t shift = raster_split_shift(C, tile_width, tile_height, n_isects);
   if (!shift) return 0;
   const uint32_t shortest = n_isects >> 6 < 4096u ? n_isects >> 6 : 4096u;
   return n_tiles + (n_isects >> shift > shortest ? n_isects >> shift : shortest);
@@ -2023,7 +2039,7 @@ static int raster_split_args(uint32_t C, uint32_t tile_width, uint32_t tile_heig
   const uint64_t n_tiles = (uint64_t)C * tile_width * tile_height;
   sp.states = (float4*)states;
   sp.item_tile = item_tile;
-  sp.shift = raster_split_shift(n_tiles, n_isects);
+  sp.shift = raster_split_shift(C, tile_width, tile_height, n_isects);
   TGS_CHECK_ARG(sp.shift, "tide_rasterize_split: this size is not split");
   sp.items = (uint32_t)(n_tiles + (n_isects >> sp.shift));
   TGS_CHECK_ARG(states && item_tile && ((uintptr_t)states & 15u) == 0,
