@@ -213,8 +213,8 @@ int tgs_segmented_sort_pairs_u32_range(uint32_t* keys, void* vals, uint32_t* key
  * intersections} up to its end.  tgs_isect_tiles_emit_plan writes what
  * tgs_isect_tiles_emit does; tgs_isect_tiles_sorted writes the sorted ids and
  * flatten ids at once (summary: a host copy), where its workspace size is not 0:
- * up to 32 cameras, tiles up to 255 x 255, no negative depth, and from 2048
- * Gaussians on (of up to 32 tiles each on average below 32768). */
+ * up to 32 cameras, tiles up to 255 x 255, no negative depth, and where it is the
+ * faster (from 2048 Gaussians on, by their and their intersections' number). */
 uint64_t tgs_isect_tiles_plan_size(uint32_t C, uint64_t N);
 int tgs_isect_tiles_plan(uint32_t C, uint64_t N, const float* means2d, const int32_t* radii,
                          const float* depths, uint32_t tile_size, uint32_t tile_width,

@@ -339,6 +339,51 @@ def test_isect_offset_encode_ragged(gpu, n, shift):
     np.testing.assert_array_equal(to_np(offs), R.isect_offset_encode(keys, C, tw, th))
 
 
+def _boxes_with_tiles(rng, C, V, n, tw, th):
+    """V Gaussians over C cameras whose tiles are n in all: each of 1, 4, 9 or 25
+    tiles well inside the image, in random order."""
+    base = max(0, -(-(n - 9 * V) // 16))
+    many, b, c = next((m, b, (n - 25 * m - (V - m) - 3 * b) // 8)
+                      for m in range(base, base + 9) for b in range(8)
+                      if (n - 25 * m - (V - m) - 3 * b) % 8 == 0
+                      and 0 <= (n - 25 * m - (V - m) - 3 * b) // 8 <= V - m - b)
+    counts = [25] * many + [4] * b + [9] * c
+    counts = rng.permutation(np.array(counts + [1] * (V - len(counts))))
+    assert counts.size == V and counts.sum() == n
+    at = rng.integers([2, 2], [tw - 3, th - 3], size=(V, 2)) * 16.0
+    m2d = np.where(counts[:, None] == 4, at, at + 8).astype(np.float32)
+    radii = np.select([counts == 1, counts == 4, counts == 9], [7, 7, 17], 33).astype(np.int32)
+    depths = rng.uniform(0.2, 500, size=V).astype(np.float32)
+    return m2d.reshape(C, -1, 2), radii.reshape(C, -1), depths.reshape(C, -1)
+
+
+@pytest.mark.parametrize("C,V,n,two", [
+    (1, 2048, 8 * 2048, True), (1, 2048, 8 * 2048 - 1, False), (1, 2046, 9 * 2046, False),
+    (1, 2500, 24 * 2500, True), (1, 32767, 8 * 32767, True),
+    (1, 1 << 15, 3 << 17, True), (1, 1 << 15, (3 << 17) - 1, False),
+    (1, 210_000, 420_000, True), (1, 210_000, 419_999, False),
+    (2, 4096, 3 << 13, True), (2, 4096, (3 << 13) - 1, False), (4, 40_000, 44_000, True),
+    (2, 2046, 3 << 13, False),
+])
+def test_isect_tiles_sort_lines(gpu, monkeypatch, C, V, n, two):
+    """Two sorts and one on either side of the rule's lines, the path taken and the
+    result: bit-exact with the oracle."""
+    announce(f"isect sort lines C={C} V={V} n={n}")
+    from tidegs_amd import _native as N
+    tw, th = 40, 30
+    arrays = _boxes_with_tiles(np.random.default_rng(V + n), C, V, n, tw, th)
+    called = []
+    call = N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: (called.append(name), call(name, *a))[1])
+    tiles, ids, flat = ops.isect_tiles(*(torch.from_numpy(a).to(gpu) for a in arrays), 16, tw, th)
+    assert ("tgs_isect_tiles_sorted" in called) == two
+    o_tiles, o_ids, o_flat = R.isect_tiles(*arrays, 16, tw, th)
+    assert o_ids.size == n
+    np.testing.assert_array_equal(to_np(tiles), o_tiles)
+    np.testing.assert_array_equal(to_np(ids), o_ids)
+    np.testing.assert_array_equal(to_np(flat), o_flat)
+
+
 @pytest.mark.parametrize("C,tw,th", [(1, 5, 5), (1, 1, 1), (3, 7, 3), (2, 16, 16)])
 def test_isect_negative_depths(gpu, C, tw, th):
     """A negative depth's sign fills the id's high word: ids, order and the bucket

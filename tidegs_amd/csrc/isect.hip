@@ -427,9 +427,7 @@ extern "C" uint32_t tgs_bit_width(uint32_t v) {
 // The reference's order in two sorts: Gaussians by depth (32-bit keys), then the
 // intersections they emit in that order by tile, stably, gives (camera, tile,
 // depth, Gaussian) with two 8-byte moves per intersection instead of the single
-// sort's five 12-byte ones.  isect_tiles and offsets, single sort and two: 1.2M
-// Gaussians, 2.7M intersections 240 and 232 us; a 500k-Gaussian 1237x822 image with
-// its backward 807 and 786 us.  The single sort takes what this does not: packed
+// sort's five 12-byte ones (both measured at the rule below).  The single sort takes what this does not: packed
 // camera ids (in any order), grids past 255 tiles a side (8-bit rectangles), more
 // cameras than the emission's segments, negative depths (their sign fills the id).
 // ---------------------------------------------------------------------------
@@ -493,13 +491,29 @@ static bool isect_sorted_layout(uint32_t C, const uint64_t* summary, uint32_t ti
   }
   o.V = o.ent[C];
   o.n = o.isect[C];
-  // Few Gaussians make few blocks of the fused emission, each a serial chain over
-  // its tiles, and a single sort of few keys is launches either way.  Two sorts and
-  // one, in us, by Gaussians and tiles of each: 300 of 4 99 and 95, of 62 170 and
-  // 106; 2000 of 16 99 and 113, of 61 196 and 138; 10k of 16 109 and 124, of 61 200
-  // and 169, of 233 386 and 269; 40k of 61 239 and 255, of 858 1493 and 1785; 100k
-  // of 61 290 and 454; 400k of 16 236 and 426, of 61 688 and 1572.
-  if (o.V < (1u << 15) && (o.V < 2048u || o.n > 32ull * o.V)) return false;
+  // Two sorts move each Gaussian once per depth pass and each intersection twice,
+  // one sort every intersection five times (six with several cameras' bits): two win
+  // where the intersections outnumber the Gaussians by enough, and past the sizes at
+  // which either is launches only (one sort of few keys has fewer).  Few Gaussians of
+  // many tiles are few blocks of the fused emission, each a serial chain.
+  // isect_tiles in two sorts and in one, in us, by Gaussians and tiles of each:
+  //   1 camera
+  //   3000     1.6 88 77, 3.2 88 80, 5 89 82      2000 of 16 99 113, of 61 196 138
+  //   12k      1.6 91 85, 3.2 97 99, 5 97 99      10k of 16 109 124, of 61 200 169
+  //   40k      1.6 110 101, 3.2 112 103, 5 113 107       40k of 61 239 255
+  //   130k     1.6 124 117, 2.5 126 126, 3.2 128 131, 5 131 146
+  //   500k     1.3 153 150, 1.6 153 154, 2 156 168, 3.2 167 186, 5 177 223
+  //   1.5M     1.3 238 208, 1.6 248 229, 2 255 238, 2.5 269 326, 5 321 455
+  //   4M       1.3 448 390, 1.6 475 427, 2 511 495, 2.5 566 605, 5 805 1199
+  //   4 cameras, Gaussians of all
+  //   5000     1.6 88 81, 3.2 89 85, 5 89 92
+  //   12k      1.3 89 85, 2 89 91, 3.2 90 104
+  //   40k      1.3 96 107, 3.2 98 112             500k 1.3 147 166, 3.2 161 194
+  //   4M       1.3 392 396, 2 432 501, 5 670 1210
+  const bool few = o.V < (1u << 15);
+  if (few && (o.V < 2048u || o.n > 32ull * o.V)) return false;
+  if (C > 1 ? o.n < (3u << 13) : few ? o.n < 8ull * o.V : o.n < (3u << 17) || o.n < 2ull * o.V)
+    return false;
   o.hist_words = tgs_tide_isect_fused_used_words(C, o.ent, o.tile_bits);
   if (o.hist_words == 0 || o.n != summary[0]) return false;
   o.sort_bytes = std::max(tgs_segmented_sort_workspace_size(o.V, C),
