@@ -837,8 +837,9 @@ def test_rasterize_masks(gpu, D, tile, bg):
 
 @pytest.mark.parametrize("B,H,W", [(1, 70, 130), (2, 37, 21)])
 def test_tide_loss_kernel(gpu, B, H, W):
-    """One-pass L1 + SSIM loss and gradient (tgs_tide_loss) against the oracle
-    restatement of base_engine.py:464-488, per image of the batch."""
+    """One-pass L1 + SSIM loss and gradient (tgs_tide_loss and the form with
+    partial sums, tgs_tide_loss_summed) against the oracle restatement of
+    base_engine.py:464-488, per image of the batch."""
     announce(f"tide loss (L1 + SSIM) B={B} {H}x{W}")
     from tidegs_amd import _native as N
 
@@ -846,16 +847,29 @@ def test_tide_loss_kernel(gpu, B, H, W):
     img = torch.rand((B, H, W, 3), generator=g)
     gt = torch.rand((B, 3, H, W), generator=g) * 300 - 20
     d_img, d_gt = img.to(gpu), gt.to(gpu)  # keep the device copies alive
+    s, nan = N.stream_handle(), float("nan")
+    forms = []
     sums = torch.zeros(2 * B, dtype=torch.float64, device=gpu)
     v = torch.empty((B, H, W, 3), device=gpu)
-    N.call("tgs_tide_loss", B, H, W, N.ptr(d_img), N.ptr(d_gt), 255.0, 0.2, N.ptr(sums), N.ptr(v),
-           N.stream_handle())
-    sums = to_np(sums)
+    N.call("tgs_tide_loss", B, H, W, N.ptr(d_img), N.ptr(d_gt), 255.0, 0.2, N.ptr(sums), N.ptr(v), s)
+    forms.append((to_np(sums), v))
+    # the form with partial sums (the step's) overwrites both, in a fixed order
+    for _ in range(2):
+        sums = torch.full((2 * B,), nan, dtype=torch.float64, device=gpu)
+        v = torch.full((B, H, W, 3), nan, device=gpu)
+        partials = torch.full((N.load().tgs_tide_loss_partials(B, H, W),), nan, dtype=torch.float64,
+                              device=gpu)
+        N.call("tgs_tide_loss_summed", B, H, W, N.ptr(d_img), N.ptr(d_gt), 255.0, 0.2,
+               N.ptr(partials), N.ptr(sums), N.ptr(v), s)
+        forms.append((to_np(sums), v))
+    np.testing.assert_array_equal(forms[1][0], forms[2][0])
+    assert all(torch.equal(forms[0][1], f[1]) for f in forms[1:])
     n = 3 * H * W
     for bi in range(B):
         loss_ref, grad_ref = S.tide_loss(img[bi].permute(2, 0, 1).numpy(), gt[bi].numpy())
-        loss = 0.8 * sums[2 * bi] / n + 0.2 * (1 - sums[2 * bi + 1] / n)
-        assert abs(loss - loss_ref) < 1e-6
+        for sums, v in forms[:2]:
+            loss = 0.8 * sums[2 * bi] / n + 0.2 * (1 - sums[2 * bi + 1] / n)
+            assert abs(loss - loss_ref) < 1e-6
         assert rel_l2(to_np(v[bi]).transpose(2, 0, 1), grad_ref) < 1e-5
 
 
@@ -1093,3 +1107,40 @@ def test_rasterize_without_gradients_leaves_no_states(gpu, monkeypatch):
     assert not split and torch.equal(img, ref)
     (img, _), split = render([leaves[0].detach(), *leaves[1:]])
     assert split and torch.equal(img, ref)
+
+
+@pytest.mark.parametrize("n,shift", [(1500, 6), (9000, 8), (17_500, 9)])
+def test_rasterize_split_matches_oracle(gpu, n, shift):
+    """The split backward against the oracle at segments of 64, 256 and 512 entries,
+    pixels that composite some 2000 entries, a ragged image.  Tolerances as for the
+    other raster forms.  The Gaussians are wide and their opacities 0.0043 to 0.005,
+    so that no alpha lies at the 1/255 test: one that rounding puts on its other
+    side, of 30M, would weigh 2e-4 in the gradients (in the whole-tile kernels too)."""
+    announce(f"split raster against the oracle n={n} segments of {1 << shift}")
+    from tidegs_amd import _native as N
+    tw = th = 8
+    *splats, offs, flat = _dense_tiles(gpu, n, tw, th, n, (0.0043, 0.005))
+    rng = np.random.default_rng(n)
+    q = np.stack([rng.uniform(0.5e-4, 1.5e-4, n * 64), rng.uniform(-0.3e-4, 0.3e-4, n * 64),
+                  rng.uniform(0.5e-4, 1.5e-4, n * 64)], 1)
+    splats[1] = torch.from_numpy(q.astype(np.float32))[None].to(gpu)
+    W, H = 16 * tw - 5, 16 * th - 9
+    n_isects = flat.numel()
+    assert N.load().tgs_tide_raster_split_items(1, tw, th, n_isects) >= 64 + (n_isects >> shift)
+    assert shift == 6 or (n_isects >> (shift - 1)) > 4096
+    assert shift == 9 or (n_isects >> shift) <= 4096
+    leaves = [t.clone().requires_grad_() for t in splats]
+    rc, ra = ops.rasterize_to_pixels(*leaves, W, H, 16, offs, flat)
+    args = (*(to_np(t)[0] for t in splats), W, H, 16, to_np(offs), to_np(flat))
+    ref_c, ref_a, ref_last = R.rasterize_fwd(*args)
+    assert rel_l2(to_np(rc), ref_c) < 1e-5 and rel_l2(to_np(ra)[..., 0], ref_a) < 1e-5
+    deep = ref_last.ravel() - to_np(offs).reshape(th, tw).repeat(16, 0).repeat(16, 1)[:H, :W].ravel()
+    assert np.median(deep) > min(n - 1, 3 << shift) * 0.99  # three segments at most pixels
+    g = torch.Generator().manual_seed(n)
+    wc, wa = torch.randn(rc.shape, generator=g), torch.randn(ra.shape, generator=g)
+    grads = torch.autograd.grad((rc, ra), leaves, (wc.to(gpu), wa.to(gpu)))
+    # from the GPU's own alphas: the walk back starts at 1 - alpha, whose rounding
+    # (2^-24 of a final transmittance down to 1e-4) would otherwise be the difference
+    ref = R.rasterize_bwd(*args, to_np(ra)[..., 0], ref_last, to_np(wc), v_alphas=to_np(wa)[..., 0])[:4]
+    for got, want in zip(grads, ref):
+        assert rel_l2(to_np(got)[0], want) < 1e-4
