@@ -136,18 +136,21 @@ __global__ void __launch_bounds__(256) isect_emit_kernel(
 // key, writing the run of empty buckets before its own, took 9 us for 2.7M keys of
 // 4293 tiles and 31 us for 1.4M where one thread met a long run (the empty rows
 // above a scene): 6 us in both here.
+// Word: int32_t where the tile bits leave the camera some of the signed word (any
+// bucket of such a word then fits it too), else int64_t.
+template <typename Word>
 __global__ void __launch_bounds__(256) isect_offset_search_kernel(
     uint64_t n_isects, const int64_t* __restrict__ isect_ids, uint64_t n_buckets, uint32_t n_tiles,
     uint32_t tile_n_bits, uint64_t top, int32_t* __restrict__ offsets) {
   const uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= n_buckets) return;
-  const int64_t tmask = ((int64_t)1 << tile_n_bits) - 1;
+  const Word tmask = (Word)(((int64_t)1 << tile_n_bits) - 1), tiles = (Word)n_tiles;
   uint64_t pos = 0;  // keys [0, pos) lie in buckets before b
   for (uint64_t step = top; step != 0u; step >>= 1) {
     const uint64_t p = pos + step;
     if (p > n_isects) continue;
-    const int64_t hi = isect_ids[p - 1] >> 32;
-    if ((hi >> tile_n_bits) * n_tiles + (hi & tmask) < (int64_t)b) pos = p;
+    const Word hi = (Word)(isect_ids[p - 1] >> 32);
+    if ((int64_t)((hi >> tile_n_bits) * tiles + (hi & tmask)) < (int64_t)b) pos = p;
   }
   offsets[b] = (int32_t)pos;
 }
@@ -656,8 +659,9 @@ extern "C" int tgs_isect_offset_encode(uint64_t n_isects, const int64_t* isect_i
   const uint32_t tile_n_bits = tgs_bit_width(n_tiles);
   uint64_t top = 1;
   while (top <= n_isects / 2) top <<= 1;
-  hipLaunchKernelGGL(isect_offset_search_kernel, dim3(tgs_blocks(total, 256)), dim3(256), 0, stream,
-                     n_isects, isect_ids, total, n_tiles, tile_n_bits, top,
-                     offsets);
+  hipLaunchKernelGGL(tile_n_bits < 31 ? isect_offset_search_kernel<int32_t>
+                                      : isect_offset_search_kernel<int64_t>,
+                     dim3(tgs_blocks(total, 256)), dim3(256), 0, stream, n_isects, isect_ids, total,
+                     n_tiles, tile_n_bits, top, offsets);
   TGS_RETURN_LAUNCH("tgs_isect_offset_encode");
 }
