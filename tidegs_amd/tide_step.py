@@ -379,8 +379,8 @@ class TideStep:
         dkeys2 = self._buf("depth_keys2", cap_v, torch.int32)
         rects2 = self._buf("entry_rects2", cap_v, torch.int64)
         tile_bits = (tw * th).bit_length()
-        hist_words = max(int(lib.tgs_tide_isect_fused_hist_words(C, cam_segs, tile_bits)), 1)
-        used_words = int(lib.tgs_tide_isect_fused_used_words(C, cam_segs, tile_bits))
+        # (asked for every batch, so this batch's words are enough)
+        hist_words = max(int(lib.tgs_tide_isect_fused_used_words(C, cam_segs, tile_bits)), 1)
         fe_hist = self._buf("fused_hist", hist_words, torch.int32)
         fe_scan = self._buf("fused_hist_scan", hist_words, torch.int32)
         ws = self._buf("scan_ws2", lib.tgs_scan_workspace_size(hist_words), torch.uint8)
@@ -400,7 +400,7 @@ class TideStep:
                 dkeys, rects, dkeys2, rects2 = dkeys2, rects2, dkeys, rects
             N.call("tgs_tide_isect_fused_count", C, cam_segs, N.ptr(rects), tw, tile_bits,
                    N.ptr(fe_hist), hist_words, s)
-            N.call("tgs_exclusive_scan_u32", N.ptr(fe_hist), N.ptr(fe_scan), used_words,
+            N.call("tgs_exclusive_scan_u32", N.ptr(fe_hist), N.ptr(fe_scan), hist_words,
                    N.ptr(ws), ws.numel(), s)
         self._end()
         self.last_depth_key_bits = key_bits
@@ -421,7 +421,7 @@ class TideStep:
                 dkeys, rects, dkeys2, rects2 = dkeys2, rects2, dkeys, rects
             N.call("tgs_tide_isect_fused_count", C, cam_segs, N.ptr(rects), tw, tile_bits,
                    N.ptr(fe_hist), hist_words, s)
-            N.call("tgs_exclusive_scan_u32", N.ptr(fe_hist), N.ptr(fe_scan), used_words,
+            N.call("tgs_exclusive_scan_u32", N.ptr(fe_hist), N.ptr(fe_scan), hist_words,
                    N.ptr(ws), ws.numel(), s)
             self._end()
         per_cam = proj_host[:C].tolist()
