@@ -430,9 +430,10 @@ extern "C" uint32_t tgs_bit_width(uint32_t v) {
 // The reference's order in two sorts: Gaussians by depth (32-bit keys), then the
 // intersections they emit in that order by tile, stably, gives (camera, tile,
 // depth, Gaussian) with two 8-byte moves per intersection instead of the single
-// sort's five 12-byte ones (both measured at the rule below).  The single sort takes what this does not: packed
-// camera ids (in any order), grids past 255 tiles a side (8-bit rectangles), more
-// cameras than the emission's segments, negative depths (their sign fills the id).
+// sort's five 12-byte ones (both measured at the rule below).  The single sort takes
+// what this does not: packed camera ids (in any order), grids past 255 tiles a side
+// (8-bit rectangles), more cameras than the emission's segments, negative depths
+// (their sign fills the id).
 // ---------------------------------------------------------------------------
 // Depth keys and tile rectangles (x0 | x1 << 8 | y0 << 16 | y1 << 24, above the
 // index) of the Gaussians that meet any tile, in order.

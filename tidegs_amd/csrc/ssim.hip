@@ -59,8 +59,10 @@ struct Taps {
 // so every ring index is a constant, and each row is loaded two steps ahead.
 // 16x16 tiles with a 26x26 halo in LDS, the form before, filtered 2.6 rows and
 // columns per output and idled threads at its barriers: one 1080p image of 3
-// channels took 90 us forward and 115 us backward, here 58 and 48 (the backward
-// at 3.1 TB/s; the forward is bound by its window products).
+// channels took 85 us forward and 103 us backward, here 55 and 54 (the mean form 60
+// and 48).  What bounds it is a row's chain through LDS and the ring at two
+// wavefronts per SIMD: the forward issues its window products at 62% of the rate
+// that the fused loss reaches on sixteen such images, the backward at 35%.
 // The mean form writes neither the map nor its gradient (a constant): forward
 // 20 bytes, backward 24 bytes per value, against 24 + 4 and 28 + 12 with the
 // mean's reduction and the gradient's expansion as passes of their own.
@@ -703,7 +705,7 @@ struct LossGrid {
 // A lone workgroup takes 0.71 us per row, four on a CU 1.2 us: 2.4 times a busy
 // CU's 0.3 us per row and workgroup.  Bands of 123 rows at every size, the rule
 // before, left small batches to a few long-running wavefronts: one 256x256 image
-// 102 -> 25 us, four 979x546 132 -> 91, one 1080p 126 -> 94; sixteen 1080p images
+// 104 -> 26 us, four 979x546 132 -> 103, one 1080p 133 -> 96; sixteen 1080p images
 // keep the 123 rows (1.10 ms; in 13-row bands 1.86).
 #define LOSS_LONE 2.4f
 #define LOSS_PERIODS 13

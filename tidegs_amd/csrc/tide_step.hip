@@ -1430,11 +1430,11 @@ extern "C" uint32_t tgs_tide_row_blocks(uint64_t n_rows) {
 }
 
 static int tide_visibility(uint64_t n_rows, const float* params, uint32_t row_stride,
-                                   uint32_t C,
-                                   const float* viewmats, const float* Ks, const float* campos,
-                                   int32_t W, int32_t H, float eps2d, float near_plane,
-                                   float far_plane, float radius_clip, uint32_t* masks,
-                                   uint32_t* counts, uint32_t* depth_range, bool init, hipStream_t stream) {
+                           uint32_t C,
+                           const float* viewmats, const float* Ks, const float* campos,
+                           int32_t W, int32_t H, float eps2d, float near_plane,
+                           float far_plane, float radius_clip, uint32_t* masks,
+                           uint32_t* counts, uint32_t* depth_range, bool init, hipStream_t stream) {
   int rc = check_cams(C);
   if (rc) return rc;
   if (init && depth_range)
@@ -1464,11 +1464,11 @@ extern "C" int tgs_tide_visibility(uint64_t n_rows, const float* params, uint32_
 
 // After tgs_tide_begin: the range is already empty.
 extern "C" int tgs_tide_visibility_begun(uint64_t n_rows, const float* params, uint32_t row_stride,
-                                   uint32_t C, const float* viewmats, const float* Ks,
-                                   const float* campos, int32_t W, int32_t H, float eps2d,
-                                   float near_plane, float far_plane, float radius_clip,
-                                   uint32_t* masks, uint32_t* counts, uint32_t* depth_range,
-                                   hipStream_t stream) {
+                                         uint32_t C, const float* viewmats, const float* Ks,
+                                         const float* campos, int32_t W, int32_t H, float eps2d,
+                                         float near_plane, float far_plane, float radius_clip,
+                                         uint32_t* masks, uint32_t* counts, uint32_t* depth_range,
+                                         hipStream_t stream) {
   return tide_visibility(n_rows, params, row_stride, C, viewmats, Ks, campos, W, H, eps2d,
                          near_plane, far_plane, radius_clip, masks, counts, depth_range, false,
                          stream);
@@ -1495,17 +1495,17 @@ extern "C" int tgs_tide_compact(uint64_t n_rows, uint32_t C, const uint32_t* mas
 }
 
 static int tide_project_fwd(uint32_t n_touched, const uint32_t* n_touched_dev,
-                                    const int32_t* touched,
-                                    const int32_t* visit_base, const int32_t* visits,
-                                    const uint32_t* masks, uint32_t C, const float* params,
-                                    uint32_t row_stride, const float* viewmats, const float* Ks,
-                                    const float* campos, int32_t W, int32_t H, float eps2d,
-                                    float near_plane, float far_plane, float radius_clip,
-                                    int32_t sh_degree, uint32_t tile_size, uint32_t tile_width,
-                                    uint32_t tile_height,
-                                    float* splats, uint32_t* depth_keys, uint64_t* entry_rects,
-                                    int64_t* isect_totals, uint32_t* depth_range, bool init,
-                                    hipStream_t stream) {
+                            const int32_t* touched,
+                            const int32_t* visit_base, const int32_t* visits,
+                            const uint32_t* masks, uint32_t C, const float* params,
+                            uint32_t row_stride, const float* viewmats, const float* Ks,
+                            const float* campos, int32_t W, int32_t H, float eps2d,
+                            float near_plane, float far_plane, float radius_clip,
+                            int32_t sh_degree, uint32_t tile_size, uint32_t tile_width,
+                            uint32_t tile_height,
+                            float* splats, uint32_t* depth_keys, uint64_t* entry_rects,
+                            int64_t* isect_totals, uint32_t* depth_range, bool init,
+                            hipStream_t stream) {
   int rc = check_cams(C);
   if (rc) return rc;
   if (init && isect_totals)
