@@ -145,47 +145,42 @@ __global__ void __launch_bounds__(SCAN_THREADS) scan_apply_kernel(const InT* __r
 }
 
 // The whole scan in one 1024-thread workgroup, SCAN_ONE_ITEMS consecutive
-// values per thread and round.  The three-kernel form spends its time in
-// launches when the array is short (a pass's histogram, the per-block counts of
-// a few hundred thousand rows): a radix pass over 7.7k counts takes 13 us
-// less with this scan.  At 25k values, three rounds of the one workgroup, the
-// three launches are as fast.
+// values per thread.  The three-kernel form spends its time in launches when the
+// array is short (a pass's histogram, the per-block counts of a few hundred
+// thousand rows): 1000 values 9.0 us in three launches and 3.5 in one, 4096 10.3
+// and 5.3, 8192 10.5 and 8.7.  A second round of the one workgroup costs what
+// three launches do: 10k values 10.7 and 10.7, 16k 10.8 and 16.1.
 #define SCAN_ONE_THREADS 1024
 #define SCAN_ONE_ITEMS 8
-#define SCAN_ONE_BLOCK_MAX 16384
+#define SCAN_ONE_BLOCK_MAX (SCAN_ONE_THREADS * SCAN_ONE_ITEMS)
 
 template <typename InT, typename OutT, bool INCLUSIVE>
 __global__ void __launch_bounds__(SCAN_ONE_THREADS) scan_one_block_kernel(
     const InT* __restrict__ in, uint32_t n, OutT* __restrict__ out) {
   __shared__ OutT s_wave[SCAN_ONE_THREADS / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  OutT carry = 0;
-  for (uint32_t base = 0; base < n; base += SCAN_ONE_THREADS * SCAN_ONE_ITEMS) {
-    const uint32_t i0 = base + threadIdx.x * SCAN_ONE_ITEMS;
-    OutT vals[SCAN_ONE_ITEMS];
-    OutT sum = 0;
+  const uint32_t i0 = threadIdx.x * SCAN_ONE_ITEMS;
+  OutT vals[SCAN_ONE_ITEMS];
+  OutT sum = 0;
 #pragma unroll
-    for (int k = 0; k < SCAN_ONE_ITEMS; ++k) {
-      vals[k] = i0 + k < n ? (OutT)in[i0 + k] : (OutT)0;
-      sum += vals[k];
-    }
-    const OutT inc = wave_inclusive_scan<OutT>(sum);
-    if (lane == 63) s_wave[wave] = inc;
-    __syncthreads();
-    OutT run = carry + inc - sum;
+  for (int k = 0; k < SCAN_ONE_ITEMS; ++k) {
+    vals[k] = i0 + k < n ? (OutT)in[i0 + k] : (OutT)0;
+    sum += vals[k];
+  }
+  const OutT inc = wave_inclusive_scan<OutT>(sum);
+  if (lane == 63) s_wave[wave] = inc;
+  __syncthreads();
+  OutT run = inc - sum;
 #pragma unroll
-    for (int w = 0; w < SCAN_ONE_THREADS / 64; ++w) {
-      const OutT t = s_wave[w];
-      if (w < wave) run += t;
-      carry += t;
-    }
+  for (int w = 0; w < SCAN_ONE_THREADS / 64; ++w) {
+    const OutT t = s_wave[w];
+    if (w < wave) run += t;
+  }
 #pragma unroll
-    for (int k = 0; k < SCAN_ONE_ITEMS; ++k) {
-      if (INCLUSIVE) run += vals[k];
-      if (i0 + k < n) out[i0 + k] = run;
-      if (!INCLUSIVE) run += vals[k];
-    }
-    __syncthreads();
+  for (int k = 0; k < SCAN_ONE_ITEMS; ++k) {
+    if (INCLUSIVE) run += vals[k];
+    if (i0 + k < n) out[i0 + k] = run;
+    if (!INCLUSIVE) run += vals[k];
   }
 }
 
