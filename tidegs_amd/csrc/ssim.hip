@@ -61,8 +61,8 @@ struct Taps {
 // columns per output and idled threads at its barriers: one 1080p image of 3
 // channels took 85 us forward and 103 us backward, here 55 and 54 (the mean form 60
 // and 48).  What bounds it is a row's chain through LDS and the ring at two
-// wavefronts per SIMD: the forward issues its window products at 67% of the rate
-// that the fused loss reaches on sixteen such images, the backward at 35%.
+// wavefronts per SIMD: the forward issues its window products at 70% of the rate
+// that the fused loss reaches on sixteen such images, the backward at 37%.
 // The mean form writes neither the map nor its gradient (a constant): forward
 // 20 bytes, backward 24 bytes per value, against 24 + 4 and 28 + 12 with the
 // mean's reduction and the gradient's expansion as passes of their own.
